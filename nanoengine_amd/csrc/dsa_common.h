@@ -70,17 +70,27 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_floa
 
 // Per-row candidate list of the exact top-k (device workspace): a score
 // threshold t_key (order key), the number of candidates appended, a flag set
-// when the list could not be used (fused indexer path), then the (key,
-// position) pairs. Filled by the top-k gather kernel or by the fused indexer.
-constexpr int kListCap = 6144;
-struct RowWs {
+// when the list could not be used (fused indexer paths), then the (key,
+// position) pairs. RowWs is filled by the top-k gather kernel; DecodeList and
+// PrefillList by the fused indexer passes, whose thresholds come from smaller
+// samples: f sampled scores are expected in the top-k, the threshold is the
+// sample's rank f + 4 sqrt(f) + 8. Of a 128K decode row f = 16: 6144 entries
+// overflowed once in 10 rows, 16384 hold 7.8 standard deviations. Of a 128K
+// prefill row f = 32: 3 rows in 10000 overflowed 6144, 8192 hold 5.8.
+template <int CAP>
+struct RowListT {
+  static constexpr int kCap = CAP;
   uint32_t t_key;
   uint32_t count;
   uint32_t failed;
   uint32_t pad;
-  uint32_t key[kListCap];
-  uint32_t pos[kListCap];
+  uint32_t key[CAP];
+  uint32_t pos[CAP];
 };
+constexpr int kListCap = 6144;  // also the entries a select keeps in LDS
+using RowWs = RowListT<kListCap>;
+using DecodeList = RowListT<16384>;
+using PrefillList = RowListT<8192>;
 
 // What the list select needs to redo a row whose list is unusable: the
 // indexer inputs of the row (query [rows, 64, 128] fp8, head weights
@@ -97,15 +107,16 @@ struct RowRepair {
   uint32_t* defer_count;
 };
 
-// Launcher of the list select of the fused indexer + top-k entry point
-// (topk.hip): the exact top-k of each row's candidate list, with the page
-// translation; a row whose list is unusable is redone in place from its
-// full logits.
-// Without a page table, row b's positions are written plus offsets[b] (NULL: 0).
-int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, RowWs* ws,
+// Launchers of the list select (topk.hip): the exact top-k of each row's
+// candidate list. Decode: with the page translation; a row whose list is
+// unusable is redone in place from its full logits.
+int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, DecodeList* ws,
                        const int32_t* page_table, int64_t pt_stride, int pt_div, uint32_t page_bits,
-                       const int32_t* offsets, int32_t* out_page, int32_t* out_raw, int top_k, int rows,
-                       hipStream_t stream);
+                       int32_t* out_page, int32_t* out_raw, int top_k, int rows, hipStream_t stream);
+// Prefill: row b's positions are written plus offsets[b]; the rows that cannot
+// be selected from their lists are deferred to the caller.
+int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, PrefillList* ws,
+                       const int32_t* offsets, int32_t* out, int top_k, int rows, hipStream_t stream);
 
 // The ragged fp8 MQA logits kernel (prefill_logits.hip). filter = false:
 // logits[i, j] for j in [ks[i], ke[i]). filter = true: nothing is stored;
@@ -113,7 +124,7 @@ int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max
 // order key is at least ws[i].t_key.
 int launch_mqa_logits(bool filter, const uint8_t* q, const uint8_t* kv, const float* kv_scale, const float* weights,
                       int64_t weights_stride, const int32_t* ks, const int32_t* ke, int num_rows, int64_t num_keys,
-                      float* logits, int64_t logits_stride, RowWs* ws, hipStream_t st);
+                      float* logits, int64_t logits_stride, PrefillList* ws, hipStream_t st);
 
 // Sparse MLA decode over physical slots of the paged fp8 cache (the body of
 // dsa_sparse_mla_decode). max_out (splits == 1 only) receives each head's

@@ -18,7 +18,7 @@
 // indexer_page.h.
 //
 // Launches: indexer_logits_kernel (one workgroup per 24 pages of a row) writes
-// the logits (the fp8_paged_mqa_logits operator), samples 16 pages per row for
+// the logits (the fp8_paged_mqa_logits operator), samples pages of each row for
 // the fused path's score threshold, or filters (batches above the persistent
 // kernel's limit); indexer_filter_kernel is the fused path's persistent filter
 // pass (one contiguous page range per wave, per-wave candidate staging).
@@ -38,7 +38,7 @@ constexpr int kIdxPagesPerWave = 6;
 // What a launch does with the logits of a page.
 enum IdxMode : int {
   kIdxStore = 0,   // logits[row, t]
-  kIdxSample = 1,  // every page_step-th page, one workgroup per row: the logits stay in LDS and
+  kIdxSample = 1,  // pages spread over the row, one workgroup per row: the logits stay in LDS and
                    // give the row's score threshold ws[row].t_key (lists reset)
   kIdxFilter = 2,  // no logits: (key, t) of every token with key >= ws[row].t_key is appended
                    // to the row's candidate list (staged in LDS, one global atomic per WG)
@@ -47,8 +47,7 @@ enum IdxMode : int {
 struct IdxOut {
   float* logits;
   int64_t logits_stride;
-  int page_step;            // kIdxSample: sampled page stride
-  RowWs* ws;                // kIdxSample: thresholds out; kIdxFilter: thresholds in, lists out
+  DecodeList* ws;                // kIdxSample: thresholds out; kIdxFilter: thresholds in, lists out
   int top_k;                // kIdxSample
 };
 
@@ -58,10 +57,18 @@ struct IdxStoreLds {  // store mode: the waves' page tiles (rows_to_operands)
   __attribute__((aligned(16))) uint8_t tr[kIdxWaves][kIdxTrBytes];
 };
 
-constexpr int kSamplePages = 16;  // sampled pages per row, one workgroup
-// The sample pass is latency-bound (one workgroup per row): its pages are
-// spread one per wave (two per wave for two query tokens, which need twice the
-// query registers).
+// Sampled pages: at most 16, evenly spread over the row's own length. (A step
+// taken from the batch's longest row leaves a short row one or two pages, so
+// that in a ragged batch of 2K to 128K tokens some row's list overflowed on
+// every call, and its repair by one CU took 330 to 540 of the step's 490 to
+// 710 us.) The pass is latency-bound (one workgroup per row): its pages go one
+// per wave (two per wave for two query tokens, which need twice the query
+// registers). 32 pages for rows over 64K tokens cost it 7 us; the list's
+// capacity covers their smaller sample instead.
+constexpr int kSamplePages = 16;
+__device__ __forceinline__ int sample_step(int npages) {
+  return max(1, (npages + kSamplePages - 1) / kSamplePages);
+}
 template <int NQ>
 constexpr int sample_threads() { return NQ == 1 ? 1024 : 512; }
 template <int NQ, int MODE>
@@ -142,14 +149,16 @@ indexer_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
   static_assert(MODE != kIdxSample || PPW * NW == kSamplePages, "sample geometry");
   const int b = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int step = MODE == kIdxSample ? o.page_step : 1;
   const int vp_begin = blockIdx.x * (NW * PPW) + wave;
   // All of the wave's block-table entries in one load, issued before the
   // context lengths arrive: every table row holds ceil(max_ctx / 64) entries,
-  // and entries past a row's context are loaded but never used.
+  // and entries past a row's context are loaded but never used. The sample
+  // guesses the step of a row of max_ctx tokens, right for a batch of equal
+  // lengths, and reloads the entries of the others.
   const int max_pages = (int)((max_ctx + kIdxPageTokens - 1) / kIdxPageTokens);
+  int step = MODE == kIdxSample ? sample_step(max_pages) : 1;
   const int spec_page = (vp_begin + NW * lane) * step;
-  const int my_page =
+  int my_page =
       (lane < PPW && spec_page < max_pages) ? block_tables[(int64_t)b * bt_stride + spec_page] : 0;
 
   int L[NQ];
@@ -163,7 +172,25 @@ indexer_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
   }
   // real pages of the row, and the virtual pages this launch walks (every
   // step-th real page)
-  const int npages = (int)((min((int64_t)Lmax, max_ctx) + kIdxPageTokens - 1) / kIdxPageTokens);
+  const int npages = (int)((min((int64_t)max(Lmax, 0), max_ctx) + kIdxPageTokens - 1) / kIdxPageTokens);
+  if constexpr (MODE == kIdxSample) {
+    if (min((int64_t)Lmax, max_ctx) <= o.top_k) {
+      // every token is selected: no threshold, and no candidate reaches this key
+      if (threadIdx.x < NQ) {
+        DecodeList& rw = o.ws[b * NQ + threadIdx.x];
+        rw.t_key = 0xffffffffu;
+        rw.count = 0u;
+        rw.failed = 0u;
+      }
+      return;
+    }
+    const int row_step = sample_step(npages);
+    if (row_step != step) {
+      step = row_step;
+      const int page = (vp_begin + NW * lane) * step;
+      my_page = (lane < PPW && page < npages) ? block_tables[(int64_t)b * bt_stride + page] : 0;
+    }
+  }
   const int nvp = (npages + step - 1) / step;
   if (MODE != kIdxSample && blockIdx.x * (NW * PPW) >= nvp) return;
 
@@ -263,17 +290,18 @@ indexer_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
     __syncthreads();  // the sampled logits are in LDS
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
-      RowWs& rw = o.ws[b * NQ + j];
+      DecodeList& rw = o.ws[b * NQ + j];
       const float* smp = sl.logit[j];
       const int len = (int)min((int64_t)max(L[j], 0), max_ctx);
       const int nv = (len + span - 1) / span;
-      uint32_t nsample = 0;
-      for (int v = 0; v < nv; ++v) nsample += (uint32_t)max(0, min(len - v * span, kIdxPageTokens));
+      // only the last sampled page can be partly filled
+      const uint32_t nsample = len > 0 ? (uint32_t)((nv - 1) * kIdxPageTokens + min(len - (nv - 1) * span, kIdxPageTokens)) : 0u;
       const float fk = (float)nsample / (float)max(len, 1) * (float)o.top_k;
       const uint32_t r = (uint32_t)(fk + 4.f * sqrtf(fk) + 8.f);
-      uint32_t t_key = 0u;  // 0: every token is a candidate
+      // 0: every token is a candidate; the largest key: none (all are selected)
+      uint32_t t_key = len > o.top_k ? 0u : 0xffffffffu;
       if (len > o.top_k && r < nsample) {
-        // this thread's sampled keys (nv * 64 <= 1024 = 4 per thread)
+        // this thread's sampled keys
         constexpr int kPer = kSamplePages * kIdxPageTokens / NT;
         uint32_t key[kPer];
         uint32_t kmin = 0xffffffffu, kmax = 0u;
@@ -350,12 +378,12 @@ indexer_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
       const uint32_t n = stage->count[j];
-      RowWs& rw = o.ws[b * NQ + j];
+      DecodeList& rw = o.ws[b * NQ + j];
       if (threadIdx.x == 0) stage->base[j] = n ? atomicAdd(&rw.count, n) : 0u;
       __syncthreads();
       const uint32_t base = stage->base[j];
       for (uint32_t e = threadIdx.x; e < n; e += NT)
-        if (base + e < (uint32_t)kListCap) {
+        if (base + e < (uint32_t)DecodeList::kCap) {
           rw.key[base + e] = stage->key[j][e];
           rw.pos[base + e] = stage->pos[j][e];
         }
@@ -392,7 +420,7 @@ __global__ void __launch_bounds__(kIdxThreads) __attribute__((amdgpu_waves_per_e
 indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kv,
                       const float* __restrict__ weights, const int32_t* __restrict__ ctx_lens,
                       const int32_t* __restrict__ block_tables, int64_t bt_stride, int64_t max_ctx, int batch,
-                      RowWs* __restrict__ ws) {
+                      int top_k, DecodeList* __restrict__ ws) {
   extern __shared__ __align__(16) uint8_t fl_smem[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   FiltWaveStage& st = reinterpret_cast<FiltWaveStage*>(fl_smem)[wave];
@@ -409,7 +437,9 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
       int lm = 0;
 #pragma unroll
       for (int j = 0; j < NQ; ++j) lm = max(lm, ctx_lens[i * NQ + j]);
-      np = (int)((min((int64_t)lm, max_ctx) + kIdxPageTokens - 1) / kIdxPageTokens);
+      lm = (int)min((int64_t)lm, max_ctx);
+      // an entry of at most top_k tokens is selected whole: its pages are not read
+      np = lm > top_k ? (lm + kIdxPageTokens - 1) / kIdxPageTokens : 0;
     }
     int v = np;
 #pragma unroll
@@ -446,7 +476,8 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
     const int64_t p = p0 + from + lane;
     int bl = 0, page = 0;
     if (p < p1) {
-      // last batch entry with prefix <= p
+      // last batch entry with prefix <= p (the one whose pages hold p: an entry
+      // without pages has the next entry's prefix)
       int lo = 0, hi = batch - 1;
       while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -473,12 +504,12 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
   auto flush = [&](int j) {
     const int c = cnt[j];
     if (c == 0) return;
-    RowWs& rw = ws[cur_b * NQ + j];
+    DecodeList& rw = ws[cur_b * NQ + j];
     uint32_t base = 0;
     if (lane == 0) base = atomicAdd(&rw.count, (uint32_t)c);
     base = __shfl(base, 0, 64);
     for (int e = lane; e < c; e += 64)
-      if (base + (uint32_t)e < (uint32_t)kListCap) {
+      if (base + (uint32_t)e < (uint32_t)DecodeList::kCap) {
         rw.key[base + e] = st.key[j][e];
         rw.pos[base + e] = st.pos[j][e];
       }
@@ -566,7 +597,7 @@ static int filter_grid() {
 // The persistent filter pass; false when the batch does not fit its LDS prefix.
 static bool launch_filter_persistent(const uint8_t* q, const uint8_t* kv, const float* weights,
                                      const int32_t* ctx_lens, const int32_t* bt, int64_t bt_stride, int batch,
-                                     int next_n, int64_t max_ctx, RowWs* ws, hipStream_t stream) {
+                                     int next_n, int64_t max_ctx, int top_k, DecodeList* ws, hipStream_t stream) {
   if (batch > kFiltMaxBatch) return false;
   const size_t smem = filt_smem_bytes(batch);
   static bool attr_set = false;
@@ -582,19 +613,19 @@ static bool launch_filter_persistent(const uint8_t* q, const uint8_t* kv, const 
   const dim3 grid((unsigned)filter_grid());
   if (next_n == 1)
     hipLaunchKernelGGL(indexer_filter_kernel<1>, grid, dim3(kIdxThreads), smem, stream, q, kv, weights, ctx_lens, bt,
-                       bt_stride, max_ctx, batch, ws);
+                       bt_stride, max_ctx, batch, top_k, ws);
   else
     hipLaunchKernelGGL(indexer_filter_kernel<2>, grid, dim3(kIdxThreads), smem, stream, q, kv, weights, ctx_lens, bt,
-                       bt_stride, max_ctx, batch, ws);
+                       bt_stride, max_ctx, batch, top_k, ws);
   return true;
 }
 
 template <int MODE>
 void launch_indexer(const uint8_t* q, const uint8_t* kv, const float* weights, const int32_t* ctx_lens,
-                    const int32_t* bt, int64_t bt_stride, int batch, int next_n, int64_t max_ctx, int64_t vpages,
+                    const int32_t* bt, int64_t bt_stride, int batch, int next_n, int64_t max_ctx, int64_t pages,
                     const IdxOut& o, hipStream_t stream) {
-  const int64_t per_block = MODE == kIdxSample ? kSamplePages : kIdxWaves * kIdxPagesPerWave;
-  const dim3 grid((unsigned)((vpages + per_block - 1) / per_block), (unsigned)batch);
+  const int64_t per_block = kIdxWaves * kIdxPagesPerWave;
+  const dim3 grid(MODE == kIdxSample ? 1u : (unsigned)((pages + per_block - 1) / per_block), (unsigned)batch);
   if (next_n == 1)
     hipLaunchKernelGGL((indexer_logits_kernel<1, MODE>), grid, dim3(idx_threads<1, MODE>()), 0, stream, q, kv, weights, ctx_lens,
                        bt, bt_stride, max_ctx, o);
@@ -626,7 +657,7 @@ extern "C" int dsa_indexer_logits(const uint8_t* q_fp8, const uint8_t* kv_cache,
   if ((reinterpret_cast<uintptr_t>(q_fp8) | reinterpret_cast<uintptr_t>(kv_cache)) & 15)
     return set_error(kInvalidArgument, "indexer: q and kv_cache must be 16-byte aligned");
   const int64_t max_pages = (max_context_len + kIdxPageTokens - 1) / kIdxPageTokens;
-  IdxOut o{logits, logits_stride, 1, nullptr, 0};
+  IdxOut o{logits, logits_stride, nullptr, 0};
   launch_indexer<kIdxStore>(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch, next_n,
                             max_context_len, max_pages, o, (hipStream_t)stream);
   return check_launch("dsa_indexer_logits");
@@ -634,14 +665,8 @@ extern "C" int dsa_indexer_logits(const uint8_t* q_fp8, const uint8_t* kv_cache,
 
 // ---------------------------------------------------------------- fused indexer + top-k
 namespace dsa {
-// Page step of the threshold sample: every step-th page, at most 16 pages (1024
-// tokens) per row, so one workgroup holds a row's sample.
-static inline int sample_step(int64_t max_pages) {
-  return (int)std::max<int64_t>(1, (max_pages + kSamplePages - 1) / kSamplePages);
-}
-
 struct FusedWs {
-  RowWs* ws;
+  DecodeList* ws;
   float* logits;  // full logits, written only for rows the list select redoes
   int64_t logits_stride;
   size_t bytes;
@@ -652,10 +677,10 @@ static inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static FusedWs fused_layout(void* base, int rows, int64_t max_ctx) {
   FusedWs f;
   f.logits_stride = (max_ctx + 3) & ~(int64_t)3;
-  const size_t ws_b = align256((size_t)rows * sizeof(RowWs));
+  const size_t ws_b = align256((size_t)rows * sizeof(DecodeList));
   const size_t logits_b = align256((size_t)rows * f.logits_stride * sizeof(float));
   uint8_t* p = static_cast<uint8_t*>(base);
-  f.ws = reinterpret_cast<RowWs*>(p);
+  f.ws = reinterpret_cast<DecodeList*>(p);
   f.logits = reinterpret_cast<float*>(p + ws_b);
   f.bytes = ws_b + logits_b;
   return f;
@@ -704,18 +729,17 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
   };
   mark(0);
   const int64_t max_pages = (max_context_len + kIdxPageTokens - 1) / kIdxPageTokens;
-  const int step = sample_step(max_pages);
-  // 1-2. logits of every step-th page (one workgroup per row, kept in LDS) ->
-  // the row's score threshold, lists reset
-  IdxOut o_s{nullptr, 0, step, f.ws, top_k};
+  // 1-2. logits of sampled pages (one workgroup per batch entry, kept in LDS)
+  // -> each row's score threshold, lists reset
+  IdxOut o_s{nullptr, 0, f.ws, top_k};
   launch_indexer<kIdxSample>(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
-                             next_n, max_context_len, (max_pages + step - 1) / step, o_s, st);
+                             next_n, max_context_len, max_pages, o_s, st);
   if (int rc = check_launch("dsa_indexer_topk(sample)")) return rc;
   mark(1);
   // 3. all pages: candidates at or above the threshold into the row lists
   if (!launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
-                                next_n, max_context_len, f.ws, st)) {
-    IdxOut o_f{nullptr, 0, 1, f.ws, top_k};
+                                next_n, max_context_len, top_k, f.ws, st)) {
+    IdxOut o_f{nullptr, 0, f.ws, top_k};
     launch_indexer<kIdxFilter>(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
                                next_n, max_context_len, max_pages, o_f, st);
   }
@@ -725,7 +749,7 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
   // whose list is unusable is redone by its workgroup from its full logits
   const RowRepair rp{q_fp8, kv_cache, weights, f.logits, f.logits_stride, nullptr, nullptr};
   const int rc = launch_list_select(rp, context_lens, max_context_len, f.ws, block_tables, block_table_stride, next_n,
-                                    6u, nullptr, out_physical, out_logical, top_k, rows, st);
+                                    6u, out_physical, out_logical, top_k, rows, st);
   mark(3);
   mark(4);
   return rc;

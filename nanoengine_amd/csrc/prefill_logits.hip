@@ -61,7 +61,7 @@ struct PfLds {
 };
 // The filter mode's per-wave candidate stage: (order key, position in the
 // row's window) of the keys at or above the row's threshold, moved to the
-// row's list in RowWs with one global atomic per flush.
+// row's PrefillList with one global atomic per flush.
 constexpr int kPfStageCap = 832;  // fills the LDS left by the key stages (157 KB of 160 KB)
 struct PfLdsFilter : PfLds {
   uint32_t st_key[kPfWaves][kPfStageCap];
@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(kPfThreads)
 mqa_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kv, const float* __restrict__ kv_scale,
                   const float* __restrict__ weights, int64_t w_stride, const int32_t* __restrict__ ks,
                   const int32_t* __restrict__ ke, int M, int64_t n_keys, int token_blocks, int64_t chunk_keys,
-                  float* __restrict__ logits, int64_t logits_stride, RowWs* __restrict__ ws) {
+                  float* __restrict__ logits, int64_t logits_stride, PrefillList* __restrict__ ws) {
   __shared__ typename std::conditional<kFilter, PfLdsFilter, PfLds>::type lds;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -183,12 +183,12 @@ mqa_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kv,
   auto flush = [&]() {
     if constexpr (kFilter) {
       if (cnt == 0) return;
-      RowWs& rw = ws[rc];
+      PrefillList& rw = ws[rc];
       uint32_t base = 0;
       if (lane == 0) base = atomicAdd(&rw.count, (uint32_t)cnt);
       base = __builtin_amdgcn_readfirstlane(base);
       for (int e = lane; e < cnt; e += 64)
-        if (base + (uint32_t)e < (uint32_t)kListCap) {
+        if (base + (uint32_t)e < (uint32_t)PrefillList::kCap) {
           rw.key[base + e] = lds.st_key[wave][e];
           rw.pos[base + e] = lds.st_pos[wave][e];
         }
@@ -341,7 +341,7 @@ prefill_windows_kernel(const void* __restrict__ cu_q, const void* __restrict__ c
 // Both modes of the logits kernel on one grid: token blocks x key chunks.
 int launch_mqa_logits(bool filter, const uint8_t* q, const uint8_t* kv, const float* kv_scale, const float* weights,
                       int64_t weights_stride, const int32_t* ks, const int32_t* ke, int num_rows, int64_t num_keys,
-                      float* logits, int64_t logits_stride, RowWs* ws, hipStream_t st) {
+                      float* logits, int64_t logits_stride, PrefillList* ws, hipStream_t st) {
   const int token_blocks = (num_rows + kPfTokens - 1) / kPfTokens;
   int64_t chunks, chunk_keys;
   if (token_blocks >= 512 && num_keys <= 32 * kPfStageKeys) {

@@ -85,13 +85,13 @@ mqa_topk_sample_keys_kernel(const uint8_t* __restrict__ kv, const float* __restr
 __global__ void __launch_bounds__(256)
 mqa_topk_threshold_kernel(const float* __restrict__ slog, int64_t s_stride, const int32_t* __restrict__ sks,
                           const int32_t* __restrict__ ske, const int32_t* __restrict__ lens, int top_k,
-                          RowWs* __restrict__ ws) {
+                          PrefillList* __restrict__ ws) {
   __shared__ __align__(16) uint32_t hist[4096];
   __shared__ uint32_t wave_sum[4];
   __shared__ uint32_t tb, above, eq;
   const int tid = threadIdx.x, b = blockIdx.x;
   const int len = lens[b];
-  RowWs& w = ws[b];
+  PrefillList& w = ws[b];
   uint32_t t_key = 0xffffffffu;
   if (len > top_k) {
     const int a = sks[b];
@@ -164,7 +164,7 @@ struct MqaTopkLayout {
     fix_rows = std::max<int64_t>(1, std::min<int64_t>(rows, kFixupLogitsBytes / (4 * std::max<int64_t>(keys, 1))));
     size_t at = 0;
     auto take = [&](size_t bytes) { const size_t p = at; at += align_up(bytes); return p; };
-    ws = take((size_t)rows * sizeof(RowWs));
+    ws = take((size_t)rows * sizeof(PrefillList));
     slog = take((size_t)rows * samples * 4);
     skv = take((size_t)samples * kHeadDim);
     sscale = take((size_t)samples * 4);
@@ -221,7 +221,7 @@ int dsa_mqa_topk(const uint8_t* q, const uint8_t* kv, const float* kv_scale, con
   hipStream_t st = (hipStream_t)stream;
   uint8_t* base = static_cast<uint8_t*>(workspace);
   auto at = [&](size_t off) { return base + off; };
-  RowWs* ws = reinterpret_cast<RowWs*>(at(L.ws));
+  PrefillList* ws = reinterpret_cast<PrefillList*>(at(L.ws));
   float* slog = reinterpret_cast<float*>(at(L.slog));
   int32_t* ke_c = reinterpret_cast<int32_t*>(at(L.ke_c));
   int32_t* lens = reinterpret_cast<int32_t*>(at(L.lens));
@@ -251,8 +251,7 @@ int dsa_mqa_topk(const uint8_t* q, const uint8_t* kv, const float* kv_scale, con
                                    nullptr, 0, ws, st))
       return rc;
   const RowRepair defer_only{nullptr, nullptr, nullptr, nullptr, 0, defer, count};
-  if (int rc = launch_list_select(defer_only, lens, max_len, ws, nullptr, 0, 1, 0u, ks, out, nullptr, top_k,
-                                  num_rows, st))
+  if (int rc = launch_list_select(defer_only, lens, max_len, ws, ks, out, top_k, num_rows, st))
     return rc;
 
   // rows whose list could not give the exact top-k

@@ -25,11 +25,12 @@
 //      needs no bound at all. The selected positions are marked in an LDS
 //      bitmap, compacted with one block prefix scan (ascending order, so the
 //      output is deterministic) and written with the page translation.
-// No global sort, no bounded candidate buffer on the exact path. The list
-// selects (one-launch kernel, the fused indexer's topk_list_kernel) radix over
+// No global sort, no bounded candidate buffer on the exact path. The
+// one-launch kernel's list select radixes over
 // [ key - t : nb bits ][ (2^18-1) - position : 18 bits ] instead, nb the bit
-// length of the largest key - t, so that their digits spread over the
-// candidates' own range.
+// length of the largest key - t, so that its digits spread over the
+// candidates' own range; the fused indexer's (topk_list_kernel) takes the
+// score's linear bin as its first digit.
 #include <mutex>
 
 #include "dsa_common.h"
@@ -67,15 +68,17 @@ constexpr size_t kTopkSmemBytes = sizeof(TopkSmem);
 // LDS of the list select: the candidates of a level's threshold bin are kept
 // as 16-bit indices into the row's list (values re-read from global), so two
 // workgroups fit on a CU. A row the kernel repairs itself uses TopkSmem.
+constexpr int kRankCap = 384;  // threshold-bin candidates ranked by counting
 struct ListSmem {
   uint32_t hist[kHistBins];
   uint32_t bitmap[kBitmapWords];
   uint16_t list[2][kListCap];
+  uint64_t rank[kRankCap];
   uint32_t wave_sum[16];
   uint32_t list_count[2];
   uint32_t tb, above, eq;
 };
-static_assert(kListCap <= 65536, "list indices are 16-bit");
+static_assert(DecodeList::kCap <= 65536 && PrefillList::kCap <= 65536, "list indices are 16-bit");
 static_assert(sizeof(ListSmem) <= sizeof(TopkSmem), "a repairing launch covers the list layout");
 
 __device__ __forceinline__ uint32_t radix_digit(int level, uint32_t key, uint32_t pos) {
@@ -178,6 +181,32 @@ __device__ void compact_bitmap(const uint32_t* bitmap, int nwords, uint32_t* wav
   *total_out = total;
 }
 
+// The same from byte flags (one per position, 0 or 1, flags[0, len) padded
+// with zeros to a multiple of 8 NT): thread t owns the positions
+// [8 q t, 8 q (t + 1)), q = ceil(len / 8NT).
+template <int NT>
+__device__ void compact_flags(const uint8_t* flags, int len, uint32_t* wave_sum, uint32_t* sel, int top_k,
+                              uint32_t* total_out) {
+  const int tid = threadIdx.x;
+  const int q = (len + 8 * NT - 1) / (8 * NT);
+  const uint64_t* mine = reinterpret_cast<const uint64_t*>(flags) + tid * q;
+  uint32_t cnt = 0;
+  for (int i = 0; i < q; ++i) cnt += __popcll(mine[i]);
+  uint32_t total = 0;
+  uint32_t at = block_exclusive_scan<NT>(wave_sum, cnt, &total);
+  __syncthreads();  // sel may alias buffers read before this call
+  for (int i = 0; i < q; ++i) {
+    uint64_t bits = mine[i];
+    while (bits) {
+      const int bit = __ffsll((unsigned long long)bits) - 1;
+      bits &= bits - 1;
+      if (at < (uint32_t)top_k) sel[at] = (uint32_t)(8 * (tid * q + i) + (bit >> 3));
+      ++at;
+    }
+  }
+  __syncthreads();
+  *total_out = total;
+}
 
 struct RowOut {
   int32_t* page;       // page-translated output (or the untranslated output)
@@ -355,7 +384,7 @@ topk_gather_kernel(const RowIn in, int top_k, RowWs* __restrict__ ws) {
 // The finish of row b by one workgroup of kTopkThreads threads (all of them
 // call it): the list select when the row's list is usable, else the full
 // exact select over the row's scores.
-__device__ void finish_row(TopkSmem& s, const RowIn& in, RowWs* __restrict__ ws, const int32_t* __restrict__ offsets,
+__device__ __forceinline__ void finish_row(TopkSmem& s, const RowIn& in, RowWs* __restrict__ ws, const int32_t* __restrict__ offsets,
                            const int32_t* __restrict__ page_table, int64_t pt_stride, int pt_div, uint32_t page_bits,
                            int32_t* __restrict__ out_page, int32_t* __restrict__ out_raw, int top_k, int b) {
   const int tid = threadIdx.x;
@@ -796,14 +825,32 @@ topk_onepass_kernel(const RowIn in, const int32_t* __restrict__ offsets, const i
 }
 
 // ---------------------------------------------------------------- list select
-// Exact top-k of a row's candidate list (fused indexer path): every candidate
-// has key >= t_key, so the radix runs over the 50-bit composite
-//   [ key - t_key : nb bits ][ (2^18-1) - position : 18 bits ]
-// where nb = bit length of (max key - t_key), in 12-bit digits from the top:
-// the digits spread over the candidates' actual range instead of the fixed
-// bit positions of the full select, where most candidates share the top
-// digits. A row whose list is unusable (fewer than k or more than the list
-// capacity) is flagged for the repair launches.
+// 4096 bins linear in the score between the scores of keys kmin and kmax. The
+// bin never decreases with the key (subtraction, multiplication by a positive
+// scale and truncation are each monotone, +-0 share a bin), so a candidate in
+// a higher bin ranks ahead. Scores that are not finite, or whose range is not,
+// fall into the end bins or all into one.
+struct ScoreBins {
+  float lo, scale;
+  __device__ __forceinline__ ScoreBins(uint32_t kmin, uint32_t kmax) {
+    lo = key_to_float(kmin);
+    const float range = key_to_float(kmax) - lo;
+    scale = range > 0.f && range < 3.0e38f ? (float)(kHistBins - 1) / range : 0.f;
+  }
+  __device__ __forceinline__ uint32_t of(uint32_t key) const {
+    const float x = (key_to_float(key) - lo) * scale;  // NaN (inf * 0) maps to bin 0
+    return (uint32_t)fminf(fmaxf(x, 0.f), (float)(kHistBins - 1));
+  }
+};
+
+// Exact top-k of a row's candidate list (fused indexer path), ranked by
+// (score, lower position). The first digit is the score's linear bin; the
+// threshold bin then holds a few candidates, whose rank each of them counts
+// directly. (Radix digits of the key's bits, all levels, took 17.0 us for four
+// rows of 4K tokens, whose scores cross zero: sign and exponent bits put most
+// candidates into a few bins, where the LDS atomics serialise.) A row whose list is unusable (fewer than k entries, more than the
+// list capacity, or more than kListCap of them sharing the first digit's
+// threshold bin, as when most of its scores tie) is redone or deferred.
 // Full indexer logits of one row by the calling workgroup (kTopkThreads
 // threads): wave w computes pages w, w + 8, ... of the row through three
 // rotating page buffers, logits[t] for t < len.
@@ -839,9 +886,9 @@ __device__ void repair_row_logits(const RowRepair& rp, const int32_t* __restrict
 // The list select of one row per workgroup. kRepair: a row whose list is
 // unusable is redone in the kernel from its full logits (rp.q set, the launch
 // reserves TopkSmem); otherwise it is appended to rp.defer_rows.
-template <bool kRepair>
+template <bool kRepair, typename RowList>
 __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_lens, int64_t max_len,
-                                                RowWs* __restrict__ ws, const int32_t* __restrict__ page_table,
+                                                RowList* __restrict__ ws, const int32_t* __restrict__ page_table,
                                                 int64_t pt_stride, int pt_div, uint32_t page_bits,
                                                 const int32_t* __restrict__ offsets, int32_t* __restrict__ out_page,
                                                 int32_t* __restrict__ out_raw, int top_k, const RowRepair& rp) {
@@ -852,7 +899,7 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   const int b = blockIdx.x;
   const int64_t l = seq_lens[b];
   const int len = (int)(l < 0 ? 0 : (l > max_len ? max_len : l));
-  RowWs& w = ws[b];
+  RowList& w = ws[b];
 
   RowOut out;
   out.page = out_page + (int64_t)b * top_k;
@@ -865,43 +912,42 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
     for (int i = tid; i < top_k; i += NT) out.emit(i, i < len ? i : -1);
     return;
   }
-  const uint32_t cand = w.count;
-  if (cand < (uint32_t)top_k || cand > (uint32_t)kListCap) {
-    // The sample misjudged this row's threshold: its list cannot give the
-    // exact top-k. Redo the row here, from its full logits, or leave it to
-    // the caller.
-    if (tid == 0) w.failed = 1u;
-    if constexpr (kRepair) {
-      repair_row_logits(rp, page_table + (int64_t)(b / pt_div) * pt_stride, b, len);
-      __syncthreads();  // the row's logits (global) are visible to the whole workgroup
-      const RowIn in{rp.logits, rp.logits_stride, seq_lens, nullptr, max_len};
-      // a repairing launch reserves the full select's LDS
-      finish_row(*reinterpret_cast<TopkSmem*>(smem_raw), in, nullptr, nullptr, page_table, pt_stride, pt_div,
-                 page_bits, out_page, out_raw, top_k, b);
-    } else {
-      if (tid == 0) rp.defer_rows[atomicAdd(rp.defer_count, 1u)] = b;
-    }
-    return;
-  }
-  const uint32_t t_key = w.t_key;
-
-  // Candidates into registers (element e = u * NT + tid), all loads in flight
-  // at once: composite (hi = key - t_key, lo = inverted position), and the
-  // block maximum of hi.
-  constexpr int kPer = kListCap / NT;
-  static_assert(kListCap % NT == 0, "list capacity must be whole rows of the block");
-  uint32_t ch[kPer], cl[kPer];
+  const uint32_t cand = __builtin_amdgcn_readfirstlane(w.count);
+  const auto select_list = [&]() -> bool {
+  // The first kReg * NT candidates into registers (element e = u * NT + tid),
+  // all loads in flight at once; any beyond them (a misjudged threshold) are
+  // read again by each pass. Slots past the list are skipped by uniform
+  // branches (most lists fill two thirds of the registers).
+  constexpr int kReg = 12;
+  uint32_t ch[kReg], cl[kReg];
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) {
+  for (int u = 0; u < kReg; ++u) {
     const uint32_t e = (uint32_t)(u * NT + tid);
-    ch[u] = e < cand ? w.key[e] : t_key;
-    cl[u] = e < cand ? w.pos[e] : 0u;
+    ch[u] = 0u;
+    cl[u] = 0u;
+    if (e < cand) {
+      ch[u] = w.key[e];
+      cl[u] = w.pos[e];
+    }
   }
-  const int nwords = (len + 31) >> 5;
-  // The row's page table, when it fits in the bitmap words past the row's,
-  // is copied to LDS with the candidates so that the output's translation
-  // reads LDS, not a dependent global load.
+  auto each = [&](auto&& f) {  // f(element, key, position) over this thread's candidates
+#pragma unroll
+    for (int u = 0; u < kReg; ++u)
+      if ((uint32_t)(u * NT) < cand && (uint32_t)(u * NT + tid) < cand) f((uint32_t)(u * NT + tid), ch[u], cl[u]);
+    for (uint32_t e = kReg * NT + tid; e < cand; e += NT) f(e, w.key[e], w.pos[e]);
+  };
+  auto composite = [&](uint32_t key, uint32_t pos) { return ((uint64_t)key << 18) | (kIdxMax - pos); };
+  // The selected positions are marked in LDS: a byte each where the row fits
+  // (plain stores), else a bit each. In a short row most positions are
+  // selected and the lanes of a wave hold consecutive ones, so that atomics on
+  // the bits serialise: 16.5 us against 11.5 for four rows of 1K to 4K tokens.
   const int npg = out.pt ? (len + (1 << page_bits) - 1) >> page_bits : 0;
+  const int flag_words = (len + 8 * NT - 1) / (8 * NT) * (2 * NT);
+  const bool bytes = flag_words + npg <= kBitmapWords;
+  const int nwords = bytes ? flag_words : (len + 31) >> 5;
+  // The row's page table, when it fits in the words past the marks, is copied
+  // to LDS with the candidates so that the output's translation reads LDS, not
+  // a dependent global load.
   const int pt_off = (nwords + 3) & ~3;
   const bool pt_lds = out.pt && pt_off + npg <= kBitmapWords;
   int32_t* const ptc = reinterpret_cast<int32_t*>(s.bitmap + pt_off);
@@ -923,64 +969,77 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   for (int i = tid; i < nwords; i += NT) s.bitmap[i] = 0u;
   for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
   if (tid == 0) s.list_count[0] = 0u;
-  uint32_t mx = 0;
+  uint32_t kmin = 0xffffffffu, kmax = 0u;
+  each([&](uint32_t, uint32_t key, uint32_t) {
+    kmin = min(kmin, key);
+    kmax = max(kmax, key);
+  });
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    ch[u] -= t_key;
-    cl[u] = kIdxMax - cl[u];
-    mx = max(mx, ch[u]);
+  for (int off = 32; off >= 1; off >>= 1) {
+    kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
+    kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
-  if (lane == 0) s.wave_sum[wave] = mx;
+  if (lane == 0) {
+    s.wave_sum[wave] = kmin;
+    s.wave_sum[NT / 64 + wave] = kmax;
+  }
   __syncthreads();
-  mx = 0;
-  for (int i = 0; i < NT / 64; ++i) mx = max(mx, s.wave_sum[i]);
-  const int nb = 32 - __clz(mx);            // bits of the key part (0: all equal)
-  const int total_bits = nb + 18;
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) {
+    kmin = min(kmin, s.wave_sum[i]);
+    kmax = max(kmax, s.wave_sum[NT / 64 + i]);
+  }
+  uint8_t* const flags = reinterpret_cast<uint8_t*>(s.bitmap);
+  auto mark = [&](uint32_t pos) {
+    if (bytes) flags[pos] = 1;
+    else atomicOr(&s.bitmap[pos >> 5], 1u << (pos & 31));
+  };
+
+  // first digit, straight from the registers: 4096 bins linear in the score,
+  // so that the threshold bin holds a few candidates whatever the scores' range
+  const ScoreBins bins(kmin, kmax);
+  uint32_t remain = (uint32_t)top_k;
+  each([&](uint32_t, uint32_t key, uint32_t) { atomicAdd(&s.hist[bins.of(key)], 1u); });
+  __syncthreads();
+  find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
+  const uint32_t tb = s.tb, above = s.above, eq = s.eq;
+  remain -= above;
+  bool last = eq == remain;  // the whole bin is selected
+  if (!last && eq > (uint32_t)kListCap) return false;  // more than LDS holds (find_threshold ended with a barrier)
+  each([&](uint32_t e, uint32_t key, uint32_t pos) {
+    const uint32_t d = bins.of(key);
+    if (d > tb || (last && d == tb)) {
+      mark(pos);
+    } else if (!last && d == tb) {
+      const uint32_t slot = atomicAdd(&s.list_count[0], 1u);
+      s.list[0][slot] = (uint16_t)e;
+      if (slot < (uint32_t)kRankCap) s.rank[slot] = composite(key, pos);
+    }
+  });
+  __syncthreads();
+  if (!last && eq <= (uint32_t)kRankCap) {
+    // each of the threshold bin's candidates counts those ahead of it
+    if ((uint32_t)tid < eq) {
+      const uint64_t mine = s.rank[tid];
+      uint32_t ahead = 0;
+      for (uint32_t j = 0; j < eq; ++j) ahead += s.rank[j] > mine ? 1u : 0u;
+      if (ahead < remain) mark(kIdxMax - (uint32_t)(mine & kIdxMax));
+    }
+    last = true;
+  }
+
+  // a crowded threshold bin (many equal or nearly equal scores): radix levels
+  // of 12 bits of [ key - kmin : nb ][ (2^18-1) - position : 18 ] over its list
+  const int total_bits = 32 - __clz(kmax - kmin) + 18;
   const int nlev = (total_bits + 11) / 12;
-  auto composite = [&](uint32_t h, uint32_t p) { return ((uint64_t)h << 18) | p; };
   // digit of level L: bits [total - 12(L+1), total - 12L) of the composite
   auto digit = [&](uint64_t c, int L) {
     const int top = total_bits - 12 * L;
     const int lo_b = max(top - 12, 0);
     return (uint32_t)((c >> lo_b) & ((1ull << (top - lo_b)) - 1ull));
   };
-  auto mark = [&](uint32_t p) {
-    const uint32_t pos = kIdxMax - p;
-    atomicOr(&s.bitmap[pos >> 5], 1u << (pos & 31));
-  };
-
-  // level 0 straight from the registers
-  uint32_t remain = (uint32_t)top_k;
-  bool last;
-  {
-    const int nbins = 1 << (total_bits - max(total_bits - 12, 0));
-#pragma unroll
-    for (int u = 0; u < kPer; ++u)
-      if ((uint32_t)(u * NT + tid) < cand) atomicAdd(&s.hist[digit(composite(ch[u], cl[u]), 0)], 1u);
-    __syncthreads();
-    find_threshold<NT>(s.hist, s.wave_sum, nbins, remain, &s.tb, &s.above, &s.eq);
-    const uint32_t tb = s.tb, above = s.above, eq = s.eq;
-    remain -= above;
-    last = (eq == remain) || nlev == 1;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      if ((uint32_t)(u * NT + tid) >= cand) continue;
-      const uint32_t d = digit(composite(ch[u], cl[u]), 0);
-      if (d > tb || (last && d == tb)) {
-        mark(cl[u]);
-      } else if (!last && d == tb) {
-        const uint32_t slot = atomicAdd(&s.list_count[0], 1u);
-        s.list[0][slot] = (uint16_t)(u * NT + tid);
-      }
-    }
-    __syncthreads();
-  }
-
-  // further levels over the (short) list of the threshold bin, in LDS
   int cur = 0;
-  for (int L = 1; L < nlev && !last; ++L) {
+  for (int L = 0; L < nlev && !last; ++L) {
     const uint32_t n = s.list_count[cur];
     const int top = total_bits - 12 * L;
     const int lo_b = max(top - 12, 0);
@@ -991,20 +1050,19 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
     for (int i = tid; i < nbins; i += NT) s.hist[i] = 0u;
     if (tid == 0) s.list_count[nxt] = 0u;
     __syncthreads();
-    // the threshold bin's candidates, re-read from the row's list (L2)
-    auto cand_h = [&](uint32_t i) { return w.key[s.list[cur][i]] - t_key; };
-    auto cand_p = [&](uint32_t i) { return kIdxMax - w.pos[s.list[cur][i]]; };
-    for (uint32_t e = tid; e < n; e += NT) atomicAdd(&s.hist[digit(composite(cand_h(e), cand_p(e)), L)], 1u);
+    // the list's candidates, re-read from the row's list (L2)
+    auto cand_c = [&](uint32_t i) { return composite(w.key[s.list[cur][i]] - kmin, w.pos[s.list[cur][i]]); };
+    for (uint32_t e = tid; e < n; e += NT) atomicAdd(&s.hist[digit(cand_c(e), L)], 1u);
     __syncthreads();
     find_threshold<NT>(s.hist, s.wave_sum, nbins, remain, &s.tb, &s.above, &s.eq);
     const uint32_t tb = s.tb, above = s.above, eq = s.eq;
     remain -= above;
     last = (eq == remain) || L == nlev - 1;
     for (uint32_t e = tid; e < n; e += NT) {
-      const uint32_t h = cand_h(e), p = cand_p(e);
-      const uint32_t d = digit(composite(h, p), L);
+      const uint64_t c = cand_c(e);
+      const uint32_t d = digit(c, L);
       if (d > tb || (last && d == tb)) {
-        mark(p);
+        mark(kIdxMax - (uint32_t)(c & kIdxMax));
       } else if (!last && d == tb) {
         const uint32_t slot = atomicAdd(&s.list_count[nxt], 1u);
         s.list[nxt][slot] = s.list[cur][e];
@@ -1015,9 +1073,11 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   }
 
   // compaction in position order and output
+  __syncthreads();  // every mark is set
   uint32_t* sel = s.hist;  // 4096 entries >= top_k
   uint32_t total = 0;
-  compact_bitmap<NT>(s.bitmap, nwords, s.wave_sum, sel, top_k, &total);
+  if (bytes) compact_flags<NT>(flags, len, s.wave_sum, sel, top_k, &total);
+  else compact_bitmap<NT>(s.bitmap, nwords, s.wave_sum, sel, top_k, &total);
   if (pt_lds) {
     const uint32_t mask = (1u << page_bits) - 1u;
     for (int i = tid; i < top_k; i += NT) {
@@ -1028,24 +1088,40 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   } else {
     for (int i = tid; i < top_k; i += NT) out.emit(i, i < (int)total ? (int32_t)sel[i] : -1);
   }
+  return true;
+  };
+  if (cand >= (uint32_t)top_k && cand <= (uint32_t)RowList::kCap && select_list()) return;
+
+  // A row whose list cannot give the exact top-k (the sample misjudged its
+  // threshold, or its scores tie) is redone here, from its full logits, or
+  // left to the caller.
+  if (tid == 0) w.failed = 1u;
+  if constexpr (kRepair) {
+    repair_row_logits(rp, page_table + (int64_t)(b / pt_div) * pt_stride, b, len);
+    __syncthreads();  // the row's logits (global) are visible to the whole workgroup
+    const RowIn in{rp.logits, rp.logits_stride, seq_lens, nullptr, max_len};
+    // a repairing launch reserves the full select's LDS
+    finish_row(*reinterpret_cast<TopkSmem*>(smem_raw), in, nullptr, nullptr, page_table, pt_stride, pt_div,
+               page_bits, out_page, out_raw, top_k, b);
+  } else {
+    if (tid == 0) rp.defer_rows[atomicAdd(rp.defer_count, 1u)] = b;
+  }
 }
 
 __global__ void __launch_bounds__(kTopkThreads)
-topk_list_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, RowWs* __restrict__ ws,
+topk_list_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, DecodeList* __restrict__ ws,
                  const int32_t* __restrict__ page_table, int64_t pt_stride, int pt_div, uint32_t page_bits,
                  int32_t* __restrict__ out_page, int32_t* __restrict__ out_raw, int top_k, const RowRepair rp) {
-  list_select_row<true>(seq_lens, max_len, ws, page_table, pt_stride, pt_div, page_bits, nullptr, out_page, out_raw,
-                        top_k, rp);
+  list_select_row<true, DecodeList>(seq_lens, max_len, ws, page_table, pt_stride, pt_div, page_bits, nullptr, out_page,
+                                    out_raw, top_k, rp);
 }
 
 // Four waves per SIMD (<= 128 VGPRs): with the list layout, two workgroups per CU.
 __global__ void __launch_bounds__(kTopkThreads) __attribute__((amdgpu_waves_per_eu(4)))
-topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, RowWs* __restrict__ ws,
-                       const int32_t* __restrict__ page_table, int64_t pt_stride, int pt_div, uint32_t page_bits,
-                       const int32_t* __restrict__ offsets, int32_t* __restrict__ out_page,
-                       int32_t* __restrict__ out_raw, int top_k, const RowRepair rp) {
-  list_select_row<false>(seq_lens, max_len, ws, page_table, pt_stride, pt_div, page_bits, offsets, out_page, out_raw,
-                         top_k, rp);
+topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, PrefillList* __restrict__ ws,
+                       const int32_t* __restrict__ offsets, int32_t* __restrict__ out, int top_k,
+                       const RowRepair rp) {
+  list_select_row<false, PrefillList>(seq_lens, max_len, ws, nullptr, 0, 1, 0u, offsets, out, nullptr, top_k, rp);
 }
 
 __global__ void topk_to_physical_kernel(const int32_t* __restrict__ topk, int64_t topk_stride,
@@ -1150,18 +1226,21 @@ static int launch_topk(const RowIn& in, int batch, const int32_t* offsets, const
   return check_launch(what);
 }
 
-int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, RowWs* ws,
+int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, DecodeList* ws,
                        const int32_t* page_table, int64_t pt_stride, int pt_div, uint32_t page_bits,
-                       const int32_t* offsets, int32_t* out_page, int32_t* out_raw, int top_k, int rows,
-                       hipStream_t stream) {
+                       int32_t* out_page, int32_t* out_raw, int top_k, int rows, hipStream_t stream) {
   if (int rc = prepare_topk_kernel()) return rc;
-  if (rp.q)
-    hipLaunchKernelGGL(topk_list_kernel, dim3(rows), dim3(kTopkThreads), kTopkSmemBytes, stream, seq_lens, max_len,
-                       ws, page_table, pt_stride, pt_div, page_bits, out_page, out_raw, top_k, rp);
-  else
-    hipLaunchKernelGGL(topk_list_defer_kernel, dim3(rows), dim3(kTopkThreads), sizeof(ListSmem), stream, seq_lens,
-                       max_len, ws, page_table, pt_stride, pt_div, page_bits, offsets, out_page, out_raw, top_k, rp);
+  hipLaunchKernelGGL(topk_list_kernel, dim3(rows), dim3(kTopkThreads), kTopkSmemBytes, stream, seq_lens, max_len, ws,
+                     page_table, pt_stride, pt_div, page_bits, out_page, out_raw, top_k, rp);
   return check_launch("dsa_indexer_topk(select)");
+}
+
+int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, PrefillList* ws,
+                       const int32_t* offsets, int32_t* out, int top_k, int rows, hipStream_t stream) {
+  if (int rc = prepare_topk_kernel()) return rc;
+  hipLaunchKernelGGL(topk_list_defer_kernel, dim3(rows), dim3(kTopkThreads), sizeof(ListSmem), stream, seq_lens,
+                     max_len, ws, offsets, out, top_k, rp);
+  return check_launch("dsa_mqa_topk(select)");
 }
 
 }  // namespace dsa

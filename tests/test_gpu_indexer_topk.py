@@ -132,3 +132,39 @@ def test_fused_max_context_below_some_rows(cuda):
     g_phys, g_logi = _fused(inp, cl, max_ctx, k, 1)
     assert np.array_equal(g_logi, e_logi)
     assert np.array_equal(g_phys, e_phys)
+
+
+@pytest.mark.parametrize("lens,n", [
+    ([28672, 28673, 2048, 2049, 1], 1),        # last row whose marks are bytes, first with bits, rows at top-k
+    ([131072, 8192, 6000, 2047], 1),           # each row is sampled by its own length
+    ([131072, 2048, 2049, 7000], 2),           # entries with one row at or below top-k and one above
+    ([2048, 5], 1),                            # no page is scored
+])
+def test_ragged_batches_sample_each_row_by_its_length(cuda, lens, n):
+    print(f"ragged fused lens={lens} n={n}", flush=True)
+    inp, cl, max_ctx = _inputs(lens, n, seed=sum(lens) + n)
+    e_phys, e_logi = _unfused(inp, cl, max_ctx, 2048, n)
+    g_phys, g_logi = _fused(inp, cl, max_ctx, 2048, n)
+    assert np.array_equal(g_logi, e_logi)
+    assert np.array_equal(g_phys, e_phys)
+
+
+@pytest.mark.parametrize("length,pages,one_score", [
+    (65536, 2, False),     # 512 copies of each score: the threshold bin is too crowded to rank by counting
+    (20000, 30, False),    # about ten copies: ranked by counting, ties by position
+    (10000, 1, True),      # one score: the list fits, its threshold bin does not fit in LDS
+    (40000, 1, True),      # one score: the list overflows
+])
+def test_repeated_scores_select_the_lowest_positions(cuda, length, pages, one_score):
+    print(f"repeated scores length={length} pages={pages}", flush=True)
+    inp, cl, max_ctx = _inputs([length, 3000], 1, seed=length)
+    width = inp.block_tables.shape[1]
+    inp.block_tables[0] = inp.block_tables[0, torch.arange(width, device="cuda") % pages]
+    if one_score:
+        page = inp.cache[int(inp.block_tables[0, 0])]
+        page[:64 * 128] = page[:128].repeat(64)
+        page[64 * 128:] = page[64 * 128:64 * 128 + 4].repeat(64)
+    e_phys, e_logi = _unfused(inp, cl, max_ctx, 2048, 1)
+    g_phys, g_logi = _fused(inp, cl, max_ctx, 2048, 1)
+    assert np.array_equal(g_logi, e_logi)
+    assert np.array_equal(g_phys, e_phys)

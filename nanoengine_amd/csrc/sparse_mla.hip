@@ -102,6 +102,11 @@ constexpr float kMinLogP = -30.0f;
 constexpr int kDropExp = -30;
 constexpr int kIdxWave = 3;                // the wave that fetches the row indices (a QK wave)
 
+// Output staging of a PV wave: 32 heads x 128 dims, rows 16 bytes apart from a
+// multiple of the banks' span (heads 4 apart fall on the other half of the banks)
+constexpr int kStageRow16 = 128 * 2 + 16, kStageRow32 = 128 * 4 + 16;
+constexpr int kStageOut = 32 * kStageRow32;
+static_assert(4 * kStageOut <= kEOff, "the output staging lies in the row and P buffers");
 static_assert(kBufBytes % 1024 == 0, "a block of rows must be whole wave-wide loads");
 static_assert(kMlaSmemBytes <= 160 * 1024, "LDS budget");
 
@@ -205,6 +210,19 @@ __device__ __forceinline__ v8i lds_read32(const uint8_t* p) {
 // of the packed block: row c / 41, byte 16 (c % 41) of it. Those (row, byte)
 // pairs are loop invariants, computed once per lane (DmaLanes).
 constexpr int kTabWave = 2;  // the wave that builds the row-address table (a QK wave: the PV waves' chain is longer)
+
+// ---- the query: 64 heads x 1152 B, staged through row buffers 1 and 2 before
+// the loop. A direct load of the MFMA operands touches 32 rows with each
+// instruction and every byte twice (both key halves' waves hold all of a head
+// half's query); 72 copies of whole 1 KB runs bring each byte once while the
+// first indices and rows are on their way. Head row r is 72 16-byte pieces,
+// piece c in slot c ^ (r % 8): 1152 B is a multiple of the LDS banks' span,
+// and the swizzle spreads one piece of 8 consecutive heads over all banks.
+constexpr int kQRowBytes = 576 * 2;
+constexpr int kQPieces = kQRowBytes / 16;                          // 72
+constexpr int kQDma = kMlaHeadsPerWG * kQRowBytes / 1024;          // 72 wave-wide copies
+static_assert(kMlaHeadsPerWG * kQRowBytes <= 2 * kBufBytes, "the query fits two row buffers");
+static_assert(kQDma % kMlaWaves == 0 && kQPieces % 8 == 0, "query copies per wave, swizzle groups");
 
 // Wave-uniform state of one workgroup's loop. Blocks [0, ncached) are 64 cache
 // slots each, blocks [ncached, nblk) 32 fresh bf16 rows each.
@@ -361,6 +379,28 @@ __device__ __forceinline__ void iteration_end() {
   barrier();
 }
 
+// End of the prologue (both roles): block 0's rows have landed and the QK
+// waves' queries are in registers, so that block 1 may take their buffer.
+__device__ __forceinline__ void prologue_end() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  barrier();
+}
+
+// This wave's share of the query copies: lane l of copy i fills slot
+// 64 i + l of the staged rows. Heads past H repeat the first one.
+__device__ __forceinline__ void issue_query(const MlaParams& P, uint8_t* smem, const MlaCtx& c, int head0) {
+  const uint16_t* q = P.q + (int64_t)c.t_tok * P.q_tok_stride;
+#pragma unroll
+  for (int i = 0; i < kQDma / kMlaWaves; ++i) {
+    const int n = c.wave * (kQDma / kMlaWaves) + i;
+    const int slot = 64 * n + c.lane;
+    const int r = slot / kQPieces;
+    const int piece = (slot - r * kQPieces) ^ (r & 7);
+    const int head = head0 + r < P.H ? head0 + r : 0;
+    dma16(q + (int64_t)head * P.q_head_stride + 8 * piece, lds_addr(smem + kBufBytes + 1024 * n));
+  }
+}
+
 // QK waves: S of block t over this wave's 32 keys, its lazy reference, P(t).
 template <bool kFresh>
 __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl) {
@@ -371,17 +411,18 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
   v4i qn[8][4];
   v4i qr[4];
   {
-    const uint16_t* qh = P.q + (int64_t)c.t_tok * P.q_tok_stride + (int64_t)(c.head_ok ? c.head : 0) * P.q_head_stride;
+    const int r = 32 * hp + c32;
+    const uint8_t* qrow = smem + kBufBytes + r * kQRowBytes;
+    const int sw = 16 * (r & 7);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) qn[k][j] = *reinterpret_cast<const v4i*>(qh + 64 * k + 32 * h + 8 * j);
+      for (int j = 0; j < 4; ++j)
+        qn[k][j] = *reinterpret_cast<const v4i*>(qrow + ((16 * (8 * k + 4 * h + j)) ^ sw));
 #pragma unroll
-    for (int r = 0; r < 4; ++r) qr[r] = *reinterpret_cast<const v4i*>(qh + 512 + 16 * r + 8 * h);
+    for (int r2 = 0; r2 < 4; ++r2) qr[r2] = *reinterpret_cast<const v4i*>(qrow + ((16 * (64 + 2 * r2 + h)) ^ sw));
   }
-  // in registers before the loop: a wait the compiler places for these loads
-  // inside the loop would also wait for every copy in flight (0x0f70 = vmcnt(0))
-  __builtin_amdgcn_s_waitcnt(0x0f70);
+  prologue_end();
   float* ref = reinterpret_cast<float*>(smem + kRefOff);
   float m_run = -__builtin_inff();  // this key half's reference per head c32 (an integer, log2 units)
   float m_max = -__builtin_inff();  // exact running maximum (log2 units), for max_out
@@ -551,6 +592,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
   const uint32_t flane = (uint32_t)((4 * h + (m16 >> 2)) * kFreshRowBytes +
                                     2 * (128 * dq + 16 * (G & 1) + 4 * (m16 & 3)));
 
+  prologue_end();
   for (int t = 0; t <= c.nblk; ++t) {
     iteration_start<kFresh>(P, smem, c, dl, t);
     if (t >= 1) {
@@ -689,19 +731,28 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
     const float inv = any ? 1.f / lt : 0.f;
     const float lse = any ? (R[mt] + __builtin_amdgcn_logf(lt)) * kLn2 : -__builtin_inff();
     const int h_half = hg_base + 32 * mt;
-    if (h_half >= P.H) continue;
+    if (h_half >= P.H) break;
     const int head = h_half + c32;
     const bool head_ok = head < P.H;
+    // Through this wave's LDS staging (the row and P buffers are free), so that
+    // the stores are whole 16-byte pieces: a head's 128 dims are 256
+    // (partials: 512) contiguous bytes, where a lane holds one dim of 16 heads.
     if (P.splits == 1) {
+      uint8_t* st = smem + dq * kStageOut;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int hr = 8 * (r >> 2) + 4 * h + (r & 3);
         const float ir = __shfl(inv, 8 * (r >> 2) + hb + (r & 3), 64);
-        if (h_half + hr < P.H) {
-          uint16_t* orow = P.out + ((int64_t)c.t_tok * P.H + h_half + hr) * kMlaDv + 128 * dq + c32;
+        uint16_t* srow = reinterpret_cast<uint16_t*>(st + (8 * (r >> 2) + 4 * h + (r & 3)) * kStageRow16) + c32;
 #pragma unroll
-          for (int nn = 0; nn < 4; ++nn) orow[32 * nn] = (uint16_t)f32_to_bf16_rne(o[mt][nn][r] * ir);
-        }
+        for (int nn = 0; nn < 4; ++nn) srow[32 * nn] = (uint16_t)f32_to_bf16_rne(o[mt][nn][r] * ir);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int hr = 4 * i + (lane >> 4);
+        const v4i_alias v = *reinterpret_cast<const v4i_alias*>(st + hr * kStageRow16 + 16 * (lane & 15));
+        if (h_half + hr < P.H)
+          *reinterpret_cast<v4i_alias*>(P.out + ((int64_t)c.t_tok * P.H + h_half + hr) * kMlaDv + 128 * dq +
+                                        8 * (lane & 15)) = v;
       }
       if (dq == 0 && h == 0 && head_ok) {
         if (P.lse) P.lse[(int64_t)c.t_tok * P.H + head] = lse;
@@ -709,15 +760,20 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
       }
     } else {
       const int64_t row0 = ((int64_t)split * P.T + c.t_tok) * P.H + h_half;
+      uint8_t* st = smem + dq * kStageOut;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int hr = 8 * (r >> 2) + 4 * h + (r & 3);
         const float ir = __shfl(inv, 8 * (r >> 2) + hb + (r & 3), 64);
-        if (h_half + hr < P.H) {
-          float* orow = P.ws_o + (row0 + hr) * kMlaDv + 128 * dq + c32;
+        float* srow = reinterpret_cast<float*>(st + (8 * (r >> 2) + 4 * h + (r & 3)) * kStageRow32) + c32;
 #pragma unroll
-          for (int nn = 0; nn < 4; ++nn) orow[32 * nn] = o[mt][nn][r] * ir;
-        }
+        for (int nn = 0; nn < 4; ++nn) srow[32 * nn] = o[mt][nn][r] * ir;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int hr = 2 * i + h;
+        const v4i_alias v = *reinterpret_cast<const v4i_alias*>(st + hr * kStageRow32 + 16 * c32);
+        if (h_half + hr < P.H)
+          *reinterpret_cast<v4i_alias*>(P.ws_o + (row0 + hr) * kMlaDv + 128 * dq + 4 * c32) = v;
       }
       if (dq == 0 && h == 0 && head_ok) P.ws_lse[row0 + c32] = lse;
     }
@@ -761,25 +817,25 @@ sparse_mla_kernel(const MlaParams P) {
   c.head = c.h_half + c.c32;
   c.head_ok = c.head < P.H;
 
-  // prologue: the indices of blocks 0-3, the address tables of blocks 0 and
-  // 1, block 0's rows
-  if (c.wave == kIdxWave) {
+  // prologue: the indices of blocks 0-3 and the query go out together, then
+  // the address tables of blocks 0 and 1, then block 0's rows
+  if (c.wave == kIdxWave)
     for (int j = 0; j < 4 && j < c.nblk; ++j) issue_index<kFresh>(P, smem, c, j);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  barrier();
+  issue_query(P, smem, c, hg * kMlaHeadsPerWG);
   const DmaLanes dl = dma_lanes(c.wave, c.lane);
+  if (c.wave == kIdxWave)  // its index copies landed (the query's may still be on their way)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kQDma / kMlaWaves) : "memory");
+  barrier();
   if (c.wave == kTabWave) {
     if (c.nblk > 0) build_addr_table<kFresh>(P, smem, c, 0);
     if (c.nblk > 1) build_addr_table<kFresh>(P, smem, c, 1);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's query copies
   barrier();
   if (c.nblk > 0) {
     if (!kFresh || c.ncached > 0) issue_block(smem, 0, dl, smem, c.wave);
     else issue_fresh_block(smem, 0, smem, c.wave, c.lane);
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  barrier();  // block 0's rows are in LDS
   // both roles run the same number of iterations and barriers
   if (c.wave < 4) qk_waves<kFresh>(P, smem, c, dl);
   else pv_waves<kFresh>(P, smem, c, dl, split);

@@ -402,7 +402,7 @@ __device__ __forceinline__ void issue_query(const MlaParams& P, uint8_t* smem, c
 }
 
 // QK waves: S of block t over this wave's 32 keys, its lazy reference, P(t).
-template <bool kFresh>
+template <bool kFresh, int kTiles>
 __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl) {
   const int lane = c.lane, h = c.h, c32 = c.c32, hp = c.hp, kh = c.kh;
   // the query as the B operand over all dims: nope chunk k (64 dims), k-step j =
@@ -435,7 +435,7 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
     if (c.wave == kTabWave && t + 2 < c.nblk) build_addr_table<kFresh>(P, smem, c, t + 2);
     // a fresh block has 32 keys, all in key half 0
     const bool fresh = kFresh && t >= c.ncached;
-    if (t < c.nblk && !(fresh && kh == 1)) {
+    if (t < c.nblk && !(fresh && kh == 1) && hp < kTiles) {
       const uint8_t* buf = smem + (t % kNumBufs) * kBufBytes;
       const int32_t slot_t = reinterpret_cast<const int32_t*>(smem + kRingOff + (t % kRingSlots) * 256)[lane];
       const uint64_t vmask = __ballot(fresh ? fresh_valid(P, slot_t, lane) : slot_valid(P, slot_t));
@@ -462,15 +462,27 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
       const uint8_t* row = buf + (32 * kh + c32) * kMlaRowBytes;
       const v4f ksc = *reinterpret_cast<const v4f*>(row + 512);
       const uint8_t* krow = row + 32 * h;
-      v8i kraw[2];
-      kraw[0] = lds_read32(krow);
+      // Chunks are read D ahead, and the schedule barriers keep them there: left
+      // alone, the compiler moves each read down to its first use and every
+      // chunk waits out the LDS latency (128 tokens: 88.4 -> 85.3 us with the
+      // same in the P.V loop).
+      constexpr int D = 2;
+      v8i kraw[D + 1];
+      v4i rope[4];
+#pragma unroll
+      for (int k = 0; k < D; ++k) kraw[k] = lds_read32(krow + 64 * k);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        if (k + 1 < 8) kraw[(k + 1) & 1] = lds_read32(krow + 64 * (k + 1));
+        if (k + D < 8) kraw[(k + D) % (D + 1)] = lds_read32(krow + 64 * (k + D));
+        else
+#pragma unroll
+          for (int r = 2 * (k + D - 8); r < 2 * (k + D - 8) + 2; ++r)
+            rope[r] = *reinterpret_cast<const v4i*>(row + 528 + 32 * r + 16 * h);
+        __builtin_amdgcn_sched_barrier(0);
         const float sc = ksc[k >> 1];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const v8i& kr = kraw[k & 1];
+          const v8i& kr = kraw[k % (D + 1)];
           v4i kb;
           kb[0] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(kr[2 * j], sc, false));
           kb[1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(kr[2 * j], sc, true));
@@ -478,12 +490,11 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
           kb[3] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(kr[2 * j + 1], sc, true));
           s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kb), as_v8bf(qn[k][j]), s, 0, 0, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const v4i rope = *reinterpret_cast<const v4i*>(row + 528 + 32 * r + 16 * h);
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(rope), as_v8bf(qr[r]), s, 0, 0, 0);
-      }
+      for (int r = 0; r < 4; ++r)
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(rope[r]), as_v8bf(qr[r]), s, 0, 0, 0);
       }
       // invalid keys score -inf (their rows are zeros); the masks are skipped
       // when every key of the block is valid, the usual case
@@ -500,7 +511,11 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
       float mloc = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
       mloc = fmaxf(mloc, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])),
                                fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
-      mloc = fmaxf(mloc, shfl_xor(mloc, 32));
+      {
+        // the other lane half's maximum (the swap pairs the two halves)
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+        mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      }
       const float mblk = mloc * P.scale_log2;
       m_max = fmaxf(m_max, mblk);
       // lazy reference: it moves (to an integer) only when a block exceeds it by 2^8
@@ -520,10 +535,10 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
         for (int r = 0; r < 16; ++r)
           if (!((vb16 >> r) & 1u)) pv[r] = 0.f;
       }
-      float lsum = 0.f;
+      float ls4[4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) lsum += pv[r];
-      l_run += lsum;
+      for (int r = 0; r < 4; ++r) ls4[r] = (pv[r] + pv[4 + r]) + (pv[8 + r] + pv[12 + r]);
+      l_run += (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
       if (fresh && !all_valid) {
         // An invalid key's V is the zero row, so any finite P' leaves O alone.
         // The PV waves scale a fresh block's P by adding f in [-30, 0] to the
@@ -562,7 +577,7 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
 // Wave dq = w - 4 owns O[64 heads x dims 128dq .. 128dq+127], exactly V tile
 // dq, as two head tiles (the head halves): each V byte is converted once per
 // workgroup, and one exponent per key scales both tiles' P.
-template <bool kFresh>
+template <bool kFresh, int kTiles>
 __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl,
                                          int split) {
   const int lane = c.lane, h = c.h, c32 = c.c32, dq = c.wave - 4;
@@ -572,14 +587,16 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
   // may alias them (so the reads stay after the writes)
   typedef int v4i_alias __attribute__((ext_vector_type(4), may_alias));
   uint16_t* et = reinterpret_cast<uint16_t*>(smem + kEOff) + dq * 256;
-  v16f o[2][4];  // o[mt][nn][r]: head 32mt + 8(r/4) + 4h + r%4 of the workgroup, dim 128dq + 32nn + c32
+  v16f o[kTiles][4];  // o[mt][nn][r]: head 32mt + 8(r/4) + 4h + r%4 of the workgroup, dim 128dq + 32nn + c32
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
+  for (int mt = 0; mt < kTiles; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[mt][i][r] = 0.f;
-  float R[2] = {-__builtin_inff(), -__builtin_inff()};  // reference of O per head tile, head c32 (log2 units)
+  float R[kTiles];  // reference of O per head tile, head c32 (log2 units)
+#pragma unroll
+  for (int mt = 0; mt < kTiles; ++mt) R[mt] = -__builtin_inff();
   // transposing V reads: lane (G = lane/16, m = lane%16) addresses key row
   // 8(e/4) + 4h + e%4 (e = m/2) and dims (G%2)*16 + 8(m%2) of each 32-dim tile
   const int m16 = lane & 15, G = lane >> 4;
@@ -610,9 +627,9 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
       }
       // each head tile's O follows the larger of its key-half references; O
       // moves by a power of two
-      int fx[2][2];
+      int fx[kTiles][2];
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
+      for (int mt = 0; mt < kTiles; ++mt) {
         const float m0 = ref[((par * 2 + mt) * 2 + 0) * 32 + c32];
         const float m1 = ref[((par * 2 + mt) * 2 + 1) * 32 + c32];
         const float mn = fmaxf(m0, m1);
@@ -655,13 +672,13 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
       // k-step ks: its P (both head tiles), exponent and V reads issued one
       // k-step ahead
       v2i vq[2][4];
-      v4i pq[2][2], eq[2];
+      v4i pq[2][kTiles], eq[2];
       {
         const uint32_t a0 = vaddr(0);
 #pragma unroll
         for (int nn = 0; nn < 4; ++nn) vq[0][nn] = lds_read_tr8_at(a0 + 32 * nn);
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) pq[0][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + lane * 16);
+        for (int mt = 0; mt < kTiles; ++mt) pq[0][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + lane * 16);
         eq[0] = *reinterpret_cast<const v4i_alias*>(et + h * 8);
       }
 #pragma unroll
@@ -672,15 +689,16 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
 #pragma unroll
           for (int nn = 0; nn < 4; ++nn) vq[nxt][nn] = lds_read_tr8_at(a1 + 32 * nn);
 #pragma unroll
-          for (int mt = 0; mt < 2; ++mt)
+          for (int mt = 0; mt < kTiles; ++mt)
             pq[nxt][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + ((ks + 1) * 64 + lane) * 16);
           eq[nxt] = *reinterpret_cast<const v4i_alias*>(et + ((ks + 1) * 2 + h) * 8);
         }
+        __builtin_amdgcn_sched_barrier(0);
         const int k2 = ks >> 1;  // k-steps 0, 1: key half 0; 2, 3: key half 1
         if (fresh && ks >= 2) continue;  // a fresh block's 32 keys are k-steps 0, 1
-        v4i pa[2];
+        v4i pa[kTiles];
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < kTiles; ++mt)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             // (bit_cast of a vector element reads element 0; copy to scalars first)
@@ -704,7 +722,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
             vop = fp8x8_to_bf16(vq[cur][nn]);
           }
 #pragma unroll
-          for (int mt = 0; mt < 2; ++mt)
+          for (int mt = 0; mt < kTiles; ++mt)
             o[mt][nn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(pa[mt]), vop, o[mt][nn], 0, 0, 0);
         }
       }
@@ -717,7 +735,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
   int hb = 4 * h;
   asm volatile("" : "+v"(hb));
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
+  for (int mt = 0; mt < kTiles; ++mt) {
     // total of P per head c32 of tile mt against R, and the exact maximum
     float lt = 0.f, mm = -__builtin_inff();
 #pragma unroll
@@ -782,7 +800,11 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
 
 // kFresh: a chunked prefill's token lists (cache slots, then fresh bf16 rows);
 // decode instantiates the kernel without that path.
-template <bool kFresh>
+// kTiles: the workgroup's head tiles of 32. With at most 32 heads in all (a
+// tensor-parallel rank's 16) the second tile would be padding: its score waves
+// idle and its P.V products are left out. (As a run-time condition this cost
+// the 64-head kernel 5%: the branches stop the P.V loop's read-ahead.)
+template <bool kFresh, int kTiles>
 __global__ void __launch_bounds__(kMlaThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 sparse_mla_kernel(const MlaParams P) {
   extern __shared__ __align__(16) uint8_t smem[];
@@ -837,8 +859,8 @@ sparse_mla_kernel(const MlaParams P) {
     else issue_fresh_block(smem, 0, smem, c.wave, c.lane);
   }
   // both roles run the same number of iterations and barriers
-  if (c.wave < 4) qk_waves<kFresh>(P, smem, c, dl);
-  else pv_waves<kFresh>(P, smem, c, dl, split);
+  if (c.wave < 4) qk_waves<kFresh, kTiles>(P, smem, c, dl);
+  else pv_waves<kFresh, kTiles>(P, smem, c, dl, split);
 }
 
 // One 64-thread workgroup per (token, head): merge the split partials.
@@ -953,12 +975,11 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
 
   static int smem_status = -1;
   if (smem_status < 0) {
-    smem_status = hipFuncSetAttribute((const void*)sparse_mla_kernel<false>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMlaSmemBytes) == hipSuccess &&
-                          hipFuncSetAttribute((const void*)sparse_mla_kernel<true>,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (int)kMlaSmemBytes) == hipSuccess
-                      ? 0 : 1;
+    smem_status = 0;
+    for (const void* k : {(const void*)sparse_mla_kernel<false, 1>, (const void*)sparse_mla_kernel<false, 2>,
+                          (const void*)sparse_mla_kernel<true, 1>, (const void*)sparse_mla_kernel<true, 2>})
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMlaSmemBytes) != hipSuccess)
+        smem_status = 1;
   }
   if (smem_status) return set_error(kLaunchFailed, "sparse_mla: cannot reserve %zu B of LDS", kMlaSmemBytes);
 
@@ -1010,12 +1031,10 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
     P.ws_lse = P.ws_o + rows * kMlaDv;
   }
   const int64_t nwg = (int64_t)num_tokens * P.head_groups * num_splits;
-  if (fresh)
-    hipLaunchKernelGGL(sparse_mla_kernel<true>, dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes,
-                       (hipStream_t)stream, P);
-  else
-    hipLaunchKernelGGL(sparse_mla_kernel<false>, dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes,
-                       (hipStream_t)stream, P);
+  void (*const kernel)(MlaParams) = num_heads <= 32
+                                        ? (fresh ? sparse_mla_kernel<true, 1> : sparse_mla_kernel<false, 1>)
+                                        : (fresh ? sparse_mla_kernel<true, 2> : sparse_mla_kernel<false, 2>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes, (hipStream_t)stream, P);
   if (int rc = check_launch("dsa_sparse_mla_decode")) return rc;
   if (num_splits > 1) {
     hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)(num_tokens * num_heads)), dim3(64), 0,

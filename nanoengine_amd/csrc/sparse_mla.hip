@@ -124,6 +124,7 @@ struct MlaParams {
   const int32_t* idx;
   int64_t idx_stride;
   int T, H, topk, splits, head_groups;
+  int whole;  // (token, head group) items [0, whole) are not split, the others `splits` ways
   float scale_log2;
   uint16_t* out;
   float* lse;
@@ -755,7 +756,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
     // Through this wave's LDS staging (the row and P buffers are free), so that
     // the stores are whole 16-byte pieces: a head's 128 dims are 256
     // (partials: 512) contiguous bytes, where a lane holds one dim of 16 heads.
-    if (P.splits == 1) {
+    if (split < 0) {
       uint8_t* st = smem + dq * kStageOut;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -815,19 +816,26 @@ sparse_mla_kernel(const MlaParams P) {
   c.c32 = c.lane & 31;
   c.hp = (c.wave & 3) >> 1;
   c.kh = c.wave & 1;
-  // XCD-aware order: consecutive logical work items (the head groups and
-  // splits of one token) land on the same XCD and share its L2.
-  const int nwg = gridDim.x;
-  int work = blockIdx.x;
-  if ((nwg & 7) == 0) work = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);
-  const int per_tok = P.head_groups * P.splits;
-  c.t_tok = work / per_tok;
-  const int rem = work % per_tok;
-  const int hg = rem / P.splits;
-  const int split = rem % P.splits;
-  const int chunk = P.topk / P.splits;
-  c.key_begin = split * chunk;
-  c.nblk = chunk / kMlaKeys;
+  // Whole items first, one workgroup each, then the splits of the others. Each
+  // part in XCD-aware order: workgroups go to the XCDs round robin, and the
+  // units (all head groups and splits of a token) are dealt to the XCDs in
+  // turn, so that a unit shares one L2 and the XCDs share a prefill's longer
+  // tokens evenly (runs of consecutive tokens per XCD: 460 -> 633 us on a
+  // causal batch without cached prefix). The last units, fewer than 8, go in order.
+  const bool is_whole = (int)blockIdx.x < P.whole;
+  const int part = is_whole ? P.whole : (int)gridDim.x - P.whole;
+  const int wg = is_whole ? blockIdx.x : blockIdx.x - P.whole;
+  const int unit = is_whole ? P.head_groups : P.head_groups * P.splits;
+  int work = wg;
+  if (wg < (part / unit & ~7) * unit) work = ((wg >> 3) / unit * 8 + (wg & 7)) * unit + (wg >> 3) % unit;
+  const int item = is_whole ? work : P.whole + work / P.splits;
+  const int split = is_whole || P.splits == 1 ? -1 : work % P.splits;
+  c.t_tok = item / P.head_groups;
+  const int hg = item % P.head_groups;
+  const int blocks = P.topk / kMlaKeys;
+  const int first = split < 0 ? 0 : blocks * split / P.splits;
+  c.key_begin = first * kMlaKeys;
+  c.nblk = (split < 0 ? blocks : blocks * (split + 1) / P.splits) - first;
   c.ncached = c.nblk;
   if (kFresh) {
     const int nc = __builtin_amdgcn_readfirstlane(P.counts[2 * c.t_tok]);
@@ -863,11 +871,14 @@ sparse_mla_kernel(const MlaParams P) {
   else pv_waves<kFresh, kTiles>(P, smem, c, dl, split);
 }
 
-// One 64-thread workgroup per (token, head): merge the split partials.
+// One 64-thread workgroup per (split item, head): merge the split partials.
 __global__ void __launch_bounds__(64)
-sparse_mla_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_lse, int T, int H,
-                          int splits, uint16_t* __restrict__ out, float* __restrict__ lse_out) {
-  const int th = blockIdx.x;
+sparse_mla_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_lse, int T, int H, int whole,
+                          int head_groups, int splits, uint16_t* __restrict__ out, float* __restrict__ lse_out) {
+  const int item = whole + (int)blockIdx.x / kMlaHeadsPerWG;
+  const int head = item % head_groups * kMlaHeadsPerWG + (int)blockIdx.x % kMlaHeadsPerWG;
+  if (head >= H) return;
+  const int64_t th = (int64_t)(item / head_groups) * H + head;
   const int64_t stride = (int64_t)T * H;
   float m = -__builtin_inff();
   for (int s = 0; s < splits; ++s) m = fmaxf(m, ws_lse[s * stride + th]);
@@ -891,7 +902,7 @@ sparse_mla_combine_kernel(const float* __restrict__ ws_o, const float* __restric
   v4i v;
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = (int)pack_bf16_rne(acc[2 * e] * inv, acc[2 * e + 1] * inv);
-  *reinterpret_cast<v4i*>(out + (int64_t)th * kMlaDv + threadIdx.x * 8) = v;
+  *reinterpret_cast<v4i*>(out + th * kMlaDv + threadIdx.x * 8) = v;
   if (threadIdx.x == 0 && lse_out) lse_out[th] = wsum > 0.f ? m + logf(wsum) : -__builtin_inff();
 }
 
@@ -903,18 +914,16 @@ int dsa_sparse_mla_num_splits(int num_tokens, int num_heads, int topk, int num_c
   if (num_tokens <= 0 || num_heads <= 0 || topk <= 0) return 1;
   if (num_cus <= 0) num_cus = 256;
   const int groups = (num_heads + dsa::kMlaHeadsPerWG - 1) / dsa::kMlaHeadsPerWG;
-  const int64_t base = (int64_t)num_tokens * groups;
-  // A workgroup's time is a fixed start-up plus a cost per 64-row block, and
-  // one workgroup runs per CU at a time: split as far as the grid still fits
-  // the CUs in one round (a second round costs a whole workgroup's time), and
-  // keep at least 4 blocks per workgroup (below that the start-up and the
-  // combine outweigh the shorter key list). Splits must divide topk into
-  // 64-row blocks.
-  const int max_splits = std::min(8, topk / (4 * dsa::kMlaKeys));
-  int splits = 1;
-  while (splits * 2 <= max_splits && base * splits * 2 <= num_cus && (topk / (splits * 2)) % dsa::kMlaKeys == 0)
-    splits *= 2;
-  return splits;
+  // A workgroup's time is a fixed start-up (~8 us) plus a cost per 64-row block
+  // (2 to 2.6 us), and one workgroup runs per CU at a time. The items that fill
+  // the CUs in whole rounds are not split; the remaining ones (all of a small
+  // batch) split as far as they still fit the CUs in one round, with at least 4
+  // blocks per workgroup (below that the start-up and the combine outweigh the
+  // shorter key list). Block counts may differ by one.
+  const int64_t rest = ((int64_t)num_tokens * groups) % num_cus;
+  if (rest == 0) return 1;
+  const int most = std::min(8, topk / (4 * dsa::kMlaKeys));
+  return std::max(1, (int)std::min<int64_t>(most, num_cus / rest));
 }
 
 size_t dsa_sparse_mla_workspace_bytes(int num_tokens, int num_heads, int num_splits) {
@@ -961,14 +970,22 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
     return set_error(kInvalidArgument, "sparse_mla: q, kv_cache and out must be 16-byte aligned");
   if ((q_token_stride % 8) || (q_head_stride % 8))
     return set_error(kInvalidArgument, "sparse_mla: q strides must be multiples of 8 elements");
-  if (num_splits <= 0) {
+  // the rule's split count leaves whole rounds of items unsplit; any other one
+  // splits every item into equal parts
+  const int64_t items = (int64_t)num_tokens * ((num_heads + kMlaHeadsPerWG - 1) / kMlaHeadsPerWG);
+  int64_t whole = 0;
+  if (num_splits != 1) {
     int dev = 0;
     (void)hipGetDevice(&dev);
-    num_splits = dsa_sparse_mla_num_splits(num_tokens, num_heads, topk, dsa_num_cus(dev));
+    const int cus = std::max(1, dsa_num_cus(dev));
+    const int rule = dsa_sparse_mla_num_splits(num_tokens, num_heads, topk, cus);
+    if (num_splits <= 0) num_splits = rule;
+    if (num_splits == rule)
+      whole = items - items % cus;
+    else if (num_splits > topk / kMlaKeys || (topk / num_splits) % kMlaKeys != 0 || topk % num_splits != 0)
+      return set_error(kInvalidArgument, "sparse_mla: num_splits=%d does not split topk=%d into 64-row blocks",
+                       num_splits, topk);
   }
-  if (num_splits > topk / kMlaKeys || (topk / num_splits) % kMlaKeys != 0 || topk % num_splits != 0)
-    return set_error(kInvalidArgument, "sparse_mla: num_splits=%d does not split topk=%d into 64-row blocks",
-                     num_splits, topk);
   const size_t need = dsa_sparse_mla_workspace_bytes(num_tokens, num_heads, num_splits);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(kWorkspaceTooSmall, "sparse_mla: workspace %zu B < %zu B", workspace_bytes, need);
@@ -998,6 +1015,7 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
   P.H = num_heads;
   P.topk = topk;
   P.splits = num_splits;
+  P.whole = (int)whole;
   P.head_groups = (num_heads + kMlaHeadsPerWG - 1) / kMlaHeadsPerWG;
   P.scale_log2 = sm_scale * kLog2e;
   P.out = static_cast<uint16_t*>(out);
@@ -1030,15 +1048,16 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
     P.ws_o = static_cast<float*>(workspace);
     P.ws_lse = P.ws_o + rows * kMlaDv;
   }
-  const int64_t nwg = (int64_t)num_tokens * P.head_groups * num_splits;
+  const int64_t nwg = whole + (items - whole) * num_splits;
   void (*const kernel)(MlaParams) = num_heads <= 32
                                         ? (fresh ? sparse_mla_kernel<true, 1> : sparse_mla_kernel<false, 1>)
                                         : (fresh ? sparse_mla_kernel<true, 2> : sparse_mla_kernel<false, 2>);
   hipLaunchKernelGGL(kernel, dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes, (hipStream_t)stream, P);
   if (int rc = check_launch("dsa_sparse_mla_decode")) return rc;
   if (num_splits > 1) {
-    hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)(num_tokens * num_heads)), dim3(64), 0,
-                       (hipStream_t)stream, P.ws_o, P.ws_lse, num_tokens, num_heads, num_splits, P.out, lse);
+    hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)((items - whole) * kMlaHeadsPerWG)), dim3(64), 0,
+                       (hipStream_t)stream, P.ws_o, P.ws_lse, num_tokens, num_heads, P.whole, P.head_groups,
+                       num_splits, P.out, lse);
     return check_launch("dsa_sparse_mla_decode(combine)");
   }
   return kOk;

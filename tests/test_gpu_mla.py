@@ -288,3 +288,31 @@ def test_qk_score_error_bound(cuda):
     hi = O.fp8_e4m3fn_decode(O.fp8_e4m3fn_encode(x / s_hi)) * s_hi
     err_hi = np.abs(np.einsum("thcd,tcd->th", hi - x, k[:, :512].reshape(-1, 8, 64)))
     assert np.median(err_hi / bound) > 100
+
+
+@pytest.mark.parametrize("T,H,K", [
+    (20, 128, 2048),    # six splits of five or six blocks
+    (40, 128, 2048),    # three splits of ten or eleven blocks
+    (130, 128, 2048),   # one whole round of workgroups, the last two tokens split eight ways
+    (257, 16, 512),     # one head tile; the last token split in two
+    (90, 192, 2048),    # three head groups: the split items begin inside a token
+    (5, 96, 320),       # five blocks: not split
+])
+def test_chosen_splits_match_the_unsplit_kernel(cuda, T, H, K):
+    """The split rule's partition against one workgroup per (token, head
+    group). P = bf16(2^(s - m)): another reference m moves the f32 rounding of
+    s - m, so a P near a rounding boundary may differ by one ulp, 2^-8 of it.
+    Over all keys that is at most 2^-8 of the softmax-weighted mean of |v|,
+    which is below 1 for N(0, 1) rows; each side then rounds o to bf16
+    (together 2^-8 |o|). The LSE sums P before its rounding: 1e-5 holds it."""
+    splits = ops.sparse_mla_num_splits(T, H, K, cuda)
+    print(f"mla splits T={T} H={H} K={K} splits={splits}", flush=True)
+    q, kv, idx = _case(T, H, K, num_blocks=80, seed=T + H + K)
+    o, lse = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5)
+    o1, lse1 = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5, num_splits=1)
+    torch.cuda.synchronize()
+    a, b = o.float(), o1.float()
+    assert torch.all((a - b).abs() <= 2.0 ** -8 * (torch.maximum(a.abs(), b.abs()) + 1.0))
+    fin = torch.isfinite(lse1)
+    assert torch.equal(torch.isfinite(lse), fin)
+    assert torch.all((lse[fin] - lse1[fin]).abs() <= 1e-5)

@@ -96,4 +96,6 @@ def check(status: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    status = getattr(_lib or load(), name)(*args)
+    if status != 0:
+        check(status, name)

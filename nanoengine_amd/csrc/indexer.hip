@@ -401,6 +401,9 @@ indexer_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
 // are staged per wave in LDS (wave-uniform counters, no LDS atomics) and
 // flushed to the row's list with one global atomic when the batch entry
 // changes, when the stage could overflow, and at the end.
+//
+// kStore: the pages' order keys go to keys[row * key_stride + t] instead (the
+// score pass of short contexts, whose select reads whole rows).
 constexpr int kFiltStageCap = 384;   // staged candidates per wave and query token
 constexpr int kFiltWindow = 64;      // block-table entries a wave holds (one per lane)
 constexpr int kFiltAdvance = 60;     // pages per window refill (a multiple of the 3- and 4-buffer rotations)
@@ -415,12 +418,12 @@ constexpr size_t filt_smem_bytes(int batch) {
 }
 static_assert(2 * filt_smem_bytes(kFiltMaxBatch) <= 160 * 1024, "two filter workgroups per CU at the largest batch");
 
-template <int NQ>
+template <int NQ, bool kStore>
 __global__ void __launch_bounds__(kIdxThreads) __attribute__((amdgpu_waves_per_eu(2)))
 indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kv,
                       const float* __restrict__ weights, const int32_t* __restrict__ ctx_lens,
                       const int32_t* __restrict__ block_tables, int64_t bt_stride, int64_t max_ctx, int batch,
-                      int top_k, DecodeList* __restrict__ ws) {
+                      int top_k, DecodeList* __restrict__ ws, uint32_t* __restrict__ keys, int64_t key_stride) {
   extern __shared__ __align__(16) uint8_t fl_smem[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   FiltWaveStage& st = reinterpret_cast<FiltWaveStage*>(fl_smem)[wave];
@@ -503,7 +506,7 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
 
   auto flush = [&](int j) {
     const int c = cnt[j];
-    if (c == 0) return;
+    if (kStore || c == 0) return;
     DecodeList& rw = ws[cur_b * NQ + j];
     uint32_t base = 0;
     if (lane == 0) base = atomicAdd(&rw.count, (uint32_t)c);
@@ -530,7 +533,7 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
         for (int r = 0; r < 4; ++r) w[j][ht][r] = wq[ht * 16 + (lane >> 4) * 4 + r];
       }
       L[j] = (int)min((int64_t)ctx_lens[b * NQ + j], max_ctx);
-      tk[j] = ws[b * NQ + j].t_key;
+      tk[j] = kStore ? 0u : ws[b * NQ + j].t_key;
     }
   };
 
@@ -548,6 +551,10 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
       const float v = page_head_sum<NQ>(pr, j, lane, qa, w);
       const int t = page * kIdxPageTokens + lane;
       const uint32_t key = order_key(v * pr.scale);
+      if constexpr (kStore) {
+        if (t < L[j]) keys[(int64_t)(b * NQ + j) * key_stride + t] = key;
+        continue;
+      }
       const bool pred = t < L[j] && key >= tk[j];
       const uint64_t m = __ballot(pred);
       if (pred) {
@@ -594,29 +601,28 @@ static int filter_grid() {
   return grid;
 }
 
-// The persistent filter pass; false when the batch does not fit its LDS prefix.
+// The persistent filter (or, with keys, score) pass; false when the batch does
+// not fit its LDS prefix.
 static bool launch_filter_persistent(const uint8_t* q, const uint8_t* kv, const float* weights,
                                      const int32_t* ctx_lens, const int32_t* bt, int64_t bt_stride, int batch,
-                                     int next_n, int64_t max_ctx, int top_k, DecodeList* ws, hipStream_t stream) {
+                                     int next_n, int64_t max_ctx, int top_k, DecodeList* ws, uint32_t* keys,
+                                     int64_t key_stride, hipStream_t stream) {
   if (batch > kFiltMaxBatch) return false;
   const size_t smem = filt_smem_bytes(batch);
+  using Kernel = decltype(&indexer_filter_kernel<1, false>);
+  static const Kernel kernels[2][2] = {{indexer_filter_kernel<1, false>, indexer_filter_kernel<1, true>},
+                                       {indexer_filter_kernel<2, false>, indexer_filter_kernel<2, true>}};
   static bool attr_set = false;
   if (!attr_set) {
-    const int max_smem = (int)filt_smem_bytes(kFiltMaxBatch);
-    if (hipFuncSetAttribute((const void*)indexer_filter_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            max_smem) != hipSuccess ||
-        hipFuncSetAttribute((const void*)indexer_filter_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            max_smem) != hipSuccess)
-      return false;
+    for (const auto& row : kernels)
+      for (Kernel k : row)
+        if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)filt_smem_bytes(kFiltMaxBatch)) != hipSuccess)
+          return false;
     attr_set = true;
   }
-  const dim3 grid((unsigned)filter_grid());
-  if (next_n == 1)
-    hipLaunchKernelGGL(indexer_filter_kernel<1>, grid, dim3(kIdxThreads), smem, stream, q, kv, weights, ctx_lens, bt,
-                       bt_stride, max_ctx, batch, top_k, ws);
-  else
-    hipLaunchKernelGGL(indexer_filter_kernel<2>, grid, dim3(kIdxThreads), smem, stream, q, kv, weights, ctx_lens, bt,
-                       bt_stride, max_ctx, batch, top_k, ws);
+  hipLaunchKernelGGL(kernels[next_n - 1][keys ? 1 : 0], dim3((unsigned)filter_grid()), dim3(kIdxThreads), smem, stream,
+                     q, kv, weights, ctx_lens, bt, bt_stride, max_ctx, batch, top_k, ws, keys, key_stride);
   return true;
 }
 
@@ -728,6 +734,23 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
     if (phase_events && phase_events[i]) (void)hipEventRecord((hipEvent_t)phase_events[i], st);
   };
   mark(0);
+  // Short contexts: every score (as order keys, in the logits buffer), then a
+  // select over whole rows. The sample pass and the list, which pay for
+  // themselves on long rows, are two thirds of the indexer's time on short ones.
+  if (max_context_len <= kRowSelectLen) {
+    uint32_t* keys = reinterpret_cast<uint32_t*>(f.logits);
+    if (launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
+                                 next_n, max_context_len, top_k, nullptr, keys, f.logits_stride, st)) {
+      if (int rc = check_launch("dsa_indexer_topk(scores)")) return rc;
+      mark(1);
+      mark(2);
+      const int rc = launch_row_select(keys, f.logits_stride, context_lens, max_context_len, block_tables,
+                                       block_table_stride, next_n, 6u, out_physical, out_logical, top_k, rows, st);
+      mark(3);
+      mark(4);
+      return rc;
+    }
+  }
   const int64_t max_pages = (max_context_len + kIdxPageTokens - 1) / kIdxPageTokens;
   // 1-2. logits of sampled pages (one workgroup per batch entry, kept in LDS)
   // -> each row's score threshold, lists reset
@@ -738,7 +761,7 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
   mark(1);
   // 3. all pages: candidates at or above the threshold into the row lists
   if (!launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
-                                next_n, max_context_len, top_k, f.ws, st)) {
+                                next_n, max_context_len, top_k, f.ws, nullptr, 0, st)) {
     IdxOut o_f{nullptr, 0, f.ws, top_k};
     launch_indexer<kIdxFilter>(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
                                next_n, max_context_len, max_pages, o_f, st);

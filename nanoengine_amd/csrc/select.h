@@ -1,0 +1,84 @@
+// Device helpers of the exact selects: key and score conversion, the linear
+// score bins, the block scan and the composite rank (gfx950).
+#pragma once
+
+#include "dsa_common.h"
+
+namespace dsa {
+
+constexpr int kHistBins = 4096;
+constexpr uint32_t kIdxMax = (1u << 18) - 1;  // positions are at most this
+constexpr int kRankCap = 384;                 // threshold-bin candidates ranked by counting
+
+// (score, lower position first) as one integer: every element is distinct.
+__device__ __forceinline__ uint64_t rank_composite(uint32_t key, uint32_t pos) {
+  return ((uint64_t)key << 18) | (kIdxMax - pos);
+}
+
+// Inverse of order_key: the float whose key is k.
+__device__ __forceinline__ float key_to_float(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k);
+}
+
+// Exclusive block prefix sum of one value per thread; returns the prefix and
+// writes the block total to *total (all threads).
+template <int NT>
+__device__ uint32_t block_exclusive_scan(uint32_t* wave_sum, uint32_t x, uint32_t* total) {
+  constexpr int kWaves = NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t v = x;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    uint32_t n = __shfl_up(v, off, 64);
+    if (lane >= off) v += n;
+  }
+  __syncthreads();
+  if (lane == 63) wave_sum[wave] = v;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+  for (int w = 0; w < kWaves; ++w) {
+    uint32_t t = wave_sum[w];
+    if (w < wave) before += t;
+    all += t;
+  }
+  *total = all;
+  return before + v - x;
+}
+
+// 4096 bins linear in the score between the scores of keys kmin and kmax. The
+// bin never decreases with the key (subtraction, multiplication by a positive
+// scale and truncation are each monotone, +-0 share a bin), so a candidate in
+// a higher bin ranks ahead. Scores that are not finite, or whose range is not,
+// fall into the end bins or all into one.
+struct ScoreBins {
+  float lo, scale;
+  __device__ __forceinline__ ScoreBins(uint32_t kmin, uint32_t kmax) {
+    lo = key_to_float(kmin);
+    const float range = key_to_float(kmax) - lo;
+    scale = range > 0.f && range < 3.0e38f ? (float)(kHistBins - 1) / range : 0.f;
+  }
+  __device__ __forceinline__ uint32_t of(uint32_t key) const {
+    const float x = (key_to_float(key) - lo) * scale;  // NaN (inf * 0) maps to bin 0
+    return (uint32_t)fminf(fmaxf(x, 0.f), (float)(kHistBins - 1));
+  }
+};
+
+// The 12-bit digits, from the top, of the composites of keys in [kmin, kmax]:
+// the key part counts from kmin, so the digits spread over the keys' own range.
+struct CompositeDigits {
+  uint32_t kmin;
+  int total_bits, levels;
+  __device__ __forceinline__ CompositeDigits(uint32_t lo, uint32_t hi)
+      : kmin(lo), total_bits(32 - __clz(hi - lo) + 18), levels((total_bits + 11) / 12) {}
+  __device__ __forceinline__ int bins(int level) const {
+    const int top = total_bits - 12 * level;
+    return 1 << (top - max(top - 12, 0));
+  }
+  __device__ __forceinline__ uint32_t of(uint32_t key, uint32_t pos, int level) const {
+    const int top = total_bits - 12 * level;
+    const int lo_b = max(top - 12, 0);
+    return (uint32_t)((rank_composite(key - kmin, pos) >> lo_b) & ((1ull << (top - lo_b)) - 1ull));
+  }
+};
+
+}  // namespace dsa

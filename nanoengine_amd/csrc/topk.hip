@@ -35,6 +35,7 @@
 
 #include "dsa_common.h"
 #include "indexer_page.h"
+#include "select.h"
 #include "../../include/dsa_amd.h"
 
 namespace dsa {
@@ -42,8 +43,6 @@ namespace dsa {
 constexpr int kTopkThreads = 512;
 constexpr int kTopkMaxLen = 1 << 18;            // positions per row
 constexpr int kBitmapWords = kTopkMaxLen / 32;  // 32 KB of LDS
-constexpr int kHistBins = 4096;
-constexpr uint32_t kIdxMax = (1u << 18) - 1;
 constexpr int kLevels = 5;
 
 // threshold / gather geometry
@@ -68,7 +67,6 @@ constexpr size_t kTopkSmemBytes = sizeof(TopkSmem);
 // LDS of the list select: the candidates of a level's threshold bin are kept
 // as 16-bit indices into the row's list (values re-read from global), so two
 // workgroups fit on a CU. A row the kernel repairs itself uses TopkSmem.
-constexpr int kRankCap = 384;  // threshold-bin candidates ranked by counting
 struct ListSmem {
   uint32_t hist[kHistBins];
   uint32_t bitmap[kBitmapWords];
@@ -105,36 +103,6 @@ __device__ __forceinline__ bool in_bucket(int level, uint32_t key, uint32_t pos,
     default:
       return key == ((thr[0] << 20) | (thr[1] << 10) | thr[2]) && (((kIdxMax - pos) >> 9) == thr[3]);
   }
-}
-
-// Inverse of order_key: the float whose key is k.
-__device__ __forceinline__ float key_to_float(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k);
-}
-
-// Exclusive block prefix sum of one value per thread; returns the prefix and
-// writes the block total to *total (all threads).
-template <int NT>
-__device__ uint32_t block_exclusive_scan(uint32_t* wave_sum, uint32_t x, uint32_t* total) {
-  constexpr int kWaves = NT / 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint32_t v = x;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    uint32_t n = __shfl_up(v, off, 64);
-    if (lane >= off) v += n;
-  }
-  __syncthreads();
-  if (lane == 63) wave_sum[wave] = v;
-  __syncthreads();
-  uint32_t before = 0, all = 0;
-  for (int w = 0; w < kWaves; ++w) {
-    uint32_t t = wave_sum[w];
-    if (w < wave) before += t;
-    all += t;
-  }
-  *total = all;
-  return before + v - x;
 }
 
 // Positions of the set bits of bitmap[0, nwords) in ascending order into
@@ -825,24 +793,6 @@ topk_onepass_kernel(const RowIn in, const int32_t* __restrict__ offsets, const i
 }
 
 // ---------------------------------------------------------------- list select
-// 4096 bins linear in the score between the scores of keys kmin and kmax. The
-// bin never decreases with the key (subtraction, multiplication by a positive
-// scale and truncation are each monotone, +-0 share a bin), so a candidate in
-// a higher bin ranks ahead. Scores that are not finite, or whose range is not,
-// fall into the end bins or all into one.
-struct ScoreBins {
-  float lo, scale;
-  __device__ __forceinline__ ScoreBins(uint32_t kmin, uint32_t kmax) {
-    lo = key_to_float(kmin);
-    const float range = key_to_float(kmax) - lo;
-    scale = range > 0.f && range < 3.0e38f ? (float)(kHistBins - 1) / range : 0.f;
-  }
-  __device__ __forceinline__ uint32_t of(uint32_t key) const {
-    const float x = (key_to_float(key) - lo) * scale;  // NaN (inf * 0) maps to bin 0
-    return (uint32_t)fminf(fmaxf(x, 0.f), (float)(kHistBins - 1));
-  }
-};
-
 // Exact top-k of a row's candidate list (fused indexer path), ranked by
 // (score, lower position). The first digit is the score's linear bin; the
 // threshold bin then holds a few candidates, whose rank each of them counts
@@ -936,7 +886,6 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
       if ((uint32_t)(u * NT) < cand && (uint32_t)(u * NT + tid) < cand) f((uint32_t)(u * NT + tid), ch[u], cl[u]);
     for (uint32_t e = kReg * NT + tid; e < cand; e += NT) f(e, w.key[e], w.pos[e]);
   };
-  auto composite = [&](uint32_t key, uint32_t pos) { return ((uint64_t)key << 18) | (kIdxMax - pos); };
   // The selected positions are marked in LDS: a byte each where the row fits
   // (plain stores), else a bit each. In a short row most positions are
   // selected and the lanes of a wave hold consecutive ones, so that atomics on
@@ -1013,7 +962,7 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
     } else if (!last && d == tb) {
       const uint32_t slot = atomicAdd(&s.list_count[0], 1u);
       s.list[0][slot] = (uint16_t)e;
-      if (slot < (uint32_t)kRankCap) s.rank[slot] = composite(key, pos);
+      if (slot < (uint32_t)kRankCap) s.rank[slot] = rank_composite(key, pos);
     }
   });
   __syncthreads();
@@ -1030,20 +979,11 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
 
   // a crowded threshold bin (many equal or nearly equal scores): radix levels
   // of 12 bits of [ key - kmin : nb ][ (2^18-1) - position : 18 ] over its list
-  const int total_bits = 32 - __clz(kmax - kmin) + 18;
-  const int nlev = (total_bits + 11) / 12;
-  // digit of level L: bits [total - 12(L+1), total - 12L) of the composite
-  auto digit = [&](uint64_t c, int L) {
-    const int top = total_bits - 12 * L;
-    const int lo_b = max(top - 12, 0);
-    return (uint32_t)((c >> lo_b) & ((1ull << (top - lo_b)) - 1ull));
-  };
+  const CompositeDigits digits(kmin, kmax);
   int cur = 0;
-  for (int L = 0; L < nlev && !last; ++L) {
+  for (int L = 0; L < digits.levels && !last; ++L) {
     const uint32_t n = s.list_count[cur];
-    const int top = total_bits - 12 * L;
-    const int lo_b = max(top - 12, 0);
-    const int nbins = 1 << (top - lo_b);
+    const int nbins = digits.bins(L);
     const int nxt = cur ^ 1;
     // list_count[cur] is read by every thread above; list_count[nxt] was last
     // read a level ago
@@ -1051,18 +991,18 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
     if (tid == 0) s.list_count[nxt] = 0u;
     __syncthreads();
     // the list's candidates, re-read from the row's list (L2)
-    auto cand_c = [&](uint32_t i) { return composite(w.key[s.list[cur][i]] - kmin, w.pos[s.list[cur][i]]); };
-    for (uint32_t e = tid; e < n; e += NT) atomicAdd(&s.hist[digit(cand_c(e), L)], 1u);
+    auto cand_key = [&](uint32_t i) { return w.key[s.list[cur][i]]; };
+    auto cand_pos = [&](uint32_t i) { return w.pos[s.list[cur][i]]; };
+    for (uint32_t e = tid; e < n; e += NT) atomicAdd(&s.hist[digits.of(cand_key(e), cand_pos(e), L)], 1u);
     __syncthreads();
     find_threshold<NT>(s.hist, s.wave_sum, nbins, remain, &s.tb, &s.above, &s.eq);
     const uint32_t tb = s.tb, above = s.above, eq = s.eq;
     remain -= above;
-    last = (eq == remain) || L == nlev - 1;
+    last = (eq == remain) || L == digits.levels - 1;
     for (uint32_t e = tid; e < n; e += NT) {
-      const uint64_t c = cand_c(e);
-      const uint32_t d = digit(c, L);
+      const uint32_t pos = cand_pos(e), d = digits.of(cand_key(e), pos, L);
       if (d > tb || (last && d == tb)) {
-        mark(kIdxMax - (uint32_t)(c & kIdxMax));
+        mark(pos);
       } else if (!last && d == tb) {
         const uint32_t slot = atomicAdd(&s.list_count[nxt], 1u);
         s.list[nxt][slot] = s.list[cur][e];
@@ -1122,6 +1062,147 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
                        const int32_t* __restrict__ offsets, int32_t* __restrict__ out, int top_k,
                        const RowRepair rp) {
   list_select_row<false, PrefillList>(seq_lens, max_len, ws, nullptr, 0, 1, 0u, offsets, out, nullptr, top_k, rp);
+}
+
+// ---------------------------------------------------------------- row select
+// Exact top-k of a short row's order keys by one workgroup: thread t holds the
+// positions [per t, per (t + 1)), per a multiple of 4 up to kRowPer, so the
+// selected ones come out in position order by one block scan of bit counts.
+// First digit: the score's linear bin; the threshold bin's few elements count
+// those ahead of them, or, where many scores tie, take radix levels.
+constexpr int kRowThreads = 1024;
+constexpr int kRowPer = kRowSelectLen / kRowThreads;  // 16
+static_assert(kRowPer % 4 == 0 && kRowPer <= 32, "a thread's positions are a 32-bit mask");
+struct RowSelectSmem {
+  uint32_t hist[kHistBins];  // then the selected positions
+  uint64_t rank[kRankCap];
+  uint32_t bits[kRowSelectLen / 32];
+  uint32_t wave_sum[2 * (kRowThreads / 64)];
+  uint32_t count, tb, above, eq;
+};
+
+__global__ void __launch_bounds__(kRowThreads)
+topk_row_kernel(const uint32_t* __restrict__ keys, int64_t key_stride, const int32_t* __restrict__ seq_lens,
+                int64_t max_len, const int32_t* __restrict__ page_table, int64_t pt_stride, int pt_div,
+                uint32_t page_bits, int32_t* __restrict__ out_page, int32_t* __restrict__ out_raw, int top_k) {
+  __shared__ __align__(16) RowSelectSmem s;
+  constexpr int NT = kRowThreads, NW = NT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x;
+  const int64_t l = seq_lens[b];
+  const int len = (int)(l < 0 ? 0 : (l > max_len ? max_len : l));
+  const RowOut out{out_page + (int64_t)b * top_k, out_raw ? out_raw + (int64_t)b * top_k : nullptr,
+                   page_table + (int64_t)(b / pt_div) * pt_stride, page_bits, 0};
+  if (len <= top_k) {
+    for (int i = tid; i < top_k; i += NT) out.emit(i, i < len ? i : -1);
+    return;
+  }
+  const int per = (len + 4 * NT - 1) / (4 * NT) * 4;
+  const int p0 = per * tid;
+  const uint32_t* row = keys + (int64_t)b * key_stride;
+  uint32_t key[kRowPer];  // 0: past the row, below every key
+#pragma unroll
+  for (int c = 0; c < kRowPer; c += 4) {
+    uint4 x = {0u, 0u, 0u, 0u};
+    if (c < per && p0 + c < len) x = *reinterpret_cast<const uint4*>(row + p0 + c);  // (rows are padded to 4 keys)
+    key[c] = x.x;
+    key[c + 1] = p0 + c + 1 < len ? x.y : 0u;
+    key[c + 2] = p0 + c + 2 < len ? x.z : 0u;
+    key[c + 3] = p0 + c + 3 < len ? x.w : 0u;
+  }
+  for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
+  if (tid < kRowSelectLen / 32) s.bits[tid] = 0u;
+  if (tid == 0) s.count = 0u;
+  uint32_t kmin = 0xffffffffu, kmax = 0u;
+#pragma unroll
+  for (int i = 0; i < kRowPer; ++i) {
+    kmin = min(kmin, key[i] ? key[i] : 0xffffffffu);
+    kmax = max(kmax, key[i]);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
+    kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
+  }
+  if (lane == 0) {
+    s.wave_sum[wave] = kmin;
+    s.wave_sum[NW + wave] = kmax;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    kmin = min(kmin, s.wave_sum[i]);
+    kmax = max(kmax, s.wave_sum[NW + i]);
+  }
+  const ScoreBins bins(kmin, kmax);
+#pragma unroll
+  for (int i = 0; i < kRowPer; ++i)
+    if (key[i]) atomicAdd(&s.hist[bins.of(key[i])], 1u);
+  __syncthreads();
+  uint32_t remain = (uint32_t)top_k;
+  find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
+  uint32_t tb = s.tb;
+  const uint32_t eq = s.eq;
+  remain -= s.above;
+  const bool whole_bin = eq == remain;
+  uint32_t mine = 0u, alive = 0u;  // selected, and undecided (in the threshold bin), of this thread's positions
+#pragma unroll
+  for (int i = 0; i < kRowPer; ++i) {
+    const uint32_t d = bins.of(key[i]);
+    if (key[i] && (d > tb || (whole_bin && d == tb))) mine |= 1u << i;
+    else if (key[i] && d == tb) alive |= 1u << i;
+  }
+  if (!whole_bin && eq <= (uint32_t)kRankCap) {
+#pragma unroll
+    for (int i = 0; i < kRowPer; ++i)
+      if ((alive >> i) & 1u) s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key[i], (uint32_t)(p0 + i));
+    __syncthreads();
+    if ((uint32_t)tid < eq) {
+      const uint64_t c = s.rank[tid];
+      uint32_t ahead = 0;
+      for (uint32_t e = 0; e < eq; ++e) ahead += s.rank[e] > c ? 1u : 0u;
+      const uint32_t pos = kIdxMax - (uint32_t)(c & kIdxMax);
+      if (ahead < remain) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kRowPer; i += 4)
+      if (i < per && ((alive >> i) & 0xfu)) mine |= (s.bits[(p0 + i) >> 5] >> ((p0 + i) & 31) & 0xfu) << i;
+  } else if (!whole_bin) {
+    const CompositeDigits digits(kmin, kmax);
+    for (int L = 0; L < digits.levels; ++L) {
+      __syncthreads();  // every thread has read the previous level's outcome
+      for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kRowPer; ++i)
+        if ((alive >> i) & 1u) atomicAdd(&s.hist[digits.of(key[i], (uint32_t)(p0 + i), L)], 1u);
+      __syncthreads();
+      find_threshold<NT>(s.hist, s.wave_sum, digits.bins(L), remain, &s.tb, &s.above, &s.eq);
+      tb = s.tb;
+      remain -= s.above;
+      const bool last = s.eq == remain || L == digits.levels - 1;
+#pragma unroll
+      for (int i = 0; i < kRowPer; ++i) {
+        if (!((alive >> i) & 1u)) continue;
+        const uint32_t d = digits.of(key[i], (uint32_t)(p0 + i), L);
+        if (d > tb || (last && d == tb)) mine |= 1u << i;
+        if (d != tb) alive &= ~(1u << i);
+      }
+      if (last) break;
+    }
+  }
+  // positions in ascending order, then the page translation
+  uint32_t total = 0;
+  uint32_t at = block_exclusive_scan<NT>(s.wave_sum, (uint32_t)__popc(mine), &total);
+  __syncthreads();  // the histogram becomes the list of selected positions
+  while (mine) {
+    const int i = __ffs(mine) - 1;
+    mine &= mine - 1;
+    s.hist[at++] = (uint32_t)(p0 + i);
+  }
+  __syncthreads();
+  for (int i = tid; i < top_k; i += NT) out.emit(i, (int32_t)s.hist[i]);
 }
 
 __global__ void topk_to_physical_kernel(const int32_t* __restrict__ topk, int64_t topk_stride,
@@ -1241,6 +1322,14 @@ int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max
   hipLaunchKernelGGL(topk_list_defer_kernel, dim3(rows), dim3(kTopkThreads), sizeof(ListSmem), stream, seq_lens,
                      max_len, ws, offsets, out, top_k, rp);
   return check_launch("dsa_mqa_topk(select)");
+}
+
+int launch_row_select(const uint32_t* keys, int64_t key_stride, const int32_t* seq_lens, int64_t max_len,
+                      const int32_t* page_table, int64_t pt_stride, int pt_div, uint32_t page_bits, int32_t* out_page,
+                      int32_t* out_raw, int top_k, int rows, hipStream_t stream) {
+  hipLaunchKernelGGL(topk_row_kernel, dim3(rows), dim3(kRowThreads), 0, stream, keys, key_stride, seq_lens, max_len,
+                     page_table, pt_stride, pt_div, page_bits, out_page, out_raw, top_k);
+  return check_launch("dsa_indexer_topk(row select)");
 }
 
 }  // namespace dsa

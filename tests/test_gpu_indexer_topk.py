@@ -168,3 +168,41 @@ def test_repeated_scores_select_the_lowest_positions(cuda, length, pages, one_sc
     g_phys, g_logi = _fused(inp, cl, max_ctx, 2048, 1)
     assert np.array_equal(g_logi, e_logi)
     assert np.array_equal(g_phys, e_phys)
+
+
+@pytest.mark.parametrize("lens,n,k", [
+    ([16384, 16383, 4097, 4096, 2049, 2048, 1], 1, 2048),   # the longest short row; 4 and 8 keys a thread; around top-k
+    ([16384, 2049, 2048, 2], 2, 2048),                      # MTP rows: one token of an entry at top-k, one above
+    ([513, 512, 511, 577, 64], 1, 512),
+    ([8193, 700, 513], 2, 512),
+    ([100, 7], 1, 2048),                                    # nothing to score
+])
+def test_short_contexts_select_whole_rows(cuda, lens, n, k):
+    print(f"short fused lens={lens} n={n} k={k}", flush=True)
+    inp, cl, max_ctx = _inputs(lens, n, seed=sum(lens) + n + k)
+    assert max_ctx <= 16384
+    e_phys, e_logi = _unfused(inp, cl, max_ctx, k, n)
+    g_phys, g_logi = _fused(inp, cl, max_ctx, k, n)
+    assert np.array_equal(g_logi, e_logi)
+    assert np.array_equal(g_phys, e_phys)
+
+
+@pytest.mark.parametrize("length,pages,one_score,max_ctx", [
+    (16384, 1, False, 16384),  # 256 copies of each score
+    (16000, 50, False, 16000), # about five copies: the threshold bin is ranked by counting
+    (16384, 1, True, 16384),   # one score: radix levels down to the position bits
+    (7000, 3, False, 3001),    # max_context_len below the row, not a page multiple
+])
+def test_short_contexts_with_repeated_scores(cuda, length, pages, one_score, max_ctx):
+    print(f"short repeated length={length} pages={pages}", flush=True)
+    inp, cl, _ = _inputs([length, 2500], 1, seed=length + pages)
+    width = inp.block_tables.shape[1]
+    inp.block_tables[0] = inp.block_tables[0, torch.arange(width, device="cuda") % pages]
+    if one_score:
+        page = inp.cache[int(inp.block_tables[0, 0])]
+        page[:64 * 128] = page[:128].repeat(64)
+        page[64 * 128:] = page[64 * 128:64 * 128 + 4].repeat(64)
+    e_phys, e_logi = _unfused(inp, cl, max_ctx, 2048, 1)
+    g_phys, g_logi = _fused(inp, cl, max_ctx, 2048, 1)
+    assert np.array_equal(g_logi, e_logi)
+    assert np.array_equal(g_phys, e_phys)

@@ -736,8 +736,11 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
   mark(0);
   // Short contexts: every score (as order keys, in the logits buffer), then a
   // select over whole rows. The sample pass and the list, which pay for
-  // themselves on long rows, are two thirds of the indexer's time on short ones.
-  if (max_context_len <= kRowSelectLen) {
+  // themselves on long rows, are two thirds of the indexer's time on short
+  // ones. Indexer us, lists against whole rows: 4 x 4K 24.5 / 15.3, 64 x 16K
+  // 50.4 / 42.6, 1024 x 8K 287 / 259; over 8K tokens the row select loses once
+  // its rows pass one round of the CUs (256 x 16K 119 / 121, 512 x 16K 237 / 249).
+  if (max_context_len <= kRowSelectLen / 2 || (max_context_len <= kRowSelectLen && rows <= 192)) {
     uint32_t* keys = reinterpret_cast<uint32_t*>(f.logits);
     if (launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
                                  next_n, max_context_len, top_k, nullptr, keys, f.logits_stride, st)) {

@@ -1066,13 +1066,13 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 
 // ---------------------------------------------------------------- row select
 // Exact top-k of a short row's order keys by one workgroup: thread t holds the
-// positions [per t, per (t + 1)), per a multiple of 4 up to kRowPer, so the
+// positions [per t, per (t + 1)), per a multiple of 4 up to kPer, so the
 // selected ones come out in position order by one block scan of bit counts.
+// Instantiated for 4K, 8K and 16K positions: the 16K kernel takes 3 us longer
+// over 64 rows of 4K than the 4K one.
 // First digit: the score's linear bin; the threshold bin's few elements count
 // those ahead of them, or, where many scores tie, take radix levels.
 constexpr int kRowThreads = 1024;
-constexpr int kRowPer = kRowSelectLen / kRowThreads;  // 16
-static_assert(kRowPer % 4 == 0 && kRowPer <= 32, "a thread's positions are a 32-bit mask");
 struct RowSelectSmem {
   uint32_t hist[kHistBins];  // then the selected positions
   uint64_t rank[kRankCap];
@@ -1081,12 +1081,14 @@ struct RowSelectSmem {
   uint32_t count, tb, above, eq;
 };
 
+template <int kRowPer>
 __global__ void __launch_bounds__(kRowThreads)
 topk_row_kernel(const uint32_t* __restrict__ keys, int64_t key_stride, const int32_t* __restrict__ seq_lens,
                 int64_t max_len, const int32_t* __restrict__ page_table, int64_t pt_stride, int pt_div,
                 uint32_t page_bits, int32_t* __restrict__ out_page, int32_t* __restrict__ out_raw, int top_k) {
   __shared__ __align__(16) RowSelectSmem s;
   constexpr int NT = kRowThreads, NW = NT / 64;
+  static_assert(kRowPer % 4 == 0 && kRowPer <= 32, "a thread's positions are a 32-bit mask");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int b = blockIdx.x;
   const int64_t l = seq_lens[b];
@@ -1327,7 +1329,10 @@ int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max
 int launch_row_select(const uint32_t* keys, int64_t key_stride, const int32_t* seq_lens, int64_t max_len,
                       const int32_t* page_table, int64_t pt_stride, int pt_div, uint32_t page_bits, int32_t* out_page,
                       int32_t* out_raw, int top_k, int rows, hipStream_t stream) {
-  hipLaunchKernelGGL(topk_row_kernel, dim3(rows), dim3(kRowThreads), 0, stream, keys, key_stride, seq_lens, max_len,
+  auto* kernel = max_len <= 4 * kRowThreads   ? topk_row_kernel<4>
+                 : max_len <= 8 * kRowThreads ? topk_row_kernel<8>
+                                              : topk_row_kernel<kRowSelectLen / kRowThreads>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(kRowThreads), 0, stream, keys, key_stride, seq_lens, max_len,
                      page_table, pt_stride, pt_div, page_bits, out_page, out_raw, top_k);
   return check_launch("dsa_indexer_topk(row select)");
 }

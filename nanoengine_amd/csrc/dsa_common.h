@@ -157,6 +157,14 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
                            float sm_scale, void* out, float* lse, int num_splits, void* workspace,
                            size_t workspace_bytes, void* stream, float* max_out, const MlaFresh* fresh);
 
+// The same kernel over bf16 rows only: token t attends over rows[indices[t][i]]
+// (row stride in elements), i < topk, a multiple of 32; an index outside
+// [0, num_rows) is skipped (the body of dsa_sparse_mla_prefill).
+int sparse_mla_rows_impl(const void* q, int64_t q_token_stride, int64_t q_head_stride, const void* rows,
+                         int64_t row_stride, int64_t num_rows, const int32_t* indices, int64_t idx_stride,
+                         int num_tokens, int num_heads, int topk, float sm_scale, void* out, float* max_out, float* lse,
+                         void* stream);
+
 template <typename T>
 __device__ __forceinline__ T shfl_xor(T v, int mask) {
   return __shfl_xor(v, mask, 64);

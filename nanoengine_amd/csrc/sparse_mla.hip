@@ -100,6 +100,9 @@ constexpr float kRescaleThreshold = 8.0f;  // log2 units
 // above 2^-126.
 constexpr float kMinLogP = -30.0f;
 constexpr int kDropExp = -30;
+// The keys of an instantiation: cache slots (decode), cache slots then bf16
+// rows (paged prefill), bf16 rows only (prefill over assembled keys).
+enum KeyKind : int { kSlots = 0, kSlotsThenRows = 1, kRows = 2 };
 constexpr int kIdxWave = 3;                // the wave that fetches the row indices (a QK wave)
 
 // Output staging of a PV wave: 32 heads x 128 dims, rows 16 bytes apart from a
@@ -232,6 +235,12 @@ struct MlaCtx {
   bool head_ok;
 };
 
+// Is block j one of bf16 rows?
+template <int kKeys>
+__device__ __forceinline__ bool rows_block(const MlaCtx& c, int j) {
+  return kKeys == kRows || (kKeys == kSlotsThenRows && j >= c.ncached);
+}
+
 // Cache block of a physical slot.
 __device__ __forceinline__ int64_t slot_block(const MlaParams& P, int32_t slot) {
   return P.kv_block_shift >= 0 ? (int64_t)(slot >> P.kv_block_shift) : (int64_t)(slot / P.kv_block_size);
@@ -263,12 +272,12 @@ __device__ __forceinline__ bool fresh_valid(const MlaParams& P, int32_t r, int l
 }
 
 // Table of block j's row addresses from ring slot j % 5 (lane = row), in table j % 2.
-template <bool kFresh>
+template <int kKeys>
 __device__ __forceinline__ void build_addr_table(const MlaParams& P, uint8_t* smem, const MlaCtx& c, int j) {
   const int lane = c.lane;
   const int32_t slot = reinterpret_cast<const int32_t*>(smem + kRingOff + (j % kRingSlots) * 256)[lane];
   uint64_t a;
-  if (!kFresh || j < c.ncached)
+  if (!rows_block<kKeys>(c, j))
     a = row_address(P, slot);
   else
     a = fresh_valid(P, slot, lane) ? reinterpret_cast<uint64_t>(P.fresh + (int64_t)slot * P.fresh_row_stride)
@@ -333,7 +342,9 @@ __device__ __forceinline__ void issue_block(const uint8_t* smem, int j, const Dm
   }
 }
 
-// A fresh block's 36 loads: five each for waves 0-3, four for waves 4-7; lane l
+// Row r's 16-byte piece c lies in slot c ^ (r % 8) of its 72 (1152 B is a
+// multiple of the banks' span: unswizzled, the 32 rows of an operand read
+// would fall on the same banks). The block's 36 loads: five each for waves 0-3, four for waves 4-7; lane l
 // of load i takes piece c = 64(first + i) + l of the packed 32 rows.
 __device__ __forceinline__ void issue_fresh_block(const uint8_t* smem, int j, const uint8_t* buf, int wave,
                                                   int lane) {
@@ -343,7 +354,7 @@ __device__ __forceinline__ void issue_fresh_block(const uint8_t* smem, int j, co
   for (int i = 0; i < cnt; ++i) {
     const int pc = 64 * (first + i) + lane;
     const int r = pc / kFreshRowPieces;
-    const uint64_t g = *reinterpret_cast<const uint64_t*>(tab + 8 * r) + 16 * (pc - r * kFreshRowPieces);
+    const uint64_t g = *reinterpret_cast<const uint64_t*>(tab + 8 * r) + 16 * ((pc - r * kFreshRowPieces) ^ (r & 7));
     dma16(reinterpret_cast<const void*>(g), lds_addr(buf + 1024 * (first + i)));
   }
 }
@@ -351,10 +362,10 @@ static_assert(4 * 5 + 4 * 4 == kFreshDma, "fresh block loads per wave");
 
 // The row indices of block j into ring slot j % 5: 64 cache slots, or 32 fresh
 // row indices (lanes 32-63 repeat lanes 0-31).
-template <bool kFresh>
+template <int kKeys>
 __device__ __forceinline__ void issue_index(const MlaParams& P, uint8_t* smem, const MlaCtx& c, int j) {
   const int32_t* src =
-      !kFresh || j < c.ncached ? P.idx + (int64_t)c.t_tok * P.idx_stride + c.key_begin + j * kMlaKeys + c.lane
+      !rows_block<kKeys>(c, j) ? P.idx + (int64_t)c.t_tok * P.idx_stride + c.key_begin + j * kMlaKeys + c.lane
                     : P.fresh_idx + (int64_t)c.t_tok * P.fresh_idx_stride + (j - c.ncached) * kFreshKeys +
                           (c.lane & (kFreshKeys - 1));
   dma4(src, __builtin_amdgcn_readfirstlane(lds_addr(smem + kRingOff + (j % kRingSlots) * 256)));
@@ -363,13 +374,13 @@ __device__ __forceinline__ void issue_index(const MlaParams& P, uint8_t* smem, c
 
 // Start of iteration t (both roles, every wave): the index load of block t+4;
 // this wave's share of block t+1's rows.
-template <bool kFresh>
+template <int kKeys>
 __device__ __forceinline__ void iteration_start(const MlaParams& P, uint8_t* smem, const MlaCtx& c,
                                                 const DmaLanes& dl, int t) {
-  if (c.wave == kIdxWave && t + 4 < c.nblk) issue_index<kFresh>(P, smem, c, t + 4);
+  if (c.wave == kIdxWave && t + 4 < c.nblk) issue_index<kKeys>(P, smem, c, t + 4);
   if (t + 1 < c.nblk) {
     uint8_t* buf = smem + ((t + 1) % kNumBufs) * kBufBytes;
-    if (!kFresh || t + 1 < c.ncached) issue_block(smem, t + 1, dl, buf, c.wave);
+    if (!rows_block<kKeys>(c, t + 1)) issue_block(smem, t + 1, dl, buf, c.wave);
     else issue_fresh_block(smem, t + 1, buf, c.wave, c.lane);
   }
 }
@@ -403,7 +414,7 @@ __device__ __forceinline__ void issue_query(const MlaParams& P, uint8_t* smem, c
 }
 
 // QK waves: S of block t over this wave's 32 keys, its lazy reference, P(t).
-template <bool kFresh, int kTiles>
+template <int kKeys, int kTiles>
 __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl) {
   const int lane = c.lane, h = c.h, c32 = c.c32, hp = c.hp, kh = c.kh;
   // the query as the B operand over all dims: nope chunk k (64 dims), k-step j =
@@ -430,12 +441,12 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
   float l_run = 0.f;                // sum of P against m_run, this lane's keys only
 
   for (int t = 0; t <= c.nblk; ++t) {
-    iteration_start<kFresh>(P, smem, c, dl, t);
+    iteration_start<kKeys>(P, smem, c, dl, t);
     // row addresses of block t+2 (its indices landed two iterations ago); the
     // table slot was last read when block t was issued, before this iteration
-    if (c.wave == kTabWave && t + 2 < c.nblk) build_addr_table<kFresh>(P, smem, c, t + 2);
+    if (c.wave == kTabWave && t + 2 < c.nblk) build_addr_table<kKeys>(P, smem, c, t + 2);
     // a fresh block has 32 keys, all in key half 0
-    const bool fresh = kFresh && t >= c.ncached;
+    const bool fresh = rows_block<kKeys>(c, t);
     if (t < c.nblk && !(fresh && kh == 1) && hp < kTiles) {
       const uint8_t* buf = smem + (t % kNumBufs) * kBufBytes;
       const int32_t slot_t = reinterpret_cast<const int32_t*>(smem + kRingOff + (t % kRingSlots) * 256)[lane];
@@ -445,19 +456,34 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = 0.f;
       if (fresh) {
-        // bf16 rows: the key operand is read as is
-        const uint8_t* frow = buf + c32 * kFreshRowBytes;
+        // bf16 rows: the key operand is read as is, one chunk of 64 dims ahead
+        // (the swizzle changes only the piece's low three bits, so a chunk's
+        // four addresses serve every chunk; formed from an opaque lane id, so
+        // that they hold no registers across the loop)
+        int r_o = c32;
+        asm volatile("" : "+v"(r_o));
+        const uint8_t* frow = buf + r_o * kFreshRowBytes;
+        const uint8_t *fn[4], *fr[4];
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
+        for (int j = 0; j < 4; ++j) {
+          fn[j] = frow + 16 * ((4 * h + j) ^ (r_o & 7));
+          fr[j] = frow + 1024 + 16 * ((2 * j + h) ^ (r_o & 7));
+        }
+        v4i kb[2][4];
+        auto read_chunk = [&](int k, v4i* dst) {  // chunk 8: the rope dims
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const v4i kb = *reinterpret_cast<const v4i*>(frow + 2 * (64 * k + 32 * h + 8 * j));
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kb), as_v8bf(qn[k][j]), s, 0, 0, 0);
-          }
+          for (int j = 0; j < 4; ++j) dst[j] = *reinterpret_cast<const v4i*>(k < 8 ? fn[j] + 128 * k : fr[j]);
+        };
+        read_chunk(0, kb[0]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const v4i rope = *reinterpret_cast<const v4i*>(frow + 2 * (512 + 16 * r + 8 * h));
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(rope), as_v8bf(qr[r]), s, 0, 0, 0);
+        for (int k = 0; k < 9; ++k) {
+          if (k + 1 < 9) read_chunk(k + 1, kb[(k + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kb[k & 1][j]), as_v8bf(k < 8 ? qn[k < 8 ? k : 0][j] : qr[j]), s,
+                                                        0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
         }
       } else {
       const uint8_t* row = buf + (32 * kh + c32) * kMlaRowBytes;
@@ -540,7 +566,7 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
 #pragma unroll
       for (int r = 0; r < 4; ++r) ls4[r] = (pv[r] + pv[4 + r]) + (pv[8 + r] + pv[12 + r]);
       l_run += (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
-      if (fresh && !all_valid) {
+      if (kKeys == kSlotsThenRows && fresh && !all_valid) {
         // An invalid key's V is the zero row, so any finite P' leaves O alone.
         // The PV waves scale a fresh block's P by adding f in [-30, 0] to the
         // bf16 exponent field with no tile-scale term, which takes a P of 0 to
@@ -578,7 +604,7 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
 // Wave dq = w - 4 owns O[64 heads x dims 128dq .. 128dq+127], exactly V tile
 // dq, as two head tiles (the head halves): each V byte is converted once per
 // workgroup, and one exponent per key scales both tiles' P.
-template <bool kFresh, int kTiles>
+template <int kKeys, int kTiles>
 __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl,
                                          int split) {
   const int lane = c.lane, h = c.h, c32 = c.c32, dq = c.wave - 4;
@@ -607,16 +633,17 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
   // transposing bf16 reads of a fresh block: lane (G = lane/16, m = lane%16)
   // addresses key row 4h + m/4 (+8) and dims 16(G%2) + 4(m%4) .. +3 of each
   // 32-dim tile, and receives dim 16(G%2) + m of four consecutive keys
-  const uint32_t flane = (uint32_t)((4 * h + (m16 >> 2)) * kFreshRowBytes +
-                                    2 * (128 * dq + 16 * (G & 1) + 4 * (m16 & 3)));
+  // (rows 4h + m/4 apart by 8 and 16 share a swizzle; 32 dims further is 64 bytes, below the row's 256-byte tile)
+  const uint32_t frow0 = (uint32_t)((4 * h + (m16 >> 2)) * kFreshRowBytes + 256 * dq);
+  const uint32_t fcol0 = (uint32_t)((32 * (G & 1) + 8 * (m16 & 3)) ^ (16 * ((4 * h + (m16 >> 2)) & 7)));
 
   prologue_end();
   for (int t = 0; t <= c.nblk; ++t) {
-    iteration_start<kFresh>(P, smem, c, dl, t);
+    iteration_start<kKeys>(P, smem, c, dl, t);
     if (t >= 1) {
       const int par = (t - 1) & 1;
       const uint8_t* bufp = smem + ((t - 1) % kNumBufs) * kBufBytes;
-      const bool fresh = kFresh && t - 1 >= c.ncached;
+      const bool fresh = rows_block<kKeys>(c, t - 1);
       if (!fresh) {
         // exponent table of block t-1, tile dq (lane = key): the tile scale's
         // exponent in the bf16 exponent field, at the PV A operand position of
@@ -670,6 +697,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
         asm volatile("" : "+v"(a));
         return a;
       };
+      constexpr int kSteps = kKeys == kRows ? kFreshKeys / 16 : kMlaKeys / 16;
       // k-step ks: its P (both head tiles), exponent and V reads issued one
       // k-step ahead
       v2i vq[2][4];
@@ -677,22 +705,24 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
       {
         const uint32_t a0 = vaddr(0);
 #pragma unroll
-        for (int nn = 0; nn < 4; ++nn) vq[0][nn] = lds_read_tr8_at(a0 + 32 * nn);
+        for (int nn = 0; nn < 4; ++nn)
+          if (kKeys != kRows) vq[0][nn] = lds_read_tr8_at(a0 + 32 * nn);
 #pragma unroll
         for (int mt = 0; mt < kTiles; ++mt) pq[0][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + lane * 16);
-        eq[0] = *reinterpret_cast<const v4i_alias*>(et + h * 8);
+        if (kKeys != kRows) eq[0] = *reinterpret_cast<const v4i_alias*>(et + h * 8);
       }
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+      for (int ks = 0; ks < kSteps; ++ks) {
         const int cur = ks & 1, nxt = cur ^ 1;
-        if (ks + 1 < 4) {
+        if (ks + 1 < kSteps) {
           const uint32_t a1 = vaddr(ks + 1);
 #pragma unroll
-          for (int nn = 0; nn < 4; ++nn) vq[nxt][nn] = lds_read_tr8_at(a1 + 32 * nn);
+          for (int nn = 0; nn < 4; ++nn)
+            if (kKeys != kRows) vq[nxt][nn] = lds_read_tr8_at(a1 + 32 * nn);
 #pragma unroll
           for (int mt = 0; mt < kTiles; ++mt)
             pq[nxt][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + ((ks + 1) * 64 + lane) * 16);
-          eq[nxt] = *reinterpret_cast<const v4i_alias*>(et + ((ks + 1) * 2 + h) * 8);
+          if (kKeys != kRows) eq[nxt] = *reinterpret_cast<const v4i_alias*>(et + ((ks + 1) * 2 + h) * 8);
         }
         __builtin_amdgcn_sched_barrier(0);
         const int k2 = ks >> 1;  // k-steps 0, 1: key half 0; 2, 3: key half 1
@@ -702,6 +732,10 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
         for (int mt = 0; mt < kTiles; ++mt)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
+            if (kKeys == kRows) {  // one key half: its reference is R, and there are no tile scales
+              pa[mt][e] = pq[cur][mt][e];
+              continue;
+            }
             // (bit_cast of a vector element reads element 0; copy to scalars first)
             const int pe = pq[cur][mt][e], ee = fresh ? 0 : eq[cur][e];
             const v2u16 sum = __builtin_bit_cast(v2u16, pe) + __builtin_bit_cast(v2u16, ee) +
@@ -713,7 +747,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
           v8bf vop;
           if (fresh) {
             // bf16 V, no tile scale: two transposing reads give keys 4h + 0..3 and 8 + 4h + 0..3
-            uint32_t a = lds_addr(bufp) + flane + 16 * ks * kFreshRowBytes + 2 * (32 * nn);
+            uint32_t a = lds_addr(bufp) + frow0 + 16 * ks * kFreshRowBytes + (fcol0 ^ (64 * nn));
             asm volatile("" : "+v"(a));
             const v4s lo = lds_read_tr16_at(a);
             const v4s hi = lds_read_tr16_at(a + 8 * kFreshRowBytes);
@@ -799,13 +833,12 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
   }
 }
 
-// kFresh: a chunked prefill's token lists (cache slots, then fresh bf16 rows);
-// decode instantiates the kernel without that path.
+// kKeys: what the keys are (KeyKind); each instantiation has only its own paths.
 // kTiles: the workgroup's head tiles of 32. With at most 32 heads in all (a
 // tensor-parallel rank's 16) the second tile would be padding: its score waves
 // idle and its P.V products are left out. (As a run-time condition this cost
 // the 64-head kernel 5%: the branches stop the P.V loop's read-ahead.)
-template <bool kFresh, int kTiles>
+template <int kKeys, int kTiles>
 __global__ void __launch_bounds__(kMlaThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 sparse_mla_kernel(const MlaParams P) {
   extern __shared__ __align__(16) uint8_t smem[];
@@ -837,11 +870,15 @@ sparse_mla_kernel(const MlaParams P) {
   c.key_begin = first * kMlaKeys;
   c.nblk = (split < 0 ? blocks : blocks * (split + 1) / P.splits) - first;
   c.ncached = c.nblk;
-  if (kFresh) {
+  if (kKeys == kSlotsThenRows) {
     const int nc = __builtin_amdgcn_readfirstlane(P.counts[2 * c.t_tok]);
     const int nf = __builtin_amdgcn_readfirstlane(P.counts[2 * c.t_tok + 1]);
     c.ncached = (nc + kMlaKeys - 1) / kMlaKeys;
     c.nblk = c.ncached + (nf + kFreshKeys - 1) / kFreshKeys;
+  }
+  if (kKeys == kRows) {
+    c.ncached = 0;
+    c.nblk = P.topk / kFreshKeys;
   }
   c.h_half = hg * kMlaHeadsPerWG + c.hp * 32;
   c.head = c.h_half + c.c32;
@@ -850,25 +887,25 @@ sparse_mla_kernel(const MlaParams P) {
   // prologue: the indices of blocks 0-3 and the query go out together, then
   // the address tables of blocks 0 and 1, then block 0's rows
   if (c.wave == kIdxWave)
-    for (int j = 0; j < 4 && j < c.nblk; ++j) issue_index<kFresh>(P, smem, c, j);
+    for (int j = 0; j < 4 && j < c.nblk; ++j) issue_index<kKeys>(P, smem, c, j);
   issue_query(P, smem, c, hg * kMlaHeadsPerWG);
   const DmaLanes dl = dma_lanes(c.wave, c.lane);
   if (c.wave == kIdxWave)  // its index copies landed (the query's may still be on their way)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kQDma / kMlaWaves) : "memory");
   barrier();
   if (c.wave == kTabWave) {
-    if (c.nblk > 0) build_addr_table<kFresh>(P, smem, c, 0);
-    if (c.nblk > 1) build_addr_table<kFresh>(P, smem, c, 1);
+    if (c.nblk > 0) build_addr_table<kKeys>(P, smem, c, 0);
+    if (c.nblk > 1) build_addr_table<kKeys>(P, smem, c, 1);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's query copies
   barrier();
   if (c.nblk > 0) {
-    if (!kFresh || c.ncached > 0) issue_block(smem, 0, dl, smem, c.wave);
+    if (!rows_block<kKeys>(c, 0)) issue_block(smem, 0, dl, smem, c.wave);
     else issue_fresh_block(smem, 0, smem, c.wave, c.lane);
   }
   // both roles run the same number of iterations and barriers
-  if (c.wave < 4) qk_waves<kFresh, kTiles>(P, smem, c, dl);
-  else pv_waves<kFresh, kTiles>(P, smem, c, dl, split);
+  if (c.wave < 4) qk_waves<kKeys, kTiles>(P, smem, c, dl);
+  else pv_waves<kKeys, kTiles>(P, smem, c, dl, split);
 }
 
 // One 64-thread workgroup per (split item, head): merge the split partials.
@@ -947,6 +984,53 @@ int dsa_sparse_mla_decode(const void* q, int64_t q_token_stride, int64_t q_head_
 
 namespace dsa {
 
+static int launch_mla(const MlaParams& P, KeyKind keys, int64_t nwg, hipStream_t stream, const char* what) {
+  static int smem_status = -1;
+  if (smem_status < 0) {
+    smem_status = 0;
+    for (const void* k : {(const void*)sparse_mla_kernel<kSlots, 1>, (const void*)sparse_mla_kernel<kSlots, 2>,
+                          (const void*)sparse_mla_kernel<kSlotsThenRows, 1>,
+                          (const void*)sparse_mla_kernel<kSlotsThenRows, 2>, (const void*)sparse_mla_kernel<kRows, 1>,
+                          (const void*)sparse_mla_kernel<kRows, 2>})
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMlaSmemBytes) != hipSuccess)
+        smem_status = 1;
+  }
+  if (smem_status) return set_error(kLaunchFailed, "sparse_mla: cannot reserve %zu B of LDS", kMlaSmemBytes);
+  if (nwg > INT32_MAX) return set_error(kInvalidArgument, "%s: grid too large", what);
+  void (*const kernels[3][2])(MlaParams) = {
+      {sparse_mla_kernel<kSlots, 1>, sparse_mla_kernel<kSlots, 2>},
+      {sparse_mla_kernel<kSlotsThenRows, 1>, sparse_mla_kernel<kSlotsThenRows, 2>},
+      {sparse_mla_kernel<kRows, 1>, sparse_mla_kernel<kRows, 2>}};
+  hipLaunchKernelGGL(kernels[keys][P.H <= 32 ? 0 : 1], dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes, stream,
+                     P);
+  return check_launch(what);
+}
+
+int sparse_mla_rows_impl(const void* q, int64_t q_token_stride, int64_t q_head_stride, const void* rows,
+                         int64_t row_stride, int64_t num_rows, const int32_t* indices, int64_t idx_stride,
+                         int num_tokens, int num_heads, int topk, float sm_scale, void* out, float* max_out, float* lse,
+                         void* stream) {
+  MlaParams P{};
+  P.q = static_cast<const uint16_t*>(q);
+  P.q_tok_stride = q_token_stride;
+  P.q_head_stride = q_head_stride;
+  P.T = num_tokens;
+  P.H = num_heads;
+  P.topk = topk;
+  P.splits = 1;
+  P.head_groups = (num_heads + kMlaHeadsPerWG - 1) / kMlaHeadsPerWG;
+  P.scale_log2 = sm_scale * kLog2e;
+  P.out = static_cast<uint16_t*>(out);
+  P.lse = lse;
+  P.max_out = max_out;
+  P.fresh = static_cast<const uint16_t*>(rows);
+  P.fresh_row_stride = row_stride;
+  P.fresh_rows = num_rows;
+  P.fresh_idx = indices;
+  P.fresh_idx_stride = idx_stride;
+  return launch_mla(P, kRows, (int64_t)num_tokens * P.head_groups, (hipStream_t)stream, "dsa_sparse_mla_prefill");
+}
+
 int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head_stride, const uint8_t* kv_cache,
                            int64_t kv_block_stride_bytes, int kv_block_size, int64_t kv_num_blocks,
                            const int32_t* indices, int64_t idx_stride, int num_tokens, int num_heads, int topk,
@@ -989,16 +1073,6 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
   const size_t need = dsa_sparse_mla_workspace_bytes(num_tokens, num_heads, num_splits);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(kWorkspaceTooSmall, "sparse_mla: workspace %zu B < %zu B", workspace_bytes, need);
-
-  static int smem_status = -1;
-  if (smem_status < 0) {
-    smem_status = 0;
-    for (const void* k : {(const void*)sparse_mla_kernel<false, 1>, (const void*)sparse_mla_kernel<false, 2>,
-                          (const void*)sparse_mla_kernel<true, 1>, (const void*)sparse_mla_kernel<true, 2>})
-      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMlaSmemBytes) != hipSuccess)
-        smem_status = 1;
-  }
-  if (smem_status) return set_error(kLaunchFailed, "sparse_mla: cannot reserve %zu B of LDS", kMlaSmemBytes);
 
   MlaParams P;
   P.kv_block_shift = (kv_block_size & (kv_block_size - 1)) == 0 ? __builtin_ctz((unsigned)kv_block_size) : -1;
@@ -1049,11 +1123,8 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
     P.ws_lse = P.ws_o + rows * kMlaDv;
   }
   const int64_t nwg = whole + (items - whole) * num_splits;
-  void (*const kernel)(MlaParams) = num_heads <= 32
-                                        ? (fresh ? sparse_mla_kernel<true, 1> : sparse_mla_kernel<false, 1>)
-                                        : (fresh ? sparse_mla_kernel<true, 2> : sparse_mla_kernel<false, 2>);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes, (hipStream_t)stream, P);
-  if (int rc = check_launch("dsa_sparse_mla_decode")) return rc;
+  if (int rc = launch_mla(P, fresh ? kSlotsThenRows : kSlots, nwg, (hipStream_t)stream, "dsa_sparse_mla_decode"))
+    return rc;
   if (num_splits > 1) {
     hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)((items - whole) * kMlaHeadsPerWG)), dim3(64), 0,
                        (hipStream_t)stream, P.ws_o, P.ws_lse, num_tokens, num_heads, P.whole, P.head_groups,

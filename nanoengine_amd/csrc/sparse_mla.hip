@@ -600,6 +600,152 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
   barrier();
 }
 
+// QK waves over bf16 rows only (kRows): a block has 32 keys, so the four waves
+// split the dims instead of the keys. Wave (hp, dh = c.kh) forms the partial
+// S^T[32 keys x 32 heads] over its half of the dims (18 MFMAs), sends the
+// partner the partial sums of the partner's 16 keys through the P slots of
+// k-steps 2 and 3 (unused here), and after a barrier finishes the scores and P
+// of its own, k-step dh. (With the keys split as for cache slots, two of the
+// four waves idled and the other two set the block time: 607 -> 484 us; the
+// dims split: 484 -> 395 us, 512 tokens.)
+template <int kTiles>
+__device__ __forceinline__ void qk_waves_rows(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl) {
+  const int lane = c.lane, h = c.h, c32 = c.c32, hp = c.hp, dh = c.kh;
+  // the query over this wave's dims: nope chunks 4dh + k, rope k-steps 2dh + i
+  v4i qn[4][4];
+  v4i qr[2];
+  {
+    const int r = 32 * hp + c32;
+    const uint8_t* qrow = smem + kBufBytes + r * kQRowBytes;
+    const int sw = 16 * (r & 7);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        qn[k][j] = *reinterpret_cast<const v4i*>(qrow + ((16 * (8 * (4 * dh + k) + 4 * h + j)) ^ sw));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) qr[i] = *reinterpret_cast<const v4i*>(qrow + ((16 * (64 + 2 * (2 * dh + i) + h)) ^ sw));
+  }
+  prologue_end();
+  float* ref = reinterpret_cast<float*>(smem + kRefOff);
+  float m_run = -__builtin_inff();  // reference of k-step dh per head c32 (an integer, log2 units)
+  float m_max = -__builtin_inff();  // exact running maximum (log2 units), for max_out
+  float l_run = 0.f;                // sum of P against m_run, this lane's keys only
+  // A operand row m is key m ^ 16dh: the kept keys (k-step dh) are result rows
+  // 0-15 (registers 0-7), the partner's rows 16-31
+  const int krow = c32 ^ (16 * dh);
+  const uint8_t *fn[4], *fr[2];  // piece addresses in buffer 0
+#pragma unroll
+  for (int j = 0; j < 4; ++j) fn[j] = smem + krow * kFreshRowBytes + 512 * dh + 16 * ((4 * h + j) ^ (krow & 7));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) fr[i] = smem + krow * kFreshRowBytes + 1024 + 16 * ((2 * (2 * dh + i) + h) ^ (krow & 7));
+  uint8_t* const x_out = smem + kPOff + (dh ^ 1) * 8192 + hp * 4096 + 2048 + lane * 16;  // the partner's slots
+  const uint8_t* const x_in = smem + kPOff + dh * 8192 + hp * 4096 + 2048 + lane * 16;
+
+  for (int t = 0; t <= c.nblk; ++t) {
+    iteration_start<kRows>(P, smem, c, dl, t);
+    if (c.wave == kTabWave && t + 2 < c.nblk) build_addr_table<kRows>(P, smem, c, t + 2);
+    const bool work = t < c.nblk && hp < kTiles;
+    float sv[8];
+    if (work) {
+      const int boff = (t % kNumBufs) * kBufBytes;
+      v16f s;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
+      v4i kb[2][4], kr[2];
+      auto read_chunk = [&](int k, v4i* dst) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dst[j] = *reinterpret_cast<const v4i*>(fn[j] + boff + 128 * k);
+      };
+      read_chunk(0, kb[0]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k + 1 < 4) read_chunk(k + 1, kb[(k + 1) & 1]);
+        else
+#pragma unroll
+          for (int i = 0; i < 2; ++i) kr[i] = *reinterpret_cast<const v4i*>(fr[i] + boff);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kb[k & 1][j]), as_v8bf(qn[k][j]), s, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kr[i]), as_v8bf(qr[i]), s, 0, 0, 0);
+      *reinterpret_cast<v4f*>(x_out) = v4f{s[8], s[9], s[10], s[11]};
+      *reinterpret_cast<v4f*>(x_out + 1024) = v4f{s[12], s[13], s[14], s[15]};
+#pragma unroll
+      for (int r = 0; r < 8; ++r) sv[r] = s[r];
+    }
+    barrier();
+    if (work) {
+      const v4f xa = *reinterpret_cast<const v4f*>(x_in);
+      const v4f xb = *reinterpret_cast<const v4f*>(x_in + 1024);
+      const int32_t row_t = reinterpret_cast<const int32_t*>(smem + kRingOff + (t % kRingSlots) * 256)[lane];
+      const uint32_t vmask = (uint32_t)__ballot(fresh_valid(P, row_t, lane));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sv[r] += xa[r];
+        sv[4 + r] += xb[r];
+      }
+      const bool all_valid = vmask == 0xffffffffu;
+      uint32_t vb8 = 0xffu;  // bit r: key 16dh + 8(r/4) + 4h + r%4 valid
+      if (!all_valid) {
+        const uint32_t vm = vmask >> (16 * dh + 4 * h);
+        vb8 = (vm & 0xfu) | ((vm >> 4) & 0xf0u);
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+          if (!((vb8 >> r) & 1u)) sv[r] = -__builtin_inff();
+      }
+      float mloc = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
+      {
+        // the other lane half's maximum (the swap pairs the two halves)
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+        mloc = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      }
+      const float mblk = mloc * P.scale_log2;
+      m_max = fmaxf(m_max, mblk);
+      const bool need = mblk > m_run + kRescaleThreshold;
+      if (__ballot(need)) {
+        const float m_new = need ? ceilf(mblk) : m_run;
+        l_run *= __builtin_amdgcn_exp2f(m_run - m_new);  // a power of two (0 from -inf)
+        m_run = m_new;
+      }
+      const float m_use = m_run == -__builtin_inff() ? 0.f : m_run;
+      float pv[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        pv[r] = __builtin_amdgcn_exp2f(fmaxf(fmaf(sv[r], P.scale_log2, -m_use), kMinLogP));
+      if (!all_valid) {
+        // out of the sum; its P is written as 1.0, not 0, which the exponent
+        // adds of the PV waves could take to -inf (its V row is zeros)
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+          if (!((vb8 >> r) & 1u)) pv[r] = 0.f;
+      }
+      l_run += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+      if (!all_valid) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+          if (!((vb8 >> r) & 1u)) pv[r] = 1.f;
+      }
+      *reinterpret_cast<v4i*>(smem + kPOff + (t & 1) * 8192 + hp * 4096 + dh * 1024 + lane * 16) =
+          v4i{cvt_pk_bf16(pv[0], pv[1]), cvt_pk_bf16(pv[2], pv[3]), cvt_pk_bf16(pv[4], pv[5]), cvt_pk_bf16(pv[6], pv[7])};
+    }
+    if (t < c.nblk && h == 0) ref[(((t & 1) * 2 + hp) * 2 + dh) * 32 + c32] = m_run;
+    iteration_end();
+  }
+  float* fin = reinterpret_cast<float*>(smem + kFinOff);
+  const float l2 = l_run + shfl_xor(l_run, 32);
+  if (h == 0) {
+    fin[(hp * 2 + dh) * 32 + c32] = l2;
+    fin[128 + (hp * 2 + dh) * 32 + c32] = m_run;
+    fin[256 + (hp * 2 + dh) * 32 + c32] = m_max;
+  }
+  barrier();
+}
+
 // PV waves: O += P'(t-1) . V(t-1) against R, then the normalised output.
 // Wave dq = w - 4 owns O[64 heads x dims 128dq .. 128dq+127], exactly V tile
 // dq, as two head tiles (the head halves): each V byte is converted once per
@@ -725,19 +871,17 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
           if (kKeys != kRows) eq[nxt] = *reinterpret_cast<const v4i_alias*>(et + ((ks + 1) * 2 + h) * 8);
         }
         __builtin_amdgcn_sched_barrier(0);
-        const int k2 = ks >> 1;  // k-steps 0, 1: key half 0; 2, 3: key half 1
+        // cache slots: k-steps 0, 1 are key half 0, 2, 3 half 1; rows only: k-step ks has its own reference
+        const int k2 = kKeys == kRows ? ks : ks >> 1;
+        if (kKeys == kRows && ks == 1) barrier();  // the QK waves' partial scores change hands
         if (fresh && ks >= 2) continue;  // a fresh block's 32 keys are k-steps 0, 1
         v4i pa[kTiles];
 #pragma unroll
         for (int mt = 0; mt < kTiles; ++mt)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            if (kKeys == kRows) {  // one key half: its reference is R, and there are no tile scales
-              pa[mt][e] = pq[cur][mt][e];
-              continue;
-            }
             // (bit_cast of a vector element reads element 0; copy to scalars first)
-            const int pe = pq[cur][mt][e], ee = fresh ? 0 : eq[cur][e];
+            const int pe = pq[cur][mt][e], ee = kKeys == kRows || fresh ? 0 : eq[cur][e];
             const v2u16 sum = __builtin_bit_cast(v2u16, pe) + __builtin_bit_cast(v2u16, ee) +
                               __builtin_bit_cast(v2u16, fx[mt][k2]);
             pa[mt][e] = __builtin_bit_cast(int, sum);
@@ -761,6 +905,8 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
             o[mt][nn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(pa[mt]), vop, o[mt][nn], 0, 0, 0);
         }
       }
+    } else if (kKeys == kRows) {
+      barrier();
     }
     iteration_end();
   }
@@ -904,8 +1050,10 @@ sparse_mla_kernel(const MlaParams P) {
     else issue_fresh_block(smem, 0, smem, c.wave, c.lane);
   }
   // both roles run the same number of iterations and barriers
-  if (c.wave < 4) qk_waves<kKeys, kTiles>(P, smem, c, dl);
-  else pv_waves<kKeys, kTiles>(P, smem, c, dl, split);
+  if (c.wave < 4) {
+    if constexpr (kKeys == kRows) qk_waves_rows<kTiles>(P, smem, c, dl);
+    else qk_waves<kKeys, kTiles>(P, smem, c, dl);
+  } else pv_waves<kKeys, kTiles>(P, smem, c, dl, split);
 }
 
 // One 64-thread workgroup per (split item, head): merge the split partials.

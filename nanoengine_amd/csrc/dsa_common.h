@@ -118,11 +118,11 @@ int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max
 int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max_len, PrefillList* ws,
                        const int32_t* offsets, int32_t* out, int top_k, int rows, hipStream_t stream);
 
-// The exact top-k of whole rows of order keys keys[row * key_stride + t], t <
-// the row's length (topk.hip), with the page translation. max_len <=
-// kRowSelectLen; key_stride is a multiple of 4.
-constexpr int kRowSelectLen = 16384;
-int launch_row_select(const uint32_t* keys, int64_t key_stride, const int32_t* seq_lens, int64_t max_len,
+// The exact top-k of whole rows of scores[row * score_stride + t], t < the
+// row's length (topk.hip), with the page translation. max_len <=
+// kRowSelectLen; 16-byte aligned rows.
+constexpr int kRowSelectLen = 65536;
+int launch_row_select(const float* scores, int64_t score_stride, const int32_t* seq_lens, int64_t max_len,
                       const int32_t* page_table, int64_t pt_stride, int pt_div, uint32_t page_bits, int32_t* out_page,
                       int32_t* out_raw, int top_k, int rows, hipStream_t stream);
 

@@ -402,8 +402,9 @@ indexer_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
 // flushed to the row's list with one global atomic when the batch entry
 // changes, when the stage could overflow, and at the end.
 //
-// kStore: the pages' order keys go to keys[row * key_stride + t] instead (the
-// score pass of short contexts, whose select reads whole rows).
+// kStore: every score of the pages goes to scores[row * score_stride + t]
+// instead (the logits operator, and the score pass of short contexts, whose
+// select reads whole rows), -inf past the row's length to the end of the page.
 constexpr int kFiltStageCap = 384;   // staged candidates per wave and query token
 constexpr int kFiltWindow = 64;      // block-table entries a wave holds (one per lane)
 constexpr int kFiltAdvance = 60;     // pages per window refill (a multiple of the 3- and 4-buffer rotations)
@@ -423,7 +424,7 @@ __global__ void __launch_bounds__(kIdxThreads) __attribute__((amdgpu_waves_per_e
 indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kv,
                       const float* __restrict__ weights, const int32_t* __restrict__ ctx_lens,
                       const int32_t* __restrict__ block_tables, int64_t bt_stride, int64_t max_ctx, int batch,
-                      int top_k, DecodeList* __restrict__ ws, uint32_t* __restrict__ keys, int64_t key_stride) {
+                      int top_k, DecodeList* __restrict__ ws, float* __restrict__ scores, int64_t score_stride) {
   extern __shared__ __align__(16) uint8_t fl_smem[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   FiltWaveStage& st = reinterpret_cast<FiltWaveStage*>(fl_smem)[wave];
@@ -550,11 +551,12 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
       if (cnt[j] > kFiltStageCap - kIdxPageTokens) flush(j);
       const float v = page_head_sum<NQ>(pr, j, lane, qa, w);
       const int t = page * kIdxPageTokens + lane;
-      const uint32_t key = order_key(v * pr.scale);
       if constexpr (kStore) {
-        if (t < L[j]) keys[(int64_t)(b * NQ + j) * key_stride + t] = key;
+        if (t < max_ctx)
+          scores[(int64_t)(b * NQ + j) * score_stride + t] = t < L[j] ? v * pr.scale : -__builtin_inff();
         continue;
       }
+      const uint32_t key = order_key(v * pr.scale);
       const bool pred = t < L[j] && key >= tk[j];
       const uint64_t m = __ballot(pred);
       if (pred) {
@@ -589,6 +591,10 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
   for (int j = 0; j < NQ; ++j) flush(j);
 }
 
+// The most tokens (rows times the longest context) scored by the persistent
+// kernel and kept; the callers give the measurements.
+constexpr int64_t kScoreTokens = 3 << 20;
+
 static int filter_grid() {
   static int grid = 0;
   if (grid == 0) {
@@ -601,12 +607,12 @@ static int filter_grid() {
   return grid;
 }
 
-// The persistent filter (or, with keys, score) pass; false when the batch does
+// The persistent filter (or, with scores, score) pass; false when the batch does
 // not fit its LDS prefix.
 static bool launch_filter_persistent(const uint8_t* q, const uint8_t* kv, const float* weights,
                                      const int32_t* ctx_lens, const int32_t* bt, int64_t bt_stride, int batch,
-                                     int next_n, int64_t max_ctx, int top_k, DecodeList* ws, uint32_t* keys,
-                                     int64_t key_stride, hipStream_t stream) {
+                                     int next_n, int64_t max_ctx, int top_k, DecodeList* ws, float* scores,
+                                     int64_t score_stride, hipStream_t stream) {
   if (batch > kFiltMaxBatch) return false;
   const size_t smem = filt_smem_bytes(batch);
   using Kernel = decltype(&indexer_filter_kernel<1, false>);
@@ -621,8 +627,8 @@ static bool launch_filter_persistent(const uint8_t* q, const uint8_t* kv, const 
           return false;
     attr_set = true;
   }
-  hipLaunchKernelGGL(kernels[next_n - 1][keys ? 1 : 0], dim3((unsigned)filter_grid()), dim3(kIdxThreads), smem, stream,
-                     q, kv, weights, ctx_lens, bt, bt_stride, max_ctx, batch, top_k, ws, keys, key_stride);
+  hipLaunchKernelGGL(kernels[next_n - 1][scores ? 1 : 0], dim3((unsigned)filter_grid()), dim3(kIdxThreads), smem, stream,
+                     q, kv, weights, ctx_lens, bt, bt_stride, max_ctx, batch, top_k, ws, scores, score_stride);
   return true;
 }
 
@@ -662,6 +668,15 @@ extern "C" int dsa_indexer_logits(const uint8_t* q_fp8, const uint8_t* kv_cache,
     return set_error(kInvalidArgument, "indexer: null pointer");
   if ((reinterpret_cast<uintptr_t>(q_fp8) | reinterpret_cast<uintptr_t>(kv_cache)) & 15)
     return set_error(kInvalidArgument, "indexer: q and kv_cache must be 16-byte aligned");
+  // The persistent score pass deals pages out evenly, whatever the lengths (33
+  // rows of 3K to 40K tokens: 23.7 us against 28.0 of one workgroup per 24
+  // pages; 64 rows of 16K 28.4 / 31.8, 32 of 64K 52 / 55). Past kScoreTokens
+  // there are workgroups enough and it loses by a little: 256 x 16K 106 / 106,
+  // 128 x 64K 220 / 205.
+  if (batch * max_context_len <= kScoreTokens &&
+      launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch, next_n,
+                               max_context_len, 0, nullptr, logits, logits_stride, (hipStream_t)stream))
+    return check_launch("dsa_indexer_logits");
   const int64_t max_pages = (max_context_len + kIdxPageTokens - 1) / kIdxPageTokens;
   IdxOut o{logits, logits_stride, nullptr, 0};
   launch_indexer<kIdxStore>(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch, next_n,
@@ -734,20 +749,21 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
     if (phase_events && phase_events[i]) (void)hipEventRecord((hipEvent_t)phase_events[i], st);
   };
   mark(0);
-  // Short contexts: every score (as order keys, in the logits buffer), then a
-  // select over whole rows. The sample pass and the list, which pay for
-  // themselves on long rows, are two thirds of the indexer's time on short
-  // ones. Indexer us, lists against whole rows: 4 x 4K 24.5 / 15.3, 64 x 16K
-  // 50.4 / 42.6, 1024 x 8K 287 / 259; over 8K tokens the row select loses once
-  // its rows pass one round of the CUs (256 x 16K 119 / 121, 512 x 16K 237 / 249).
-  if (max_context_len <= kRowSelectLen / 2 || (max_context_len <= kRowSelectLen && rows <= 192)) {
-    uint32_t* keys = reinterpret_cast<uint32_t*>(f.logits);
+  // Short contexts and few long ones: every score (in the logits buffer), then
+  // a select over whole rows. The sample pass and the list pay for themselves
+  // where the scores' own bytes and the row select's rounds of the CUs do not.
+  // Indexer us, lists against whole rows: 4 x 4K 24.5 / 15.3, 64 x 16K 49.7 /
+  // 39.4, 1024 x 8K 284 / 256, 200 x 16K 77 / 67 but 250 x 16K 116 / 120;
+  // 8 x 32K 32.9 / 24.3, 64 x 32K 71.2 / 67.6 but 128 x 32K 116 / 122; 1 x 64K
+  // 36.1 / 28.7, 8 x 64K 39.8 / 40.0, 32 x 64K 71 / 76.
+  if (max_context_len <= 8192 || (max_context_len <= 32768 && rows * max_context_len <= kScoreTokens) ||
+      (max_context_len <= kRowSelectLen && rows <= 2)) {
     if (launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,
-                                 next_n, max_context_len, top_k, nullptr, keys, f.logits_stride, st)) {
+                                 next_n, max_context_len, top_k, nullptr, f.logits, f.logits_stride, st)) {
       if (int rc = check_launch("dsa_indexer_topk(scores)")) return rc;
       mark(1);
       mark(2);
-      const int rc = launch_row_select(keys, f.logits_stride, context_lens, max_context_len, block_tables,
+      const int rc = launch_row_select(f.logits, f.logits_stride, context_lens, max_context_len, block_tables,
                                        block_table_stride, next_n, 6u, out_physical, out_logical, top_k, rows, st);
       mark(3);
       mark(4);

@@ -52,15 +52,18 @@ __device__ uint32_t block_exclusive_scan(uint32_t* wave_sum, uint32_t x, uint32_
 // fall into the end bins or all into one.
 struct ScoreBins {
   float lo, scale;
-  __device__ __forceinline__ ScoreBins(uint32_t kmin, uint32_t kmax) {
-    lo = key_to_float(kmin);
-    const float range = key_to_float(kmax) - lo;
+  __device__ __forceinline__ ScoreBins(float lowest, float highest) {
+    lo = lowest;
+    const float range = highest - lowest;
     scale = range > 0.f && range < 3.0e38f ? (float)(kHistBins - 1) / range : 0.f;
   }
-  __device__ __forceinline__ uint32_t of(uint32_t key) const {
-    const float x = (key_to_float(key) - lo) * scale;  // NaN (inf * 0) maps to bin 0
+  __device__ __forceinline__ ScoreBins(uint32_t kmin, uint32_t kmax)
+      : ScoreBins(key_to_float(kmin), key_to_float(kmax)) {}
+  __device__ __forceinline__ uint32_t bin(float score) const {
+    const float x = (score - lo) * scale;  // NaN (inf * 0) maps to bin 0
     return (uint32_t)fminf(fmaxf(x, 0.f), (float)(kHistBins - 1));
   }
+  __device__ __forceinline__ uint32_t of(uint32_t key) const { return bin(key_to_float(key)); }
 };
 
 // The 12-bit digits, from the top, of the composites of keys in [kmin, kmax]:
@@ -73,6 +76,10 @@ struct CompositeDigits {
   __device__ __forceinline__ int bins(int level) const {
     const int top = total_bits - 12 * level;
     return 1 << (top - max(top - 12, 0));
+  }
+  // the digits above `level`, as one number
+  __device__ __forceinline__ uint64_t above(uint32_t key, uint32_t pos, int level) const {
+    return rank_composite(key - kmin, pos) >> (total_bits - 12 * level);
   }
   __device__ __forceinline__ uint32_t of(uint32_t key, uint32_t pos, int level) const {
     const int top = total_bits - 12 * level;

@@ -7,9 +7,9 @@
 // positions (NaN ranks as -inf). Digits are 12/10/10 bits of the score key and
 // 9/9 bits of the inverted position.
 //
-// Rows of at most 64K positions take one launch (topk_onepass_kernel: the
-// row in registers, a 1/8 sample for the threshold, the candidates listed in
-// LDS). Longer or ragged rows take three launches on the caller's stream:
+// Aligned rows of at most 64K positions take one launch (topk_row_kernel: the
+// row in registers, binned by score). Longer, ragged or unaligned rows take
+// three launches on the caller's stream:
 //   1. threshold (one workgroup per row): a 1/8 sample of the row (contiguous
 //      1024-element chunks, one in eight) gives, by a two-digit radix on the
 //      sample, a score threshold t with about k + 4 sqrt(k) elements expected
@@ -25,12 +25,9 @@
 //      needs no bound at all. The selected positions are marked in an LDS
 //      bitmap, compacted with one block prefix scan (ascending order, so the
 //      output is deterministic) and written with the page translation.
-// No global sort, no bounded candidate buffer on the exact path. The
-// one-launch kernel's list select radixes over
-// [ key - t : nb bits ][ (2^18-1) - position : 18 bits ] instead, nb the bit
-// length of the largest key - t, so that its digits spread over the
-// candidates' own range; the fused indexer's (topk_list_kernel) takes the
-// score's linear bin as its first digit.
+// No global sort, no bounded candidate buffer on the exact path. The row
+// select and the fused indexer's list select (topk_list_kernel) take the
+// score's linear bin as their first digit.
 #include <mutex>
 
 #include "dsa_common.h"
@@ -486,312 +483,6 @@ topk_finish_kernel(const RowIn in, RowWs* __restrict__ ws, const int32_t* __rest
              out_page, out_raw, top_k, blockIdx.x);
 }
 
-// ---------------------------------------------------------------- one launch
-// Rows of up to 64K positions: one 512-thread workgroup per row holds the
-// whole row in registers (128 order keys per thread), so every pass after the
-// one HBM read runs on registers and LDS:
-//   1. a 1/8 sample (every 8th register slot, spread over the row) gives the
-//      score threshold t by a two-digit radix, exactly as the threshold kernel;
-//   2. each thread counts its keys >= t; one block scan gives every thread its
-//      place in the candidate list, which goes to LDS in thread order;
-//   3. if the list holds between k and kListCap entries, the exact top-k is the
-//      exact top-k of the list (radix levels in LDS); otherwise the levels run
-//      over the registers (the same result without any bound);
-//   4. bitmap compaction in position order and the page translation.
-constexpr int kRegThreads = 512;
-constexpr int kRegPerThread = 128;
-constexpr int kRegMaxLen = kRegThreads * kRegPerThread;  // 65536
-
-// Position of register slot i of thread t (slot i = element i%4 of float4 chunk i/4).
-__device__ __forceinline__ int reg_pos(int t, int i) { return 4 * kRegThreads * (i >> 2) + 4 * t + (i & 3); }
-
-// Exact selection of the `remain` largest of the n composites in list 0 of
-// LDS (hi = key - t_key, lo = (2^18 - 1) - position, so every composite is
-// distinct and equal keys favour the lower position): radix levels of 12
-// bits from the top of the nb + 18 bit composite, nb = bit length of the
-// largest hi (`hmax`), so that the digits spread over the candidates' own
-// range. Marks the selected positions in the (cleared) LDS bitmap. All NT
-// threads call it after a barrier; it ends with one.
-template <int NT>
-__device__ void composite_select(TopkSmem& s, uint32_t n, uint32_t remain, uint32_t hmax) {
-  const int tid = threadIdx.x;
-  const int nb = 32 - __clz(hmax);  // bits of the key part (0: all equal)
-  const int total_bits = nb + 18;
-  const int nlev = (total_bits + 11) / 12;
-  auto digit = [&](uint32_t h, uint32_t p, int L) {
-    const uint64_t c = ((uint64_t)h << 18) | p;
-    const int top = total_bits - 12 * L;
-    const int lo_b = max(top - 12, 0);
-    return (uint32_t)((c >> lo_b) & ((1ull << (top - lo_b)) - 1ull));
-  };
-  int cur = 0;
-  for (int L = 0; L < nlev; ++L) {
-    const int top = total_bits - 12 * L;
-    const int nbins = 1 << (top - max(top - 12, 0));
-    const int nxt = cur ^ 1;
-    // list_count[cur] (the length of this level's list) was read by every
-    // thread before the previous barrier; list_count[nxt] is free
-    for (int i = tid; i < nbins; i += NT) s.hist[i] = 0u;
-    if (tid == 0) s.list_count[nxt] = 0u;
-    __syncthreads();
-    for (uint32_t e = tid; e < n; e += NT) atomicAdd(&s.hist[digit(s.list_key[cur][e], s.list_pos[cur][e], L)], 1u);
-    __syncthreads();
-    find_threshold<NT>(s.hist, s.wave_sum, nbins, remain, &s.tb, &s.above, &s.eq);
-    const uint32_t tb = s.tb, above = s.above, eq = s.eq;
-    remain -= above;
-    const bool last = (eq == remain) || L == nlev - 1;
-    for (uint32_t e = tid; e < n; e += NT) {
-      const uint32_t h = s.list_key[cur][e], p = s.list_pos[cur][e];
-      const uint32_t d = digit(h, p, L);
-      if (d > tb || (last && d == tb)) {
-        const uint32_t pos = kIdxMax - p;
-        atomicOr(&s.bitmap[pos >> 5], 1u << (pos & 31));
-      } else if (!last && d == tb) {
-        const uint32_t slot = atomicAdd(&s.list_count[nxt], 1u);
-        s.list_key[nxt][slot] = h;
-        s.list_pos[nxt][slot] = p;
-      }
-    }
-    __syncthreads();
-    if (last) break;
-    n = s.list_count[nxt];
-    cur = nxt;
-    __syncthreads();  // every thread has read the next level's length
-  }
-}
-
-__global__ void __launch_bounds__(kRegThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
-topk_onepass_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32_t* __restrict__ page_table,
-                    int64_t pt_stride, uint32_t page_bits, int32_t* __restrict__ out_page,
-                    int32_t* __restrict__ out_raw, int top_k) {
-  extern __shared__ __align__(16) uint8_t smem_raw[];
-  TopkSmem& s = *reinterpret_cast<TopkSmem*>(smem_raw);
-  constexpr int NT = kRegThreads;
-  const int tid = threadIdx.x;
-  const int b = blockIdx.x;
-  const int len = in.len(b);
-  const float* row = in.row(b);
-
-  RowOut out;
-  out.page = out_page + (int64_t)b * top_k;
-  out.raw = out_raw ? out_raw + (int64_t)b * top_k : nullptr;
-  out.pt = page_table ? page_table + (int64_t)b * pt_stride : nullptr;
-  out.page_bits = page_bits;
-  out.offset = offsets ? offsets[b] : 0;
-
-  if (len <= top_k) {
-    for (int i = tid; i < top_k; i += NT) out.emit(i, i < len ? i : -1);
-    return;
-  }
-
-  // ---- the row, as order keys (0 = beyond the row: below every real key).
-  // The launcher guarantees 16-byte aligned rows.
-  uint32_t key[kRegPerThread];
-  // Every load is in bounds: a chunk past the row's storage re-reads the
-  // row's last aligned chunk (len > top_k >= 4 here), and the keys of
-  // positions >= len are masked to 0, so no load sits behind a branch.
-  const int last = (int)((in.max_len - 4) & ~(int64_t)3);
-#pragma unroll
-  for (int j = 0; j < kRegPerThread / 4; ++j) {
-    const int p = 4 * kRegThreads * j + 4 * tid;
-    const v4f v = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(row + min(p, last)));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) key[4 * j + e] = p + e < len ? in.key(v[e]) : 0u;
-  }
-
-  const int nwords = (len + 31) >> 5;
-  for (int i = tid; i < nwords; i += NT) s.bitmap[i] = 0u;
-  for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
-  if (tid < 2) s.list_count[tid] = 0u;
-  __syncthreads();
-
-  // ---- 1. threshold from the sample (slots 0, 8, 16, ...): a key at or
-  // below the sample's rank-r key, from two 1024-bin histogram levels over the
-  // sample's own [min, max] key range (binning raw order keys would put the
-  // sample into the few bins its sign and exponent span, and the LDS atomics
-  // would serialise)
-  uint32_t my_samples = 0, kmin = 0xffffffffu, kmax = 0u;
-#pragma unroll
-  for (int m = 0; m < kRegPerThread / 8; ++m)
-    if (key[8 * m]) {
-      ++my_samples;
-      kmin = min(kmin, key[8 * m]);
-      kmax = max(kmax, key[8 * m]);
-    }
-  const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
-    kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
-  }
-  if (lane == 0) {
-    s.list_count[0] = 0u;
-    s.bitmap[kBitmapWords - 1 - wave] = kmin;  // scratch words far past any row of <= 64K positions
-    s.bitmap[kBitmapWords - 1 - NT / 64 - wave] = kmax;
-  }
-  uint32_t nsample = 0;
-  (void)block_exclusive_scan<NT>(s.wave_sum, my_samples, &nsample);
-  __syncthreads();
-#pragma unroll
-  for (int w2 = 0; w2 < NT / 64; ++w2) {
-    kmin = min(kmin, s.bitmap[kBitmapWords - 1 - w2]);
-    kmax = max(kmax, s.bitmap[kBitmapWords - 1 - NT / 64 - w2]);
-  }
-  const float fk = (float)nsample / (float)len * (float)top_k;
-  const uint32_t r = (uint32_t)(fk + 4.f * sqrtf(fk) + 8.f);
-  uint32_t t_key = 1u;  // every real key is >= 0x007fffff
-  if (r < nsample) {
-    const int shift = max(0, 32 - (int)__clz(kmax - kmin) - 10);
-#pragma unroll
-    for (int m = 0; m < kRegPerThread / 8; ++m)
-      if (key[8 * m]) atomicAdd(&s.hist[(key[8 * m] - kmin) >> shift], 1u);
-    __syncthreads();
-    find_threshold<NT>(s.hist, s.wave_sum, 1024, r, &s.tb, &s.above, &s.eq);
-    const uint32_t tb0 = s.tb, rem0 = r - s.above;
-    t_key = kmin + (tb0 << shift);
-    if (shift > 0) {
-      const int shift2 = max(0, shift - 10);
-      __syncthreads();
-      for (int i = tid; i < 1024; i += NT) s.hist[i] = 0u;
-      __syncthreads();
-#pragma unroll
-      for (int m = 0; m < kRegPerThread / 8; ++m)
-        if (key[8 * m] && ((key[8 * m] - kmin) >> shift) == tb0)
-          atomicAdd(&s.hist[((key[8 * m] - kmin) >> shift2) & 1023u], 1u);
-      __syncthreads();
-      find_threshold<NT>(s.hist, s.wave_sum, 1024, rem0, &s.tb, &s.above, &s.eq);
-      t_key += s.tb << shift2;
-    }
-    t_key = max(t_key, 1u);
-  }
-
-  // ---- 2. candidates >= t, written in thread order after one block scan; a
-  // slot that no lane of the wave fills costs one compare and one ballot
-  uint32_t mine = 0;
-#pragma unroll
-  for (int i = 0; i < kRegPerThread; ++i) mine += key[i] >= t_key ? 1u : 0u;
-  uint32_t total_cand = 0;
-  uint32_t put = block_exclusive_scan<NT>(s.wave_sum, mine, &total_cand);
-  if (total_cand <= (uint32_t)kListCap) {
-    // positions recomputed here from an opaque thread id: computed once and
-    // kept, they would take as many registers as the keys
-    int t_o = tid;
-    uint32_t t_k = t_key;  // opaque too: the counting loop's compares are not kept
-    asm volatile("" : "+v"(t_o), "+v"(t_k));
-#pragma unroll
-    for (int i = 0; i < kRegPerThread; ++i) {
-      const bool pred = key[i] >= t_k;
-      if (__ballot(pred)) {
-        if (pred) {
-          s.list_key[0][put] = key[i];
-          s.list_pos[0][put] = (uint32_t)reg_pos(t_o, i);
-        }
-        put += pred ? 1u : 0u;
-      }
-    }
-  }
-  const uint32_t cand = total_cand;
-  const bool listed = cand >= (uint32_t)top_k && cand <= (uint32_t)kListCap;
-  if (listed) {
-    // ---- 3. exact select over the list: composites in place, their max
-    __syncthreads();  // the list is written
-    uint32_t mx = 0;
-    for (uint32_t e = tid; e < cand; e += NT) {
-      const uint32_t h = s.list_key[0][e] - t_key;
-      s.list_key[0][e] = h;
-      s.list_pos[0][e] = kIdxMax - s.list_pos[0][e];
-      mx = max(mx, h);
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
-    if (lane == 0) s.wave_sum[wave] = mx;
-    __syncthreads();
-    mx = 0;
-#pragma unroll
-    for (int w2 = 0; w2 < NT / 64; ++w2) mx = max(mx, s.wave_sum[w2]);
-    __syncthreads();  // wave_sum is read before composite_select reuses it
-    composite_select<NT>(s, cand, (uint32_t)top_k, mx);
-  } else {
-  for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
-  __syncthreads();
-  if (listed) {
-    for (uint32_t e = tid; e < cand; e += NT) atomicAdd(&s.hist[s.list_key[0][e] >> 20], 1u);
-  } else {
-#pragma unroll
-    for (int i = 0; i < kRegPerThread; ++i)
-      if (key[i]) atomicAdd(&s.hist[key[i] >> 20], 1u);
-  }
-  __syncthreads();
-
-  // ---- 3. exact radix levels over the list (LDS) or, when the sample missed,
-  // over the row re-read from memory (the registers are free by then)
-  uint32_t thr[kLevels] = {0, 0, 0, 0, 0};
-  uint32_t remain = (uint32_t)top_k;
-  bool source_mode = !listed;
-  int cur = 0;
-  uint32_t list_n = listed ? cand : 0u;
-  for (int level = 0; level < kLevels; ++level) {
-    find_threshold<NT>(s.hist, s.wave_sum, radix_bins(level), remain, &s.tb, &s.above, &s.eq);
-    const uint32_t tb = s.tb, above = s.above, eq = s.eq;
-    thr[level] = tb;
-    remain -= above;
-    const bool take_all = (eq == remain) || level == kLevels - 1;
-    const bool collect = !take_all && (!source_mode || eq <= (uint32_t)kListCap);
-    const int nxt = cur ^ 1;
-    __syncthreads();
-    if (!take_all) {
-      for (int i = tid; i < radix_bins(level + 1); i += NT) s.hist[i] = 0u;
-      if (tid == 0) s.list_count[nxt] = 0u;
-    }
-    __syncthreads();
-    auto visit = [&](uint32_t k, uint32_t pos) {
-      const uint32_t d = radix_digit(level, k, pos);
-      if (d > tb || (take_all && d == tb)) atomicOr(&s.bitmap[pos >> 5], 1u << (pos & 31));
-      if (!take_all && d == tb) {
-        atomicAdd(&s.hist[radix_digit(level + 1, k, pos)], 1u);
-        if (collect) {
-          const uint32_t sl = atomicAdd(&s.list_count[nxt], 1u);
-          s.list_key[nxt][sl] = k;
-          s.list_pos[nxt][sl] = pos;
-        }
-      }
-    };
-    if (source_mode) {
-      for (int base = 0; base < len; base += 4 * NT) {
-        float x[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = base + j * NT + tid;
-          x[j] = i < len ? row[i] : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = base + j * NT + tid;
-          const uint32_t k = in.key(x[j]);
-          if (i < len && in_bucket(level, k, (uint32_t)i, thr)) visit(k, (uint32_t)i);
-        }
-      }
-    } else {
-      for (uint32_t e = tid; e < list_n; e += NT) visit(s.list_key[cur][e], s.list_pos[cur][e]);
-    }
-    __syncthreads();
-    if (take_all) break;
-    if (collect) {
-      source_mode = false;
-      cur = nxt;
-      list_n = s.list_count[cur];
-    }
-  }
-
-  }
-
-  // ---- 4. compaction in position order (two words per thread) and output
-  uint32_t* sel = s.list_pos[0];
-  uint32_t total = 0;
-  compact_bitmap<NT>(s.bitmap, nwords, s.wave_sum, sel, top_k, &total);
-  for (int i = tid; i < top_k; i += NT) out.emit(i, i < (int)total ? (int32_t)sel[i] : -1);
-}
-
 // ---------------------------------------------------------------- list select
 // Exact top-k of a row's candidate list (fused indexer path), ranked by
 // (score, lower position). The first digit is the score's linear bin; the
@@ -1065,14 +756,23 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 }
 
 // ---------------------------------------------------------------- row select
-// Exact top-k of a short row's order keys by one workgroup: thread t holds the
-// positions [per t, per (t + 1)), per a multiple of 4 up to kPer, so the
-// selected ones come out in position order by one block scan of bit counts.
-// Instantiated for 4K, 8K and 16K positions: the 16K kernel takes 3 us longer
-// over 64 rows of 4K than the 4K one.
-// First digit: the score's linear bin; the threshold bin's few elements count
-// those ahead of them, or, where many scores tie, take radix levels.
+// Exact top-k of a row of up to 64K scores by one workgroup, which reads the
+// row once: thread t holds positions [4t, 4t + 4) of every chunk of 4096 in
+// registers. First digit: the score's linear bin, counted over the whole row;
+// the threshold bin's few elements count those ahead of them, or, where many
+// scores tie, take radix levels. The selected positions are a bitmap in LDS,
+// compacted in position order by one block scan.
+//
+// What bounds it: a chain of short phases in one CU (loads, extremes, LDS
+// histogram, threshold, ranks, compaction). A 1/8 sample's threshold, the
+// candidates above it listed and three radix levels over the list took
+// 35.5 us for 33 rows of 3K to 40K where this takes 16.4; 64 rows of 16K take 8.7.
+// Instantiated per power of two of the row's chunks: a kernel for longer rows
+// spends its registers and tests on chunks that a short one does not have.
 constexpr int kRowThreads = 1024;
+constexpr int kRowChunk = 4 * kRowThreads;
+constexpr int kRowMaxChunks = kRowSelectLen / kRowChunk;
+static_assert(kRowMaxChunks == 16, "the largest instantiation");
 struct RowSelectSmem {
   uint32_t hist[kHistBins];  // then the selected positions
   uint64_t rank[kRankCap];
@@ -1081,130 +781,223 @@ struct RowSelectSmem {
   uint32_t count, tb, above, eq;
 };
 
-template <int kRowPer>
+// Bitwise or over each group of 8 lanes.
+__device__ __forceinline__ uint32_t or_8_lanes(uint32_t x) {
+  x |= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true);   // lane ^ 1
+  x |= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true);   // lane ^ 2
+  x |= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, true);  // lane ^ 7: the other four
+  return x;
+}
+
+template <int kChunks>
 __global__ void __launch_bounds__(kRowThreads)
-topk_row_kernel(const uint32_t* __restrict__ keys, int64_t key_stride, const int32_t* __restrict__ seq_lens,
-                int64_t max_len, const int32_t* __restrict__ page_table, int64_t pt_stride, int pt_div,
-                uint32_t page_bits, int32_t* __restrict__ out_page, int32_t* __restrict__ out_raw, int top_k) {
+topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32_t* __restrict__ page_table,
+                int64_t pt_stride, int pt_div, uint32_t page_bits, int32_t* __restrict__ out_page,
+                int32_t* __restrict__ out_raw, int top_k) {
   __shared__ __align__(16) RowSelectSmem s;
   constexpr int NT = kRowThreads, NW = NT / 64;
-  static_assert(kRowPer % 4 == 0 && kRowPer <= 32, "a thread's positions are a 32-bit mask");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int b = blockIdx.x;
-  const int64_t l = seq_lens[b];
-  const int len = (int)(l < 0 ? 0 : (l > max_len ? max_len : l));
+  const int len = in.len(b);
   const RowOut out{out_page + (int64_t)b * top_k, out_raw ? out_raw + (int64_t)b * top_k : nullptr,
-                   page_table + (int64_t)(b / pt_div) * pt_stride, page_bits, 0};
+                   page_table ? page_table + (int64_t)(b / pt_div) * pt_stride : nullptr, page_bits,
+                   offsets ? offsets[b] : 0};
   if (len <= top_k) {
     for (int i = tid; i < top_k; i += NT) out.emit(i, i < len ? i : -1);
     return;
   }
-  const int per = (len + 4 * NT - 1) / (4 * NT) * 4;
-  const int p0 = per * tid;
-  const uint32_t* row = keys + (int64_t)b * key_stride;
-  uint32_t key[kRowPer];  // 0: past the row, below every key
+  const float* row = in.row(b);
+  const int nch = (len + kRowChunk - 1) / kRowChunk;
+  const float inf = __builtin_inff();
+
+  // ---- the row. The launcher guarantees 16-byte aligned rows; a quad that
+  // would pass the row's storage reads the last whole quad instead, so no load
+  // sits behind a lane's branch, and the storage's last max_len % 4 scores are
+  // read one by one. Positions at or past the length hold -inf: they rank
+  // behind all len > top_k real elements, so they are never selected.
+  const int last = (int)((in.max_len - 4) & ~(int64_t)3);
+  float x[4 * kChunks];
 #pragma unroll
-  for (int c = 0; c < kRowPer; c += 4) {
-    uint4 x = {0u, 0u, 0u, 0u};
-    if (c < per && p0 + c < len) x = *reinterpret_cast<const uint4*>(row + p0 + c);  // (rows are padded to 4 keys)
-    key[c] = x.x;
-    key[c + 1] = p0 + c + 1 < len ? x.y : 0u;
-    key[c + 2] = p0 + c + 2 < len ? x.z : 0u;
-    key[c + 3] = p0 + c + 3 < len ? x.w : 0u;
+  for (int c = 0; c < kChunks; ++c) {
+    v4f v = {-inf, -inf, -inf, -inf};
+    if (c < nch) v = *reinterpret_cast<const v4f*>(row + min(kRowChunk * c + 4 * tid, last));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[4 * c + e] = v[e];
   }
   for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
-  if (tid < kRowSelectLen / 32) s.bits[tid] = 0u;
   if (tid == 0) s.count = 0u;
-  uint32_t kmin = 0xffffffffu, kmax = 0u;
+  // scores that rank as -inf: NaN, and for the indexer's tail |x| >= 1e30
+  const float cap = in.mask_extreme ? __uint_as_float(__float_as_uint(1e30f) - 1u) : inf;
+  auto score = [&](int p, int e, float v) {  // v: what was read for position p + e
+    if (p > last) v = p + e < len ? row[p + e] : -inf;
+    return p + e < len && fabsf(v) <= cap ? v : -inf;
+  };
+  float lo = inf, hi = -inf;  // the extremes; lo of the scores above -inf
 #pragma unroll
-  for (int i = 0; i < kRowPer; ++i) {
-    kmin = min(kmin, key[i] ? key[i] : 0xffffffffu);
-    kmax = max(kmax, key[i]);
-  }
+  for (int c = 0; c < kChunks; ++c)
+    if (c < nch) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float& v = x[4 * c + e];
+        v = score(kRowChunk * c + 4 * tid, e, v);
+        lo = fminf(lo, v > -inf ? v : inf);
+        hi = fmaxf(hi, v);
+      }
+    }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
-    kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
-    kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
+    lo = fminf(lo, __shfl_xor(lo, off, 64));
+    hi = fmaxf(hi, __shfl_xor(hi, off, 64));
   }
+  float* wave_f = reinterpret_cast<float*>(s.wave_sum);
   if (lane == 0) {
-    s.wave_sum[wave] = kmin;
-    s.wave_sum[NW + wave] = kmax;
+    wave_f[wave] = lo;
+    wave_f[NW + wave] = hi;
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    kmin = min(kmin, s.wave_sum[i]);
-    kmax = max(kmax, s.wave_sum[NW + i]);
+    lo = fminf(lo, wave_f[i]);
+    hi = fmaxf(hi, wave_f[NW + i]);
   }
-  const ScoreBins bins(kmin, kmax);
+  // infinities fall into the end bins and do not widen the range
+  const ScoreBins bins(lo, fminf(hi, 3.4028235e38f));
+
+  // ---- first digit
 #pragma unroll
-  for (int i = 0; i < kRowPer; ++i)
-    if (key[i]) atomicAdd(&s.hist[bins.of(key[i])], 1u);
+  for (int c = 0; c < kChunks; ++c)
+    if (c < nch && kRowChunk * c + 4 * tid < len) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) atomicAdd(&s.hist[bins.bin(x[4 * c + e])], 1u);
+    }
   __syncthreads();
   uint32_t remain = (uint32_t)top_k;
   find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
-  uint32_t tb = s.tb;
-  const uint32_t eq = s.eq;
+  const uint32_t tb = s.tb, eq = s.eq;
   remain -= s.above;
   const bool whole_bin = eq == remain;
-  uint32_t mine = 0u, alive = 0u;  // selected, and undecided (in the threshold bin), of this thread's positions
+  const uint32_t sure = whole_bin ? tb : tb + 1;  // bins selected whole
+  const bool ranked = !whole_bin && eq <= (uint32_t)kRankCap;
 #pragma unroll
-  for (int i = 0; i < kRowPer; ++i) {
-    const uint32_t d = bins.of(key[i]);
-    if (key[i] && (d > tb || (whole_bin && d == tb))) mine |= 1u << i;
-    else if (key[i] && d == tb) alive |= 1u << i;
-  }
-  if (!whole_bin && eq <= (uint32_t)kRankCap) {
+  for (int c = 0; c < kChunks; ++c)
+    if (c < nch) {
+      const int p = kRowChunk * c + 4 * tid;
+      uint32_t quad = 0u;
+      if (p < len) {
 #pragma unroll
-    for (int i = 0; i < kRowPer; ++i)
-      if ((alive >> i) & 1u) s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key[i], (uint32_t)(p0 + i));
-    __syncthreads();
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t d = bins.bin(x[4 * c + e]);
+          if (d >= sure) quad |= 1u << e;
+          else if (ranked && d == tb)
+            s.rank[atomicAdd(&s.count, 1u)] = rank_composite(order_key(x[4 * c + e]), (uint32_t)(p + e));
+        }
+      }
+      // eight lanes' quads are a word of the bitmap
+      const uint32_t word = or_8_lanes(quad << (4 * (lane & 7)));
+      if ((lane & 7) == 0) s.bits[p >> 5] = word;
+    }
+  __syncthreads();
+  if (ranked) {
     if ((uint32_t)tid < eq) {
-      const uint64_t c = s.rank[tid];
+      const uint64_t mine = s.rank[tid];
       uint32_t ahead = 0;
-      for (uint32_t e = 0; e < eq; ++e) ahead += s.rank[e] > c ? 1u : 0u;
-      const uint32_t pos = kIdxMax - (uint32_t)(c & kIdxMax);
+      for (uint32_t e = 0; e < eq; ++e) ahead += s.rank[e] > mine ? 1u : 0u;
+      const uint32_t pos = kIdxMax - (uint32_t)(mine & kIdxMax);
       if (ahead < remain) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
+    }
+  } else if (!whole_bin) {
+    // Radix levels over the threshold bin's elements, from their own keys'
+    // range. The row is read again (its second look hits L2), so that this
+    // rare path costs the others no registers.
+    auto each = [&](auto&& visit) {
+#pragma unroll 1
+      for (int c = 0; c < nch; ++c) {
+        const int p = kRowChunk * c + 4 * tid;
+        if (p >= len) continue;
+        const v4f v = *reinterpret_cast<const v4f*>(row + min(p, last));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y = score(p, e, v[e]);
+          if (bins.bin(y) == tb) visit(order_key(y), (uint32_t)(p + e));
+        }
+      }
+    };
+    uint32_t kmin = 0xffffffffu, kmax = 0u;
+    each([&](uint32_t key, uint32_t) {
+      kmin = min(kmin, key);
+      kmax = max(kmax, key);
+    });
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
+      kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
+    }
+    if (lane == 0) {
+      s.wave_sum[wave] = kmin;
+      s.wave_sum[NW + wave] = kmax;
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kRowPer; i += 4)
-      if (i < per && ((alive >> i) & 0xfu)) mine |= (s.bits[(p0 + i) >> 5] >> ((p0 + i) & 31) & 0xfu) << i;
-  } else if (!whole_bin) {
+    for (int i = 0; i < NW; ++i) {
+      kmin = min(kmin, s.wave_sum[i]);
+      kmax = max(kmax, s.wave_sum[NW + i]);
+    }
     const CompositeDigits digits(kmin, kmax);
+    uint64_t prefix = 0;  // the digits chosen so far
     for (int L = 0; L < digits.levels; ++L) {
       __syncthreads();  // every thread has read the previous level's outcome
       for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
       __syncthreads();
-#pragma unroll
-      for (int i = 0; i < kRowPer; ++i)
-        if ((alive >> i) & 1u) atomicAdd(&s.hist[digits.of(key[i], (uint32_t)(p0 + i), L)], 1u);
+      each([&](uint32_t key, uint32_t pos) {
+        if (digits.above(key, pos, L) == prefix) atomicAdd(&s.hist[digits.of(key, pos, L)], 1u);
+      });
       __syncthreads();
       find_threshold<NT>(s.hist, s.wave_sum, digits.bins(L), remain, &s.tb, &s.above, &s.eq);
-      tb = s.tb;
+      const uint32_t t = s.tb;
       remain -= s.above;
-      const bool last = s.eq == remain || L == digits.levels - 1;
-#pragma unroll
-      for (int i = 0; i < kRowPer; ++i) {
-        if (!((alive >> i) & 1u)) continue;
-        const uint32_t d = digits.of(key[i], (uint32_t)(p0 + i), L);
-        if (d > tb || (last && d == tb)) mine |= 1u << i;
-        if (d != tb) alive &= ~(1u << i);
-      }
-      if (last) break;
+      const bool done = s.eq == remain || L == digits.levels - 1;
+      each([&](uint32_t key, uint32_t pos) {
+        const uint32_t d = digits.of(key, pos, L);
+        if (digits.above(key, pos, L) == prefix && (d > t || (done && d == t)))
+          atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
+      });
+      if (done) break;
+      prefix = prefix * (uint32_t)digits.bins(L) + t;
     }
   }
-  // positions in ascending order, then the page translation
+  __syncthreads();
+
+  // ---- positions in ascending order (thread t: `per` of them, a power of two,
+  // at most two words), then the page translation
+  int per = 4;
+  while (per < 4 * nch) per *= 2;
+  uint64_t mine = 0;
+  if (tid * per < nch * kRowChunk) {
+    const uint32_t* w = s.bits + ((tid * per) >> 5);
+    mine = per == 64 ? w[0] | ((uint64_t)w[1] << 32) : (w[0] >> ((tid * per) & 31)) & (0xffffffffu >> (32 - per));
+  }
   uint32_t total = 0;
-  uint32_t at = block_exclusive_scan<NT>(s.wave_sum, (uint32_t)__popc(mine), &total);
+  uint32_t at = block_exclusive_scan<NT>(s.wave_sum, (uint32_t)__popcll(mine), &total);
   __syncthreads();  // the histogram becomes the list of selected positions
   while (mine) {
-    const int i = __ffs(mine) - 1;
+    const int i = __ffsll((unsigned long long)mine) - 1;
     mine &= mine - 1;
-    s.hist[at++] = (uint32_t)(p0 + i);
+    s.hist[at++] = (uint32_t)(tid * per + i);
   }
   __syncthreads();
   for (int i = tid; i < top_k; i += NT) out.emit(i, (int32_t)s.hist[i]);
+}
+
+static void launch_row(const RowIn& in, const int32_t* offsets, const int32_t* page_table, int64_t pt_stride,
+                       int pt_div, uint32_t page_bits, int32_t* out_page, int32_t* out_raw, int top_k, int rows,
+                       hipStream_t stream) {
+  auto* kernel = in.max_len <= kRowChunk       ? topk_row_kernel<1>
+                 : in.max_len <= 2 * kRowChunk ? topk_row_kernel<2>
+                 : in.max_len <= 4 * kRowChunk ? topk_row_kernel<4>
+                 : in.max_len <= 8 * kRowChunk ? topk_row_kernel<8>
+                                               : topk_row_kernel<kRowMaxChunks>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(kRowThreads), 0, stream, in, offsets, page_table, pt_stride, pt_div,
+                     page_bits, out_page, out_raw, top_k);
 }
 
 __global__ void topk_to_physical_kernel(const int32_t* __restrict__ topk, int64_t topk_stride,
@@ -1231,9 +1024,6 @@ static int prepare_topk_kernel() {
   if (status < 0) {
     hipError_t e = hipFuncSetAttribute((const void*)topk_finish_kernel,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTopkSmemBytes);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)topk_onepass_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kTopkSmemBytes);
     if (e == hipSuccess)
       e = hipFuncSetAttribute((const void*)topk_list_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kTopkSmemBytes);
@@ -1284,10 +1074,9 @@ static int launch_topk(const RowIn& in, int batch, const int32_t* offsets, const
                        const char* what) {
   if (int rc = prepare_topk_kernel()) return rc;
   const bool aligned = (reinterpret_cast<uintptr_t>(in.scores) & 15) == 0 && (in.stride & 3) == 0 && !in.row_starts;
-  if (in.max_len <= kRegMaxLen && aligned) {
+  if (in.max_len <= kRowSelectLen && aligned) {
     // the whole row fits in one workgroup's registers: one launch, no workspace
-    hipLaunchKernelGGL(topk_onepass_kernel, dim3(batch), dim3(kRegThreads), kTopkSmemBytes, stream, in, offsets,
-                       page_table, pt_stride, page_bits, out_page, out_raw, top_k);
+    launch_row(in, offsets, page_table, pt_stride, 1, page_bits, out_page, out_raw, top_k, batch, stream);
     return check_launch(what);
   }
   RowWs* ws = nullptr;
@@ -1326,14 +1115,11 @@ int launch_list_select(const RowRepair& rp, const int32_t* seq_lens, int64_t max
   return check_launch("dsa_mqa_topk(select)");
 }
 
-int launch_row_select(const uint32_t* keys, int64_t key_stride, const int32_t* seq_lens, int64_t max_len,
+int launch_row_select(const float* scores, int64_t score_stride, const int32_t* seq_lens, int64_t max_len,
                       const int32_t* page_table, int64_t pt_stride, int pt_div, uint32_t page_bits, int32_t* out_page,
                       int32_t* out_raw, int top_k, int rows, hipStream_t stream) {
-  auto* kernel = max_len <= 4 * kRowThreads   ? topk_row_kernel<4>
-                 : max_len <= 8 * kRowThreads ? topk_row_kernel<8>
-                                              : topk_row_kernel<kRowSelectLen / kRowThreads>;
-  hipLaunchKernelGGL(kernel, dim3(rows), dim3(kRowThreads), 0, stream, keys, key_stride, seq_lens, max_len,
-                     page_table, pt_stride, pt_div, page_bits, out_page, out_raw, top_k);
+  const RowIn in{scores, score_stride, seq_lens, nullptr, max_len, 0};
+  launch_row(in, nullptr, page_table, pt_stride, pt_div, page_bits, out_page, out_raw, top_k, rows, stream);
   return check_launch("dsa_indexer_topk(row select)");
 }
 

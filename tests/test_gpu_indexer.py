@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle as O
-from nanoengine_amd import deep_gemm, indexer as nidx, synth
+from nanoengine_amd import deep_gemm, indexer as nidx, ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -183,3 +183,33 @@ def ops_logits(cuda, q4, cache, w, lens, bt):
                              torch.from_numpy(bt).to(cuda), 64)
     torch.cuda.synchronize()
     return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("next_n", [1, 2])
+def test_both_logits_kernels_agree(cuda, next_n):
+    """The logits kernel is chosen by the batch's size (rows times the longest
+    context): the persistent one's scores, and the -inf to the end of each
+    row's last page, are bit for bit those of the per-workgroup one; neither
+    writes past that page."""
+    lens = [1, 64, 65, 1000, 1537, 4095, 4096, 2500] * 8
+    inp = synth.make_indexer_inputs(lens, next_n=next_n, seed=12, device=cuda)
+    B = len(lens)
+    ctx = nidx._expand_decode_context_lens(inp.context_lens, next_n)
+    q4 = inp.q_fp8.view(torch.float8_e4m3fn).view(B, next_n, 64, 128)
+    kv = inp.cache.view(inp.cache.shape[0], -1)
+    got = []
+    for max_ctx in (4096, 65536):
+        bt = torch.zeros(B, max_ctx // 64, dtype=torch.int32, device=cuda)
+        bt[:, :inp.block_tables.shape[1]] = inp.block_tables
+        out = torch.full((B * next_n, max_ctx), 7.0, device=cuda)
+        ops.indexer_logits(q4, kv, inp.weights, ctx, bt, max_ctx, out=out)
+        got.append(out)
+    assert torch.equal(got[0], got[1][:, :4096])
+    assert (got[1][:, 4096:] == 7.0).all()
+    for b, L in enumerate(lens):
+        end = -(-L // 64) * 64
+        for j in range(next_n):
+            row = got[0][b * next_n + j]
+            real = int(ctx[b, j])
+            assert torch.isfinite(row[:real]).all() and (row[real:end] == -float("inf")).all()
+            assert (row[end:] == 7.0).all()

@@ -135,10 +135,10 @@ def test_fused_max_context_below_some_rows(cuda):
 
 
 @pytest.mark.parametrize("lens,n", [
-    ([28672, 28673, 2048, 2049, 1], 1),        # last row whose marks are bytes, first with bits, rows at top-k
+    ([28672, 28673, 2048, 2049, 1, 70000], 1),  # last row whose marks are bytes, first with bits, rows at top-k
     ([131072, 8192, 6000, 2047], 1),           # each row is sampled by its own length
     ([131072, 2048, 2049, 7000], 2),           # entries with one row at or below top-k and one above
-    ([2048, 5], 1),                            # no page is scored
+    ([2048, 5, 2047], 1),                      # no page is scored
 ])
 def test_ragged_batches_sample_each_row_by_its_length(cuda, lens, n):
     print(f"ragged fused lens={lens} n={n}", flush=True)
@@ -157,7 +157,7 @@ def test_ragged_batches_sample_each_row_by_its_length(cuda, lens, n):
 ])
 def test_repeated_scores_select_the_lowest_positions(cuda, length, pages, one_score):
     print(f"repeated scores length={length} pages={pages}", flush=True)
-    inp, cl, max_ctx = _inputs([length, 3000], 1, seed=length)
+    inp, cl, max_ctx = _inputs([length, 3000, 70000], 1, seed=length)  # the longest row: lists, not whole rows
     width = inp.block_tables.shape[1]
     inp.block_tables[0] = inp.block_tables[0, torch.arange(width, device="cuda") % pages]
     if one_score:
@@ -176,11 +176,13 @@ def test_repeated_scores_select_the_lowest_positions(cuda, length, pages, one_sc
     ([513, 512, 511, 577, 64], 1, 512),
     ([8193, 700, 513], 2, 512),
     ([100, 7], 1, 2048),                                    # nothing to score
+    ([32768, 32767, 20481, 16385, 9000], 1, 2048),          # 32K contexts: 8 chunks
+    ([65536, 61441], 1, 2048),                              # two rows of 64K: 16 chunks
 ])
 def test_short_contexts_select_whole_rows(cuda, lens, n, k):
     print(f"short fused lens={lens} n={n} k={k}", flush=True)
     inp, cl, max_ctx = _inputs(lens, n, seed=sum(lens) + n + k)
-    assert max_ctx <= 16384
+    assert max_ctx <= 65536
     e_phys, e_logi = _unfused(inp, cl, max_ctx, k, n)
     g_phys, g_logi = _fused(inp, cl, max_ctx, k, n)
     assert np.array_equal(g_logi, e_logi)

@@ -225,3 +225,36 @@ def test_indexer_select_masks_extreme_logits(cuda, width, k, with_ws):
     torch.cuda.synchronize()
     exp = O.indexer_decode_topk(logits, ctx, k)
     assert np.array_equal(out.cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("width", [2049, 4096, 4099, 8193, 16385, 32767, 32772, 65533])
+@pytest.mark.parametrize("top_k", [512, 2048])
+def test_whole_row_select_at_chunk_edges(cuda, width, top_k):
+    """The select that holds a row of up to 64K scores in registers (chunks of
+    4096 positions, one instantiation per power of two of them): lengths on both
+    sides of a chunk, a quad and a storage that ends inside a quad (the last row
+    ends the buffer), scores that spread, tie in one bin (its few and its many
+    elements), all tie, or carry infinities, and two outliers that put every
+    other score into one bin. The positions are exact."""
+    rng = np.random.default_rng(width + top_k)
+    stride = (width + 3) & ~3
+    lens = np.array([width, width - 1, max(width - 4095, top_k + 1), top_k + 1, width, width, width, width], np.int32)
+    B = len(lens)
+    scores = rng.standard_normal((B, width)).astype(np.float32)
+    scores[3] = rng.integers(0, 3, width)
+    scores[4] = -np.inf
+    scores[4, ::7] = np.inf
+    scores[5] = np.where(rng.random(width) < 0.2, scores[5], np.float32(-0.0))
+    scores[6, 17], scores[6, 1000] = 3e38, -3e38
+    scores[7, 17], scores[7, width - 1] = 1e9, np.inf
+    flat = torch.full(((B - 1) * stride + width,), float("nan"), dtype=torch.float32, device=cuda)
+    padded = flat.as_strided((B, width), (stride, 1))
+    padded.copy_(torch.from_numpy(scores))
+    pt = np.stack([rng.permutation((width + 63) // 64) for _ in range(B)]).astype(np.int32)
+    out = torch.empty(B, top_k, dtype=torch.int32, device=cuda)
+    raw = torch.empty_like(out)
+    ops.topk_transform(padded, torch.from_numpy(lens).to(cuda), torch.from_numpy(pt).to(cuda), out, 64, top_k, raw)
+    torch.cuda.synchronize()
+    e_page, e_raw = O.topk_transform(scores, lens, pt, 64, top_k)
+    assert np.array_equal(raw.cpu().numpy(), e_raw)
+    assert np.array_equal(out.cpu().numpy(), e_page)

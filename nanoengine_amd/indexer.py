@@ -94,9 +94,8 @@ def indexer_decode_topk(q_fp8: torch.Tensor, weights: torch.Tensor, kv_cache_buf
     max_context_len = block_tables.shape[-1] * page_size
     ctx = _expand_decode_context_lens(context_lens.to(torch.int32), ntps)
     bt = block_tables.to(torch.int32)
-    if not _uses_linear_mtp_indexer_path(is_prefill=is_prefill, ntps=ntps):
-        if schedule_meta is None:
-            schedule_meta = deep_gemm.get_paged_mqa_logits_metadata(ctx, page_size, None)
+    # schedule_meta is taken as the reference takes it; the logits kernels balance
+    # their pages themselves, so none is built here
     logits = deep_gemm.fp8_paged_mqa_logits(q4, kv_cache, weights, ctx, bt, schedule_meta,
                                             max_context_len, clean_logits=False) \
         if logits_out is None else _logits_into(q4, kv_cache, weights, ctx, bt, max_context_len, logits_out)

@@ -26,7 +26,8 @@
 // Grid: token blocks x key chunks, with the chunk count a multiple of 8 and
 // chunk c placed on XCD c % 8 (workgroups are dealt to the 8 XCDs round
 // robin), so the workgroups sharing a chunk's keys share one L2; a short key
-// set with many query blocks runs as one chunk (each query block read once).
+// set is cut only as far as the CUs need workgroups (each query block is read
+// once per chunk).
 //
 // Filter mode (the fused top-k of prefill_topk.hip): instead of storing the
 // logit, each wave compares the order key of its 64 logits with its row's
@@ -54,6 +55,7 @@ constexpr int kPfStageBytes = kPfStageKeys * 128;       // 16 KB of keys
 constexpr int kPfKeyTiles = kPfStageKeys / 32;
 constexpr int kPfBufs = 3;
 constexpr int kPfHeads = 64;
+constexpr int kPfFewStages = 32;  // 4096 keys, 512 KB
 
 struct PfLds {
   uint8_t key[kPfBufs][kPfStageBytes];
@@ -125,18 +127,16 @@ __global__ void __launch_bounds__(kPfThreads)
 mqa_logits_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__ kv, const float* __restrict__ kv_scale,
                   const float* __restrict__ weights, int64_t w_stride, const int32_t* __restrict__ ks,
                   const int32_t* __restrict__ ke, int M, int64_t n_keys, int token_blocks, int64_t chunk_keys,
-                  float* __restrict__ logits, int64_t logits_stride, PrefillList* __restrict__ ws) {
+                  bool by_block, float* __restrict__ logits, int64_t logits_stride, PrefillList* __restrict__ ws) {
   __shared__ typename std::conditional<kFilter, PfLdsFilter, PfLds>::type lds;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // workgroup -> (token block, chunk): XCD b % 8 takes chunks c with c % 8 == b % 8
-  // (one chunk covers every key: workgroup b takes token block b; any
-  // workgroup past the last token block exits)
+  // workgroup -> (token block, chunk): XCD b % 8 takes chunks c with c % 8 == b % 8;
+  // of few keys (by_block), which every L2 holds, the blocks of a chunk lie together
   const int b = blockIdx.x;
-  const bool one_chunk = chunk_keys >= n_keys;
-  const int r = b >> 3;
-  const int tb = one_chunk ? b : r % token_blocks;
-  const int chunk = one_chunk ? 0 : (r / token_blocks) * 8 + (b & 7);
+  const int r = by_block ? b : b >> 3;
+  const int tb = r % token_blocks;
+  const int chunk = by_block ? r / token_blocks : (r / token_blocks) * 8 + (b & 7);
   const int r0 = tb * kPfTokens;
   // key range of the block's 16 rows, intersected with the chunk
   int lo_i = INT32_MAX, hi_i = INT32_MIN;
@@ -324,9 +324,18 @@ prefill_windows_kernel(const void* __restrict__ cu_q, const void* __restrict__ c
     if (cu(cu_q, 0) != 0 || cu(cu_k, 0) != 0) bits |= 1;
     if (cu(cu_q, num_seqs) != num_queries) bits |= 2;
   }
-  atomicOr(&s_bits, bits);
-  atomicMax(&s_maxk, maxk);
-  atomicMax(&s_maxp, maxp);
+  // one atomic per wave (256 lanes on one word serialise)
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    bits |= __shfl_xor(bits, off, 64);
+    maxk = max(maxk, (unsigned long long)__shfl_xor(maxk, off, 64));
+    maxp = max(maxp, (unsigned long long)__shfl_xor(maxp, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicOr(&s_bits, bits);
+    atomicMax(&s_maxk, maxk);
+    atomicMax(&s_maxp, maxp);
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     status[0] = (int64_t)s_bits;
@@ -344,10 +353,23 @@ int launch_mqa_logits(bool filter, const uint8_t* q, const uint8_t* kv, const fl
                       float* logits, int64_t logits_stride, PrefillList* ws, hipStream_t st) {
   const int token_blocks = (num_rows + kPfTokens - 1) / kPfTokens;
   int64_t chunks, chunk_keys;
-  if (token_blocks >= 512 && num_keys <= 32 * kPfStageKeys) {
-    // few keys, many rows: one chunk, so that each query block is read once
-    chunks = 1;
-    chunk_keys = std::max<int64_t>(num_keys, 1);
+  const int64_t stages = (num_keys + kPfStageKeys - 1) / kPfStageKeys;
+  const bool by_block = stages <= kPfFewStages;
+  if (by_block) {
+    // few keys: loading its query block costs a workgroup about one stage, so
+    // the chunks that take the least rounds of the CUs times (stages + 1), not
+    // always eight (the sampled scores of 2045 rows over 642 keys: 39.5 us in
+    // 8 chunks, 18.0 in 2)
+    int64_t best = INT64_MAX, per = 1;
+    for (int64_t p = 1; p <= std::max<int64_t>(stages, 1); ++p) {
+      const int64_t rounds = (token_blocks * ((stages + p - 1) / p) + 255) / 256;
+      if (rounds * (p + 1) <= best) {
+        best = rounds * (p + 1);
+        per = p;
+      }
+    }
+    chunks = std::max<int64_t>(1, (stages + per - 1) / per);
+    chunk_keys = per * kPfStageKeys;
   } else {
     // chunks: a multiple of 8 (one XCD each), enough workgroups for the 256 CUs
     chunks = 8;
@@ -359,12 +381,12 @@ int launch_mqa_logits(bool filter, const uint8_t* q, const uint8_t* kv, const fl
   if (grid > INT32_MAX) return set_error(kInvalidArgument, "mqa logits: grid too large");
   if (filter)
     hipLaunchKernelGGL(mqa_logits_kernel<true>, dim3((unsigned)grid), dim3(kPfThreads), 0, st, q, kv, kv_scale,
-                       weights, weights_stride, ks, ke, num_rows, num_keys, token_blocks, chunk_keys, logits,
-                       logits_stride, ws);
+                       weights, weights_stride, ks, ke, num_rows, num_keys, token_blocks, chunk_keys, by_block,
+                       logits, logits_stride, ws);
   else
     hipLaunchKernelGGL(mqa_logits_kernel<false>, dim3((unsigned)grid), dim3(kPfThreads), 0, st, q, kv, kv_scale,
-                       weights, weights_stride, ks, ke, num_rows, num_keys, token_blocks, chunk_keys, logits,
-                       logits_stride, ws);
+                       weights, weights_stride, ks, ke, num_rows, num_keys, token_blocks, chunk_keys, by_block,
+                       logits, logits_stride, ws);
   return check_launch(filter ? "mqa logits (filter)" : "dsa_mqa_logits");
 }
 

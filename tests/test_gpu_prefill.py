@@ -135,3 +135,35 @@ def test_mqa_logits_within_the_derived_mfma_bound(cuda):
     print(rep, flush=True)
     assert rep["over_rtol"] > 0, rep
     assert rep["ok"], rep
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (1, 4096), (17, 128), (100, 129), (2040, 642), (4096, 257), (4100, 384),
+                                 (700, 4096), (700, 4097)])
+def test_mqa_logits_few_keys_in_any_chunks(cuda, M, N):
+    """Up to 4096 keys are cut into as many chunks as the CUs need, from one
+    per key stage to one in all: every logit of every window is there once, the
+    ones of sampled rows within the oracle's bound, and equal to the logits of
+    the same keys in a longer key set (cut into eight)."""
+    print(f"mqa_logits few keys M={M} N={N}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(M + N)
+    longer = 4300
+    q = (torch.randn(M, 64, 128, generator=g, device=cuda) * 40).to(torch.float8_e4m3fn)
+    kv = (torch.randn(longer, 128, generator=g, device=cuda) * 40).to(torch.float8_e4m3fn)
+    sc = torch.rand(longer, generator=g, device=cuda) * 9e-3 + 1e-3
+    w = torch.randn(M, 64, generator=g, device=cuda) * 1e-4
+    ks = torch.randint(0, max(N // 3, 1), (M,), generator=g, device=cuda, dtype=torch.int32)
+    ke = torch.clamp(ks + torch.randint(0, N + 1, (M,), generator=g, device=cuda, dtype=torch.int32), max=N)
+    ke[0] = N
+    got = torch.full((M, N), float("nan"), device=cuda)
+    ops.mqa_logits(q, kv[:N], sc[:N].contiguous(), w, ks, ke, got, False)
+    other = torch.full((M, longer), float("nan"), device=cuda)
+    ops.mqa_logits(q, kv, sc, w, ks, ke, other, False)
+    cols = torch.arange(N, device=cuda)
+    inside = (cols >= ks[:, None]) & (cols < ke[:, None])
+    assert torch.equal(torch.isnan(got), ~inside)
+    assert torch.equal(got[inside], other[:, :N][inside])
+    rows = sorted({0, M // 2, M - 1})
+    host = lambda t: t[rows].cpu().numpy()
+    exp = O.mqa_logits(host(q.view(torch.uint8)), kv[:N].view(torch.uint8).cpu().numpy(), sc[:N].cpu().numpy(), host(w),
+                       host(ks), host(ke), clean_logits=True)
+    _check_windows(host(got), exp, host(ks), host(ke))

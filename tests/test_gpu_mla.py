@@ -316,3 +316,22 @@ def test_chosen_splits_match_the_unsplit_kernel(cuda, T, H, K):
     fin = torch.isfinite(lse1)
     assert torch.equal(torch.isfinite(lse), fin)
     assert torch.all((lse[fin] - lse1[fin]).abs() <= 1e-5)
+
+
+@pytest.mark.parametrize("splits,K", [(2, 2048), (8, 2048), (16, 2048), (64, 8192), (128, 8192)])
+def test_combine_takes_any_number_of_splits(cuda, splits, K):
+    """The combine reads eight splits at a time and one LSE per lane: one
+    group, several, and more splits than lanes, some of them without a valid
+    key. Bounds as for the chosen splits above."""
+    T, H = 2, 128
+    q, kv, idx = _case(T, H, K, num_blocks=160, seed=splits + K)
+    idx = idx.clone()
+    idx[:, K // 2:] = -1          # the later splits hold no key
+    idx[1, :] = -1                # nor does any split of token 1
+    o, lse = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5, num_splits=splits)
+    o1, lse1 = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5, num_splits=1)
+    torch.cuda.synchronize()
+    a, b = o.float(), o1.float()
+    assert torch.all((a - b).abs() <= 2.0 ** -8 * (torch.maximum(a.abs(), b.abs()) + 1.0))
+    assert torch.all((lse[0] - lse1[0]).abs() <= 1e-5)
+    assert (o[1] == 0).all() and torch.equal(lse[1], lse1[1])

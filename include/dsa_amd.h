@@ -92,14 +92,19 @@ DSA_API size_t dsa_indexer_topk_workspace_bytes(int batch, int next_n, int64_t m
  * must translate with dsa_topk_to_physical instead.
  * Selection, order (ascending position), ties (lowest positions) and padding are
  * those of dsa_topk_transform over dsa_indexer_logits' logits, exactly.
- * Launch sequence on `stream`: logits of 16 sampled pages per row -> per-row
- * score threshold -> all pages, keeping only (key, position) of tokens at or
- * above the threshold in per-row lists -> exact top-k of each list; a row whose
- * list is unusable (fewer than top_k or more than the list capacity) is redone
- * inside that last launch, by the row's workgroup, from the row's full logits.
+ * Launch sequence on `stream`: logits of up to 16 pages sampled over each row's
+ * own length -> per-row score threshold -> all pages, keeping only (key,
+ * position) of tokens at or above the threshold in per-row lists of 16384 ->
+ * exact top-k of each list; a row whose list is unusable (fewer than top_k or
+ * more than the list capacity) is redone inside that last launch, by the row's
+ * workgroup, from the row's full logits. Short contexts and small batches
+ * (max_context_len <= 8192; <= 32768 with at most 3M tokens in rows *
+ * max_context_len; <= 65536 with at most two rows) take two launches: every
+ * score into the workspace, then the exact top-k of whole rows.
  * phase_events: NULL, or five hipEvent_t (entries may be NULL) recorded on
  * `stream` before the first launch and after the sample, filter and select
- * phases (the last two entries both after the select), for timing.
+ * phases (the last two entries both after the select; where whole rows are
+ * selected, the second and third both after the scores), for timing.
  * top_k in {512, 2048}; rows of at most dsa_topk_max_len() positions. The
  * workspace (dsa_indexer_topk_workspace_bytes) should be zero-filled before its
  * first use; a stale one gives the same results, its first call more slowly.
@@ -205,7 +210,10 @@ DSA_API int dsa_topk_to_physical(const int32_t* topk_indices, int64_t topk_strid
                          int table_width, int rows, int topk, int rows_per_table,
                          int block_size, int32_t* out, void* stream);
 
-/* Split count the sparse MLA decode uses for this shape (1 = no workspace). */
+/* Split count the sparse MLA decode uses for this shape (1 = no workspace):
+ * of the (token, 64-head group) items, those that fill the CUs in whole rounds
+ * run unsplit, and each of the rest splits its keys this many ways (at most 8,
+ * at least four 64-key blocks each, block counts that differ by at most one). */
 DSA_API int dsa_sparse_mla_num_splits(int num_tokens, int num_heads, int topk, int num_cus);
 
 /* Workspace bytes dsa_sparse_mla_decode needs for `num_splits`. */
@@ -230,7 +238,9 @@ DSA_API size_t dsa_sparse_mla_workspace_bytes(int num_tokens, int num_heads, int
  * no valid index yields o = 0 and lse = -inf.
  * num_heads % 16 == 0; topk % 64 == 0; num_splits in [1, topk/64] with
  * workspace >= dsa_sparse_mla_workspace_bytes(...) when num_splits > 1
- * (num_splits <= 0 picks dsa_sparse_mla_num_splits for this device).
+ * (num_splits <= 0 picks dsa_sparse_mla_num_splits for this device). The
+ * rule's own count splits as described there; any other must cut topk into
+ * equal splits of whole 64-key blocks, and applies to every item.
  * Replaces flash_mla.flash_mla_with_kvcache(q, k_cache, None, None,
  * head_dim_v=512, sched_meta, None, softmax_scale, causal=False,
  * is_fp8_kvcache=True, indices=...) as called by FlashMlaAttention.forward

@@ -17,11 +17,12 @@
 // pages in flight while one is multiplied. The page primitives live in
 // indexer_page.h.
 //
-// Launches: indexer_logits_kernel (one workgroup per 24 pages of a row) writes
-// the logits (the fp8_paged_mqa_logits operator), samples pages of each row for
-// the fused path's score threshold, or filters (batches above the persistent
-// kernel's limit); indexer_filter_kernel is the fused path's persistent filter
-// pass (one contiguous page range per wave, per-wave candidate staging).
+// Launches: indexer_logits_kernel (one workgroup per 24 pages of a row) samples
+// pages of each row for the fused path's score threshold, writes the logits of
+// large batches (the fp8_paged_mqa_logits operator), or filters (batches above
+// the persistent kernel's limit); indexer_filter_kernel is the persistent pass
+// (one contiguous page range per wave): the fused path's filter (per-wave
+// candidate staging), and the scores kept for small batches and short contexts.
 #include <algorithm>
 #include <type_traits>
 

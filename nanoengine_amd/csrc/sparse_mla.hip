@@ -40,15 +40,19 @@
 //            indices into a 64-entry row-address table in LDS, so a load costs
 //            a table read and an add. Invalid indices read a zero row.
 // One barrier per block: P, the references and the next block's rows change
-// hands there; no score, maximum or sum is exchanged inside a block.
+// hands there; over cache slots no score, maximum or sum is exchanged inside a
+// block.
 // Chunked prefill: after a token's cache-slot blocks come blocks of 32 fresh
 // bf16 rows [576] (the chunk's own keys, not yet in the cache). They go to LDS
 // the same way; the key half 0 QK waves read them as bf16 operands, and the
 // PV waves read V with ds_read_b64_tr_b16 (no tile scale), so cached and
 // fresh keys share one softmax.
-// Splits over the key list (for small batches) write normalised partial
-// outputs and LSEs to a caller-provided workspace; a combine kernel merges
-// them with the LSE rule of merge_attention_states.
+// bf16 rows only (kRows, a prefill over assembled keys): blocks of 32 rows; the
+// QK waves split the dims instead of the keys and exchange half of their
+// partial scores in the middle of an iteration.
+// Splits over the key list (the items of the last, partial round of the CUs)
+// write normalised partial outputs and LSEs to a caller-provided workspace; a
+// combine kernel merges them with the LSE rule of merge_attention_states.
 #include <algorithm>
 #include <cmath>
 

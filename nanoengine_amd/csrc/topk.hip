@@ -766,7 +766,7 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 // What bounds it: a chain of short phases in one CU (loads, extremes, LDS
 // histogram, threshold, ranks, compaction). A 1/8 sample's threshold, the
 // candidates above it listed and three radix levels over the list took
-// 35.5 us for 33 rows of 3K to 40K where this takes 16.4; 64 rows of 16K take 8.7.
+// 35.5 us for 33 rows of 3K to 40K where this takes 16.4; four rows of 4K take 6.9.
 // Instantiated per power of two of the row's chunks: a kernel for longer rows
 // spends its registers and tests on chunks that a short one does not have.
 constexpr int kRowThreads = 1024;

@@ -66,6 +66,24 @@ struct ScoreBins {
   __device__ __forceinline__ uint32_t of(uint32_t key) const { return bin(key_to_float(key)); }
 };
 
+// 4096 bins linear in the bits of the scores from `lowest` > 0 to `highest`
+// (positive floats order as their bits); lower scores share bin 0, higher ones
+// the last.
+struct BitBins {
+  float lo;
+  uint32_t base;
+  int shift;
+  __device__ __forceinline__ BitBins(float lowest, float highest) {
+    const float top = fmaxf(highest, lowest);
+    lo = lowest;
+    base = __float_as_uint(lowest);
+    shift = max(0, 32 - (int)__clz((int)(__float_as_uint(top) - base)) - 12);
+  }
+  __device__ __forceinline__ uint32_t bin(float score) const {
+    return score < lo ? 0u : min((__float_as_uint(score) - base) >> shift, (uint32_t)(kHistBins - 1));
+  }
+};
+
 // The 12-bit digits, from the top, of the composites of keys in [kmin, kmax]:
 // the key part counts from kmin, so the digits spread over the keys' own range.
 struct CompositeDigits {

@@ -758,7 +758,7 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 // ---------------------------------------------------------------- row select
 // Exact top-k of a row of up to 64K scores by one workgroup, which reads the
 // row once: thread t holds positions [4t, 4t + 4) of every chunk of 4096 in
-// registers. First digit: the score's linear bin, counted over the whole row;
+// registers. First digit: the score's bin (linear in its bits or in the score),
 // the threshold bin's few elements count those ahead of them, or, where many
 // scores tie, take radix levels. The selected positions are a bitmap in LDS,
 // compacted in position order by one block scan.
@@ -766,7 +766,9 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 // What bounds it: a chain of short phases in one CU (loads, extremes, LDS
 // histogram, threshold, ranks, compaction). A 1/8 sample's threshold, the
 // candidates above it listed and three radix levels over the list took
-// 35.5 us for 33 rows of 3K to 40K where this takes 16.4; four rows of 4K take 6.9.
+// 30 us a call for 33 rows of 40000 scores where this takes 19.7, for normal
+// scores as for ones with an outlier or a long tail. (Bins linear in the score
+// alone: 17.4 for normal scores, but 91 with one outlier of 1e9.)
 // Instantiated per power of two of the row's chunks: a kernel for longer rows
 // spends its registers and tests on chunks that a short one does not have.
 constexpr int kRowThreads = 1024;
@@ -778,6 +780,7 @@ struct RowSelectSmem {
   uint64_t rank[kRankCap];
   uint32_t bits[kRowSelectLen / 32];
   uint32_t wave_sum[2 * (kRowThreads / 64)];
+  float floors[kRowThreads / 64];
   uint32_t count, tb, above, eq;
 };
 
@@ -833,6 +836,7 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
     return p + e < len && fabsf(v) <= cap ? v : -inf;
   };
   float lo = inf, hi = -inf;  // the extremes; lo of the scores above -inf
+  float second = -inf;        // this thread's second highest
 #pragma unroll
   for (int c = 0; c < kChunks; ++c)
     if (c < nch) {
@@ -841,37 +845,57 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
         float& v = x[4 * c + e];
         v = score(kRowChunk * c + 4 * tid, e, v);
         lo = fminf(lo, v > -inf ? v : inf);
+        second = fmaxf(second, fminf(hi, v));
         hi = fmaxf(hi, v);
       }
     }
+  auto block_extremes = [&](float& low, float& high) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    lo = fminf(lo, __shfl_xor(lo, off, 64));
-    hi = fmaxf(hi, __shfl_xor(hi, off, 64));
-  }
-  float* wave_f = reinterpret_cast<float*>(s.wave_sum);
-  if (lane == 0) {
-    wave_f[wave] = lo;
-    wave_f[NW + wave] = hi;
-  }
-  __syncthreads();
+    for (int off = 32; off >= 1; off >>= 1) {
+      low = fminf(low, __shfl_xor(low, off, 64));
+      high = fmaxf(high, __shfl_xor(high, off, 64));
+    }
+    float* wave_f = reinterpret_cast<float*>(s.wave_sum);
+    if (lane == 0) {
+      wave_f[wave] = low;
+      wave_f[NW + wave] = high;
+    }
+    __syncthreads();
 #pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    lo = fminf(lo, wave_f[i]);
-    hi = fmaxf(hi, wave_f[NW + i]);
-  }
-  // infinities fall into the end bins and do not widen the range
-  const ScoreBins bins(lo, fminf(hi, 3.4028235e38f));
+    for (int i = 0; i < NW; ++i) {
+      low = fminf(low, wave_f[i]);
+      high = fmaxf(high, wave_f[NW + i]);
+    }
+  };
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) second = fminf(second, __shfl_xor(second, off, 64));
+  if (lane == 0) s.floors[wave] = second;
+  block_extremes(lo, hi);
+#pragma unroll
+  for (int i = 0; i < NW; ++i) second = fminf(second, s.floors[i]);
+  uint32_t remain = (uint32_t)top_k;
+  auto decide = [&](const auto bins) {
 
-  // ---- first digit
+  // ---- first digit. Scores with a long tail (or many at the lowest value)
+  // fill bin 0: it is counted in registers, where one LDS word would serialise.
+  auto add_lowest = [&](uint32_t n) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) n += (uint32_t)__shfl_xor(n, off, 64);
+    if (lane == 0 && n) atomicAdd(&s.hist[0], n);
+  };
+  uint32_t lowest = 0;
 #pragma unroll
   for (int c = 0; c < kChunks; ++c)
     if (c < nch && kRowChunk * c + 4 * tid < len) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) atomicAdd(&s.hist[bins.bin(x[4 * c + e])], 1u);
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t d = bins.bin(x[4 * c + e]);
+        if (d) atomicAdd(&s.hist[d], 1u);
+        else ++lowest;
+      }
     }
+  add_lowest(lowest);
   __syncthreads();
-  uint32_t remain = (uint32_t)top_k;
   find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
   const uint32_t tb = s.tb, eq = s.eq;
   remain -= s.above;
@@ -897,35 +921,75 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
       if ((lane & 7) == 0) s.bits[p >> 5] = word;
     }
   __syncthreads();
-  if (ranked) {
-    if ((uint32_t)tid < eq) {
+  // the threshold bin's n listed elements: those with fewer than `room` ahead of them
+  auto rank_listed = [&](uint32_t n, uint32_t room) {
+    if ((uint32_t)tid < n) {
       const uint64_t mine = s.rank[tid];
       uint32_t ahead = 0;
-      for (uint32_t e = 0; e < eq; ++e) ahead += s.rank[e] > mine ? 1u : 0u;
+      for (uint32_t e = 0; e < n; ++e) ahead += s.rank[e] > mine ? 1u : 0u;
       const uint32_t pos = kIdxMax - (uint32_t)(mine & kIdxMax);
-      if (ahead < remain) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
+      if (ahead < room) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
     }
+  };
+  if (ranked) {
+    rank_listed(eq, remain);
   } else if (!whole_bin) {
-    // Radix levels over the threshold bin's elements, from their own keys'
-    // range. The row is read again (its second look hits L2), so that this
-    // rare path costs the others no registers.
+    // Too many elements for that: the bin's own range in 4096 bins again
+    // (outliers and long tails leave most scores in one bin), and, where they
+    // tie, radix levels. The row is read again (from L2, four chunks in flight),
+    // so that these paths cost the usual one no registers.
     auto each = [&](auto&& visit) {
 #pragma unroll 1
-      for (int c = 0; c < nch; ++c) {
-        const int p = kRowChunk * c + 4 * tid;
-        if (p >= len) continue;
-        const v4f v = *reinterpret_cast<const v4f*>(row + min(p, last));
+      for (int c0 = 0; c0 < nch; c0 += 4) {
+        v4f v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float y = score(p, e, v[e]);
-          if (bins.bin(y) == tb) visit(order_key(y), (uint32_t)(p + e));
+        for (int u = 0; u < 4; ++u)
+          if (c0 + u < nch) v[u] = *reinterpret_cast<const v4f*>(row + min(kRowChunk * (c0 + u) + 4 * tid, last));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int p = kRowChunk * (c0 + u) + 4 * tid;
+          if (p >= len) continue;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float y = score(p, e, v[u][e]);
+            if (bins.bin(y) == tb) visit(y, (uint32_t)(p + e));
+          }
         }
       }
     };
+    float zlo = inf, zhi = -inf;
+    each([&](float y, uint32_t) {
+      zlo = fminf(zlo, y > -inf ? y : inf);
+      zhi = fmaxf(zhi, y);
+    });
+    block_extremes(zlo, zhi);
+    const ScoreBins zoom(zlo, fminf(zhi, 3.4028235e38f));
+    for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
+    __syncthreads();
+    lowest = 0;
+    each([&](float y, uint32_t) {
+      const uint32_t d = zoom.bin(y);
+      if (d) atomicAdd(&s.hist[d], 1u);
+      else ++lowest;
+    });
+    add_lowest(lowest);
+    __syncthreads();
+    find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
+    const uint32_t tb2 = s.tb, eq2 = s.eq, room = remain - s.above;
+    const bool whole2 = eq2 == room;
+    if (whole2 || eq2 <= (uint32_t)kRankCap) {
+      each([&](float y, uint32_t pos) {
+        const uint32_t d = zoom.bin(y);
+        if (d > tb2 || (whole2 && d == tb2)) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
+        else if (d == tb2) s.rank[atomicAdd(&s.count, 1u)] = rank_composite(order_key(y), pos);
+      });
+      __syncthreads();
+      if (!whole2) rank_listed(eq2, room);
+    } else {
     uint32_t kmin = 0xffffffffu, kmax = 0u;
-    each([&](uint32_t key, uint32_t) {
-      kmin = min(kmin, key);
-      kmax = max(kmax, key);
+    each([&](float y, uint32_t) {
+      kmin = min(kmin, order_key(y));
+      kmax = max(kmax, order_key(y));
     });
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -948,7 +1012,8 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
       __syncthreads();  // every thread has read the previous level's outcome
       for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
       __syncthreads();
-      each([&](uint32_t key, uint32_t pos) {
+      each([&](float y, uint32_t pos) {
+        const uint32_t key = order_key(y);
         if (digits.above(key, pos, L) == prefix) atomicAdd(&s.hist[digits.of(key, pos, L)], 1u);
       });
       __syncthreads();
@@ -956,15 +1021,25 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
       const uint32_t t = s.tb;
       remain -= s.above;
       const bool done = s.eq == remain || L == digits.levels - 1;
-      each([&](uint32_t key, uint32_t pos) {
-        const uint32_t d = digits.of(key, pos, L);
+      each([&](float y, uint32_t pos) {
+        const uint32_t key = order_key(y), d = digits.of(key, pos, L);
         if (digits.above(key, pos, L) == prefix && (d > t || (done && d == t)))
           atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
       });
       if (done) break;
       prefix = prefix * (uint32_t)digits.bins(L) + t;
     }
+    }
   }
+  };
+  // The 2 x 1024 scores that are some thread's highest two are at least `second`,
+  // so that the top-k (at most 2048) is: above it the bins are linear in the
+  // float's bits (outliers and long tails then cost a few octaves of bins, not
+  // the range), unless it is negative (rows of a few scores per thread), where
+  // that would spend the bins around zero. Infinities fall into the end bins.
+  const float top = fminf(hi, 3.4028235e38f);
+  if (second > 0.f) decide(BitBins(second, top));
+  else decide(ScoreBins(lo, top));
   __syncthreads();
 
   // ---- positions in ascending order (thread t: `per` of them, a power of two,

@@ -238,7 +238,7 @@ def test_whole_row_select_at_chunk_edges(cuda, width, top_k):
     other score into one bin. The positions are exact."""
     rng = np.random.default_rng(width + top_k)
     stride = (width + 3) & ~3
-    lens = np.array([width, width - 1, max(width - 4095, top_k + 1), top_k + 1, width, width, width, width], np.int32)
+    lens = np.array([width, width - 1, max(width - 4095, top_k + 1), top_k + 1] + [width] * 7, np.int32)
     B = len(lens)
     scores = rng.standard_normal((B, width)).astype(np.float32)
     scores[3] = rng.integers(0, 3, width)
@@ -247,6 +247,10 @@ def test_whole_row_select_at_chunk_edges(cuda, width, top_k):
     scores[5] = np.where(rng.random(width) < 0.2, scores[5], np.float32(-0.0))
     scores[6, 17], scores[6, 1000] = 3e38, -3e38
     scores[7, 17], scores[7, width - 1] = 1e9, np.inf
+    scores[8] = np.exp(4 * scores[8])                       # a long tail: the bin's own range is binned again
+    scores[9, width - 1] = 1e9
+    scores[10] = np.where(rng.random(width) < 0.5, scores[10], np.float32(-0.5))
+    scores[10, 5] = 1e6
     flat = torch.full(((B - 1) * stride + width,), float("nan"), dtype=torch.float32, device=cuda)
     padded = flat.as_strided((B, width), (stride, 1))
     padded.copy_(torch.from_numpy(scores))

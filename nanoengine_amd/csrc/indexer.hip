@@ -756,7 +756,8 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
   // Indexer us, lists against whole rows: 4 x 4K 24.5 / 15.3, 64 x 16K 49.7 /
   // 39.4, 1024 x 8K 284 / 256, 200 x 16K 77 / 67 but 250 x 16K 116 / 120;
   // 8 x 32K 32.9 / 24.3, 64 x 32K 71.2 / 67.6 but 128 x 32K 116 / 122; 1 x 64K
-  // 36.1 / 28.7, 8 x 64K 39.8 / 40.0, 32 x 64K 71 / 76.
+  // 36.1 / 28.7, 8 x 64K 39.8 / 40.0, 32 x 64K 71 / 76. (The row select has
+  // since become 1 to 2 us slower, for scores that crowd linear bins.)
   if (max_context_len <= 8192 || (max_context_len <= 32768 && rows * max_context_len <= kScoreTokens) ||
       (max_context_len <= kRowSelectLen && rows <= 2)) {
     if (launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,

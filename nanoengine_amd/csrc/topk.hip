@@ -759,8 +759,8 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 // Exact top-k of a row of up to 64K scores by one workgroup, which reads the
 // row once: thread t holds positions [4t, 4t + 4) of every chunk of 4096 in
 // registers. First digit: the score's bin (linear in its bits or in the score),
-// the threshold bin's few elements count those ahead of them, or, where many
-// scores tie, take radix levels. The selected positions are a bitmap in LDS,
+// counted over the whole row; the threshold bin's few elements count those ahead
+// of them, a crowded bin is binned again, and ties take radix levels. The selected positions are a bitmap in LDS,
 // compacted in position order by one block scan.
 //
 // What bounds it: a chain of short phases in one CU (loads, extremes, LDS

@@ -48,8 +48,9 @@
 // PV waves read V with ds_read_b64_tr_b16 (no tile scale), so cached and
 // fresh keys share one softmax.
 // bf16 rows only (kRows, a prefill over assembled keys): blocks of 32 rows; the
-// QK waves split the dims instead of the keys and exchange half of their
-// partial scores in the middle of an iteration.
+// QK waves split the dims instead of the keys and exchange their partial scores
+// in the middle of an iteration. Every key of a block shares one reference, the
+// largest score when it last moved, so P needs no exponent adds.
 // Splits over the key list (the items of the last, partial round of the CUs)
 // write normalised partial outputs and LSEs to a caller-provided workspace; a
 // combine kernel merges them with the LSE rule of merge_attention_states.
@@ -92,6 +93,16 @@ constexpr int kRingOff = kFinOff + 3 * 128 * 4;        // row indices, one 64-en
 constexpr int kRingSlots = 5;
 constexpr int kAddrOff = kRingOff + kRingSlots * 256;  // row addresses of blocks being gathered, [2][64] u64
 constexpr size_t kMlaSmemBytes = kAddrOff + 2 * kMlaKeys * 8;
+// bf16 rows only: row buffers of one block of bf16 rows, the QK waves' partial
+// scores behind them (four waves of 32 f32 a lane, over what are the P and
+// exponent tables of the other kinds), P past the rest: [2][2 hp][2 k-steps]
+// [64 lanes][8 bf16]. References: [2][2 hp][32]; final sums: [2 hp][4][32], then
+// the maxima [2 hp][32].
+constexpr int kRowsBufBytes = kFreshKeys * kFreshRowBytes;  // 36864
+constexpr int kRowsXOff = kNumBufs * kRowsBufBytes;
+constexpr int kRowsPOff = (int)kMlaSmemBytes;
+constexpr size_t kRowsSmemBytes = kMlaSmemBytes + 2 * 2 * 2 * 64 * 16;
+static_assert(kRowsXOff + 4 * 8192 <= kRefOff && kRowsPOff % 16 == 0, "the partial scores end before the references");
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kRescaleThreshold = 8.0f;  // log2 units
@@ -107,6 +118,8 @@ constexpr int kDropExp = -30;
 // The keys of an instantiation: cache slots (decode), cache slots then bf16
 // rows (paged prefill), bf16 rows only (prefill over assembled keys).
 enum KeyKind : int { kSlots = 0, kSlotsThenRows = 1, kRows = 2 };
+template <int kKeys>
+constexpr int buf_bytes() { return kKeys == kRows ? kRowsBufBytes : kBufBytes; }
 constexpr int kIdxWave = 3;                // the wave that fetches the row indices (a QK wave)
 
 // Output staging of a PV wave: 32 heads x 128 dims, rows 16 bytes apart from a
@@ -115,7 +128,8 @@ constexpr int kStageRow16 = 128 * 2 + 16, kStageRow32 = 128 * 4 + 16;
 constexpr int kStageOut = 32 * kStageRow32;
 static_assert(4 * kStageOut <= kEOff, "the output staging lies in the row and P buffers");
 static_assert(kBufBytes % 1024 == 0, "a block of rows must be whole wave-wide loads");
-static_assert(kMlaSmemBytes <= 160 * 1024, "LDS budget");
+static_assert(kMlaSmemBytes <= 160 * 1024 && kRowsSmemBytes <= 160 * 1024, "LDS budget");
+static_assert(4 * kStageOut <= kRowsXOff, "the output staging lies in the row buffers");
 
 // Source of the pieces of an invalid row (cache or fresh): zero bytes.
 __device__ __align__(16) uint8_t g_mla_zero_row[kFreshRowBytes];
@@ -229,7 +243,7 @@ constexpr int kTabWave = 2;  // the wave that builds the row-address table (a QK
 constexpr int kQRowBytes = 576 * 2;
 constexpr int kQPieces = kQRowBytes / 16;                          // 72
 constexpr int kQDma = kMlaHeadsPerWG * kQRowBytes / 1024;          // 72 wave-wide copies
-static_assert(kMlaHeadsPerWG * kQRowBytes <= 2 * kBufBytes, "the query fits two row buffers");
+static_assert(kMlaHeadsPerWG * kQRowBytes <= 2 * kRowsBufBytes, "the query fits two row buffers of either size");
 static_assert(kQDma % kMlaWaves == 0 && kQPieces % 8 == 0, "query copies per wave, swizzle groups");
 
 // Wave-uniform state of one workgroup's loop. Blocks [0, ncached) are 64 cache
@@ -383,7 +397,7 @@ __device__ __forceinline__ void iteration_start(const MlaParams& P, uint8_t* sme
                                                 const DmaLanes& dl, int t) {
   if (c.wave == kIdxWave && t + 4 < c.nblk) issue_index<kKeys>(P, smem, c, t + 4);
   if (t + 1 < c.nblk) {
-    uint8_t* buf = smem + ((t + 1) % kNumBufs) * kBufBytes;
+    uint8_t* buf = smem + ((t + 1) % kNumBufs) * buf_bytes<kKeys>();
     if (!rows_block<kKeys>(c, t + 1)) issue_block(smem, t + 1, dl, buf, c.wave);
     else issue_fresh_block(smem, t + 1, buf, c.wave, c.lane);
   }
@@ -403,7 +417,9 @@ __device__ __forceinline__ void prologue_end() {
 }
 
 // This wave's share of the query copies: lane l of copy i fills slot
-// 64 i + l of the staged rows. Heads past H repeat the first one.
+// 64 i + l of the staged rows. Heads past H repeat the first one (bf16 rows
+// only: are zeros), and are not written out.
+template <int kKeys>
 __device__ __forceinline__ void issue_query(const MlaParams& P, uint8_t* smem, const MlaCtx& c, int head0) {
   const uint16_t* q = P.q + (int64_t)c.t_tok * P.q_tok_stride;
 #pragma unroll
@@ -412,8 +428,10 @@ __device__ __forceinline__ void issue_query(const MlaParams& P, uint8_t* smem, c
     const int slot = 64 * n + c.lane;
     const int r = slot / kQPieces;
     const int piece = (slot - r * kQPieces) ^ (r & 7);
-    const int head = head0 + r < P.H ? head0 + r : 0;
-    dma16(q + (int64_t)head * P.q_head_stride + 8 * piece, lds_addr(smem + kBufBytes + 1024 * n));
+    const bool ok = head0 + r < P.H;
+    const uint16_t* src = q + (int64_t)(ok ? head0 + r : 0) * P.q_head_stride;
+    if (kKeys == kRows && !ok) src = reinterpret_cast<const uint16_t*>(g_mla_zero_row);
+    dma16(src + 8 * piece, lds_addr(smem + buf_bytes<kKeys>() + 1024 * n));
   }
 }
 
@@ -606,60 +624,71 @@ __device__ __forceinline__ void qk_waves(const MlaParams& P, uint8_t* smem, cons
 
 // QK waves over bf16 rows only (kRows): a block has 32 keys, so the four waves
 // split the dims instead of the keys. Wave (hp, dh = c.kh) forms the partial
-// S^T[32 keys x 32 heads] over its half of the dims (18 MFMAs), sends the
-// partner the partial sums of the partner's 16 keys through the P slots of
-// k-steps 2 and 3 (unused here), and after a barrier finishes the scores and P
-// of its own, k-step dh. (With the keys split as for cache slots, two of the
-// four waves idled and the other two set the block time: 607 -> 484 us; the
-// dims split: 484 -> 395 us, 512 tokens.)
+// S^T[32 keys x 32 heads] over quarters 2dh and 2dh + 1 of the dims (a quarter:
+// 128 nope and 16 rope dims, 9 MFMAs), exchanges both with its partner through
+// LDS, and after a barrier adds the four quarters of every score: both waves
+// hold them all, so that neither waits for the other's maximum, and P of the 16
+// keys of k-step dh is this wave's. The sum of a score of key group g (8 keys)
+// starts at quarter g and goes round; the reference is the block's true largest
+// score when it moves, for all 32 keys, so that a row whose weight lies on one
+// key gives that key's P as exactly 1 (a reference per k-step, rounded up to an
+// integer, rounds that P too: 391 us, but a relative error of 1.4e-3 for a row
+// of one key). (512 tokens of 128 heads over 15000 rows: with the keys split as
+// for cache slots, two of the four waves idled and the other two set the block
+// time, 484 us; every wave doing both phases, 607; this, 411.)
 template <int kTiles>
 __device__ __forceinline__ void qk_waves_rows(const MlaParams& P, uint8_t* smem, const MlaCtx& c, const DmaLanes& dl) {
   const int lane = c.lane, h = c.h, c32 = c.c32, hp = c.hp, dh = c.kh;
-  // the query over this wave's dims: nope chunks 4dh + k, rope k-steps 2dh + i
-  v4i qn[4][4];
+  // the query over this wave's quarters: nope k-step ks of quarter q is dims
+  // 128q + 16ks + 8h .. +7, its rope k-step dims 512 + 16q + 8h .. +7
+  v4i qn[2][8];
   v4i qr[2];
   {
     const int r = 32 * hp + c32;
-    const uint8_t* qrow = smem + kBufBytes + r * kQRowBytes;
+    const uint8_t* qrow = smem + kRowsBufBytes + r * kQRowBytes;
     const int sw = 16 * (r & 7);
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int i = 0; i < 2; ++i) {
+      const int q = 2 * dh + i;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        qn[k][j] = *reinterpret_cast<const v4i*>(qrow + ((16 * (8 * (4 * dh + k) + 4 * h + j)) ^ sw));
-#pragma unroll
-    for (int i = 0; i < 2; ++i) qr[i] = *reinterpret_cast<const v4i*>(qrow + ((16 * (64 + 2 * (2 * dh + i) + h)) ^ sw));
+      for (int ks = 0; ks < 8; ++ks) qn[i][ks] = *reinterpret_cast<const v4i*>(qrow + ((16 * (16 * q + 2 * ks + h)) ^ sw));
+      qr[i] = *reinterpret_cast<const v4i*>(qrow + ((16 * (64 + 2 * q + h)) ^ sw));
+    }
   }
   prologue_end();
   float* ref = reinterpret_cast<float*>(smem + kRefOff);
-  float m_run = -__builtin_inff();  // reference of k-step dh per head c32 (an integer, log2 units)
+  float m_run = -__builtin_inff();  // reference per head c32 (log2 units), the same in both waves
   float m_max = -__builtin_inff();  // exact running maximum (log2 units), for max_out
-  float l_run = 0.f;                // sum of P against m_run, this lane's keys only
-  // A operand row m is key m ^ 16dh: the kept keys (k-step dh) are result rows
-  // 0-15 (registers 0-7), the partner's rows 16-31
-  const int krow = c32 ^ (16 * dh);
-  const uint8_t *fn[4], *fr[2];  // piece addresses in buffer 0
+  float l_run[2] = {0.f, 0.f};      // sums of P against m_run of key groups 2dh, 2dh + 1, this lane's keys only
+  // piece addresses in buffer 0: a nope k-step's piece is 16q + 2ks + h, of
+  // which the swizzle changes the low three bits
+  const uint8_t *fn[4], *fr[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) fn[j] = smem + krow * kFreshRowBytes + 512 * dh + 16 * ((4 * h + j) ^ (krow & 7));
+  for (int j = 0; j < 4; ++j) fn[j] = smem + c32 * kFreshRowBytes + 512 * dh + 16 * ((2 * j + h) ^ (c32 & 7));
 #pragma unroll
-  for (int i = 0; i < 2; ++i) fr[i] = smem + krow * kFreshRowBytes + 1024 + 16 * ((2 * (2 * dh + i) + h) ^ (krow & 7));
-  uint8_t* const x_out = smem + kPOff + (dh ^ 1) * 8192 + hp * 4096 + 2048 + lane * 16;  // the partner's slots
-  const uint8_t* const x_in = smem + kPOff + dh * 8192 + hp * 4096 + 2048 + lane * 16;
+  for (int i = 0; i < 2; ++i) fr[i] = smem + c32 * kFreshRowBytes + 1024 + 16 * ((2 * (2 * dh + i) + h) ^ (c32 & 7));
+  uint8_t* const x_out = smem + kRowsXOff + (2 * hp + dh) * 8192 + lane * 16;
+  const uint8_t* const x_in = smem + kRowsXOff + (2 * hp + (dh ^ 1)) * 8192 + lane * 16;
 
   for (int t = 0; t <= c.nblk; ++t) {
     iteration_start<kRows>(P, smem, c, dl, t);
     if (c.wave == kTabWave && t + 2 < c.nblk) build_addr_table<kRows>(P, smem, c, t + 2);
     const bool work = t < c.nblk && hp < kTiles;
-    float sv[8];
+    v16f s[2];
     if (work) {
-      const int boff = (t % kNumBufs) * kBufBytes;
-      v16f s;
+      const int boff = (t % kNumBufs) * kRowsBufBytes;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = 0.f;
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[i][r] = 0.f;
       v4i kb[2][4], kr[2];
+      // chunk k: k-steps 2k and 2k + 1 of both quarters
       auto read_chunk = [&](int k, v4i* dst) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dst[j] = *reinterpret_cast<const v4i*>(fn[j] + boff + 128 * k);
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            dst[2 * i + u] = *reinterpret_cast<const v4i*>(fn[2 * (k & 1) + u] + boff + 256 * i + 128 * (k >> 1));
       };
       read_chunk(0, kb[0]);
 #pragma unroll
@@ -670,39 +699,52 @@ __device__ __forceinline__ void qk_waves_rows(const MlaParams& P, uint8_t* smem,
           for (int i = 0; i < 2; ++i) kr[i] = *reinterpret_cast<const v4i*>(fr[i] + boff);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kb[k & 1][j]), as_v8bf(qn[k][j]), s, 0, 0, 0);
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kb[k & 1][2 * i + u]), as_v8bf(qn[i][2 * k + u]),
+                                                           s[i], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kr[i]), as_v8bf(qr[i]), s, 0, 0, 0);
-      *reinterpret_cast<v4f*>(x_out) = v4f{s[8], s[9], s[10], s[11]};
-      *reinterpret_cast<v4f*>(x_out + 1024) = v4f{s[12], s[13], s[14], s[15]};
+        s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_v8bf(kr[i]), as_v8bf(qr[i]), s[i], 0, 0, 0);
 #pragma unroll
-      for (int r = 0; r < 8; ++r) sv[r] = s[r];
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<v4f*>(x_out + (4 * i + g) * 1024) =
+              v4f{s[i][4 * g], s[i][4 * g + 1], s[i][4 * g + 2], s[i][4 * g + 3]};
     }
     barrier();
     if (work) {
-      const v4f xa = *reinterpret_cast<const v4f*>(x_in);
-      const v4f xb = *reinterpret_cast<const v4f*>(x_in + 1024);
+      v4f x[2][4];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) x[i][g] = *reinterpret_cast<const v4f*>(x_in + (4 * i + g) * 1024);
       const int32_t row_t = reinterpret_cast<const int32_t*>(smem + kRingOff + (t % kRingSlots) * 256)[lane];
       const uint32_t vmask = (uint32_t)__ballot(fresh_valid(P, row_t, lane));
+      // sv[r]: key 8(r/4) + 4h + r%4, head c32
+      float sv[16];
+      auto add_quarters = [&](auto quarter) {  // quarter(q, r): this score's partial over quarter q
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        sv[r] += xa[r];
-        sv[4 + r] += xb[r];
-      }
-      const bool all_valid = vmask == 0xffffffffu;
-      uint32_t vb8 = 0xffu;  // bit r: key 16dh + 8(r/4) + 4h + r%4 valid
-      if (!all_valid) {
-        const uint32_t vm = vmask >> (16 * dh + 4 * h);
-        vb8 = (vm & 0xfu) | ((vm >> 4) & 0xf0u);
+        for (int r = 0; r < 16; ++r) {
+          const int g = r >> 2;
+          sv[r] = ((quarter(g, r) + quarter((g + 1) & 3, r)) + quarter((g + 2) & 3, r)) + quarter((g + 3) & 3, r);
+        }
+      };
+      if (dh == 0) add_quarters([&](int q, int r) { return q < 2 ? s[q & 1][r] : x[q & 1][r >> 2][r & 3]; });
+      else add_quarters([&](int q, int r) { return q < 2 ? x[q & 1][r >> 2][r & 3] : s[q & 1][r]; });
+      if (vmask != 0xffffffffu) {
+        const uint32_t vm = vmask >> (4 * h);
 #pragma unroll
-        for (int r = 0; r < 8; ++r)
-          if (!((vb8 >> r) & 1u)) sv[r] = -__builtin_inff();
+        for (int r = 0; r < 16; ++r)
+          if (!((vm >> (8 * (r >> 2) + (r & 3))) & 1u)) sv[r] = -__builtin_inff();
       }
       float mloc = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
+      mloc = fmaxf(mloc, fmaxf(fmaxf(fmaxf(sv[8], sv[9]), fmaxf(sv[10], sv[11])),
+                               fmaxf(fmaxf(sv[12], sv[13]), fmaxf(sv[14], sv[15]))));
       {
         // the other lane half's maximum (the swap pairs the two halves)
         const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
@@ -710,43 +752,35 @@ __device__ __forceinline__ void qk_waves_rows(const MlaParams& P, uint8_t* smem,
       }
       const float mblk = mloc * P.scale_log2;
       m_max = fmaxf(m_max, mblk);
+      // lazy reference: it moves only when a block exceeds it by 2^8
       const bool need = mblk > m_run + kRescaleThreshold;
       if (__ballot(need)) {
-        const float m_new = need ? ceilf(mblk) : m_run;
-        l_run *= __builtin_amdgcn_exp2f(m_run - m_new);  // a power of two (0 from -inf)
+        const float m_new = need ? mblk : m_run;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 from -inf
+        l_run[0] *= alpha;
+        l_run[1] *= alpha;
         m_run = m_new;
       }
       const float m_use = m_run == -__builtin_inff() ? 0.f : m_run;
       float pv[8];
 #pragma unroll
       for (int r = 0; r < 8; ++r)
-        pv[r] = __builtin_amdgcn_exp2f(fmaxf(fmaf(sv[r], P.scale_log2, -m_use), kMinLogP));
-      if (!all_valid) {
-        // out of the sum; its P is written as 1.0, not 0, which the exponent
-        // adds of the PV waves could take to -inf (its V row is zeros)
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-          if (!((vb8 >> r) & 1u)) pv[r] = 0.f;
-      }
-      l_run += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
-      if (!all_valid) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-          if (!((vb8 >> r) & 1u)) pv[r] = 1.f;
-      }
-      *reinterpret_cast<v4i*>(smem + kPOff + (t & 1) * 8192 + hp * 4096 + dh * 1024 + lane * 16) =
+        pv[r] = __builtin_amdgcn_exp2f(fmaf(dh == 0 ? sv[r] : sv[8 + r], P.scale_log2, -m_use));
+      l_run[0] += (pv[0] + pv[1]) + (pv[2] + pv[3]);
+      l_run[1] += (pv[4] + pv[5]) + (pv[6] + pv[7]);
+      *reinterpret_cast<v4i*>(smem + kRowsPOff + (t & 1) * 4096 + hp * 2048 + dh * 1024 + lane * 16) =
           v4i{cvt_pk_bf16(pv[0], pv[1]), cvt_pk_bf16(pv[2], pv[3]), cvt_pk_bf16(pv[4], pv[5]), cvt_pk_bf16(pv[6], pv[7])};
     }
-    if (t < c.nblk && h == 0) ref[(((t & 1) * 2 + hp) * 2 + dh) * 32 + c32] = m_run;
+    if (t < c.nblk && h == 0 && dh == 0) ref[((t & 1) * 2 + hp) * 32 + c32] = m_run;
     iteration_end();
   }
   float* fin = reinterpret_cast<float*>(smem + kFinOff);
-  const float l2 = l_run + shfl_xor(l_run, 32);
-  if (h == 0) {
-    fin[(hp * 2 + dh) * 32 + c32] = l2;
-    fin[128 + (hp * 2 + dh) * 32 + c32] = m_run;
-    fin[256 + (hp * 2 + dh) * 32 + c32] = m_max;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float l2 = l_run[i] + shfl_xor(l_run[i], 32);
+    if (h == 0) fin[(4 * hp + 2 * dh + i) * 32 + c32] = l2;
   }
+  if (h == 0 && dh == 0) fin[256 + hp * 32 + c32] = m_max;
   barrier();
 }
 
@@ -792,7 +826,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
     iteration_start<kKeys>(P, smem, c, dl, t);
     if (t >= 1) {
       const int par = (t - 1) & 1;
-      const uint8_t* bufp = smem + ((t - 1) % kNumBufs) * kBufBytes;
+      const uint8_t* bufp = smem + ((t - 1) % kNumBufs) * buf_bytes<kKeys>();
       const bool fresh = rows_block<kKeys>(c, t - 1);
       if (!fresh) {
         // exponent table of block t-1, tile dq (lane = key): the tile scale's
@@ -803,17 +837,23 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
         const int pos = ((key >> 4) * 2 + ((key >> 2) & 1)) * 8 + 4 * ((key >> 3) & 1) + (key & 3);
         et[pos] = (uint16_t)((uint32_t)((((int)((sb >> 23) & 0xffu)) - 127) << 7) & 0xffffu);
       }
-      // each head tile's O follows the larger of its key-half references; O
-      // moves by a power of two
+      // each head tile's O follows the larger of its key-half references, moving
+      // by a power of two; over bf16 rows only it follows the one reference
       int fx[kTiles][2];
 #pragma unroll
       for (int mt = 0; mt < kTiles; ++mt) {
-        const float m0 = ref[((par * 2 + mt) * 2 + 0) * 32 + c32];
-        const float m1 = ref[((par * 2 + mt) * 2 + 1) * 32 + c32];
-        const float mn = fmaxf(m0, m1);
+        float m0, m1 = 0.f, mn;
+        if constexpr (kKeys == kRows) {
+          mn = m0 = ref[(par * 2 + mt) * 32 + c32];
+        } else {
+          m0 = ref[((par * 2 + mt) * 2 + 0) * 32 + c32];
+          m1 = ref[((par * 2 + mt) * 2 + 1) * 32 + c32];
+          mn = fmaxf(m0, m1);
+        }
         const bool up = mn > R[mt];
         if (__ballot(up)) {
-          const float alpha = up ? __builtin_amdgcn_exp2f(R[mt] - mn) : 1.f;  // 0 from -inf
+          // 0 from -inf (a head of bf16 rows that stays at -inf has NaN sums already)
+          const float alpha = up || kKeys == kRows ? __builtin_amdgcn_exp2f(R[mt] - mn) : 1.f;
           R[mt] = up ? mn : R[mt];
           int hb = 4 * h;
           asm volatile("" : "+v"(hb));
@@ -825,6 +865,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[mt][nn][r] *= ar[r];
         }
+        if constexpr (kKeys == kRows) continue;
         // per key half: m_kh - R (<= 0) for the bf16 exponent field (a key half
         // with no valid key yet has only zero rows in this block, so any finite
         // P' is fine there; a half more than 2^30 below R is scaled by 2^-30
@@ -837,7 +878,8 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
           fx[mt][k2] |= fx[mt][k2] << 16;
         }
       }
-      const uint8_t* pb = smem + kPOff + par * 8192;
+      constexpr int kPTile = kKeys == kRows ? 2048 : 4096;  // P of one head tile
+      const uint8_t* pb = smem + (kKeys == kRows ? kRowsPOff : kPOff) + par * 2 * kPTile;
       const uint32_t vb = lds_addr(bufp) + vlane;
       // The transposing reads take no immediate offset, so each address is
       // formed from an opaque base right before use; otherwise all of them
@@ -858,7 +900,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
         for (int nn = 0; nn < 4; ++nn)
           if (kKeys != kRows) vq[0][nn] = lds_read_tr8_at(a0 + 32 * nn);
 #pragma unroll
-        for (int mt = 0; mt < kTiles; ++mt) pq[0][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + lane * 16);
+        for (int mt = 0; mt < kTiles; ++mt) pq[0][mt] = *reinterpret_cast<const v4i*>(pb + mt * kPTile + lane * 16);
         if (kKeys != kRows) eq[0] = *reinterpret_cast<const v4i_alias*>(et + h * 8);
       }
 #pragma unroll
@@ -871,13 +913,15 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
             if (kKeys != kRows) vq[nxt][nn] = lds_read_tr8_at(a1 + 32 * nn);
 #pragma unroll
           for (int mt = 0; mt < kTiles; ++mt)
-            pq[nxt][mt] = *reinterpret_cast<const v4i*>(pb + mt * 4096 + ((ks + 1) * 64 + lane) * 16);
+            pq[nxt][mt] = *reinterpret_cast<const v4i*>(pb + mt * kPTile + ((ks + 1) * 64 + lane) * 16);
           if (kKeys != kRows) eq[nxt] = *reinterpret_cast<const v4i_alias*>(et + ((ks + 1) * 2 + h) * 8);
         }
         __builtin_amdgcn_sched_barrier(0);
-        // cache slots: k-steps 0, 1 are key half 0, 2, 3 half 1; rows only: k-step ks has its own reference
-        const int k2 = kKeys == kRows ? ks : ks >> 1;
-        if (kKeys == kRows && ks == 1) barrier();  // the QK waves' partial scores change hands
+        const int k2 = ks >> 1;  // k-steps 0, 1 are key half 0, 2, 3 half 1
+        // the QK waves' partial scores change hands: before the first product, as
+        // their softmax is the longer half (before nn = 2: 418 us where this takes
+        // 411, before ks = 1: 430, 512 tokens of 128 heads)
+        if (kKeys == kRows && ks == 0) barrier();
         if (fresh && ks >= 2) continue;  // a fresh block's 32 keys are k-steps 0, 1
         v4i pa[kTiles];
 #pragma unroll
@@ -885,7 +929,11 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             // (bit_cast of a vector element reads element 0; copy to scalars first)
-            const int pe = pq[cur][mt][e], ee = kKeys == kRows || fresh ? 0 : eq[cur][e];
+            const int pe = pq[cur][mt][e], ee = fresh ? 0 : eq[cur][e];
+            if (kKeys == kRows) {  // P as it is: one reference, no tile scale
+              pa[mt][e] = pe;
+              continue;
+            }
             const v2u16 sum = __builtin_bit_cast(v2u16, pe) + __builtin_bit_cast(v2u16, ee) +
                               __builtin_bit_cast(v2u16, fx[mt][k2]);
             pa[mt][e] = __builtin_bit_cast(int, sum);
@@ -923,8 +971,13 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
   for (int mt = 0; mt < kTiles; ++mt) {
     // total of P per head c32 of tile mt against R, and the exact maximum
     float lt = 0.f, mm = -__builtin_inff();
+    if constexpr (kKeys == kRows) {
+      const float* lg = fin + 4 * mt * 32 + c32;
+      lt = (lg[0] + lg[32]) + (lg[64] + lg[96]);
+      mm = fin[256 + mt * 32 + c32];
+    }
 #pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) {
+    for (int k2 = 0; k2 < 2 && kKeys != kRows; ++k2) {
       const float lk = fin[(mt * 2 + k2) * 32 + c32];
       const float mk = fin[128 + (mt * 2 + k2) * 32 + c32];
       if (mk != -__builtin_inff()) lt += lk * __builtin_amdgcn_exp2f(mk - R[mt]);
@@ -1038,7 +1091,7 @@ sparse_mla_kernel(const MlaParams P) {
   // the address tables of blocks 0 and 1, then block 0's rows
   if (c.wave == kIdxWave)
     for (int j = 0; j < 4 && j < c.nblk; ++j) issue_index<kKeys>(P, smem, c, j);
-  issue_query(P, smem, c, hg * kMlaHeadsPerWG);
+  issue_query<kKeys>(P, smem, c, hg * kMlaHeadsPerWG);
   const DmaLanes dl = dma_lanes(c.wave, c.lane);
   if (c.wave == kIdxWave)  // its index copies landed (the query's may still be on their way)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kQDma / kMlaWaves) : "memory");
@@ -1174,17 +1227,17 @@ static int launch_mla(const MlaParams& P, KeyKind keys, int64_t nwg, hipStream_t
                           (const void*)sparse_mla_kernel<kSlotsThenRows, 1>,
                           (const void*)sparse_mla_kernel<kSlotsThenRows, 2>, (const void*)sparse_mla_kernel<kRows, 1>,
                           (const void*)sparse_mla_kernel<kRows, 2>})
-      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMlaSmemBytes) != hipSuccess)
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRowsSmemBytes) != hipSuccess)
         smem_status = 1;
   }
-  if (smem_status) return set_error(kLaunchFailed, "sparse_mla: cannot reserve %zu B of LDS", kMlaSmemBytes);
+  if (smem_status) return set_error(kLaunchFailed, "sparse_mla: cannot reserve %zu B of LDS", kRowsSmemBytes);
   if (nwg > INT32_MAX) return set_error(kInvalidArgument, "%s: grid too large", what);
   void (*const kernels[3][2])(MlaParams) = {
       {sparse_mla_kernel<kSlots, 1>, sparse_mla_kernel<kSlots, 2>},
       {sparse_mla_kernel<kSlotsThenRows, 1>, sparse_mla_kernel<kSlotsThenRows, 2>},
       {sparse_mla_kernel<kRows, 1>, sparse_mla_kernel<kRows, 2>}};
-  hipLaunchKernelGGL(kernels[keys][P.H <= 32 ? 0 : 1], dim3((unsigned)nwg), dim3(kMlaThreads), kMlaSmemBytes, stream,
-                     P);
+  hipLaunchKernelGGL(kernels[keys][P.H <= 32 ? 0 : 1], dim3((unsigned)nwg), dim3(kMlaThreads),
+                     keys == kRows ? kRowsSmemBytes : kMlaSmemBytes, stream, P);
   return check_launch(what);
 }
 

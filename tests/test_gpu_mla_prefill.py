@@ -96,3 +96,60 @@ def test_prefill_on_dequantised_rows_equals_decode_on_fp8_rows(cuda):
     torch.cuda.synchronize()
     assert (o_p.float() - o_d.float()).abs().max().item() <= 2e-2
     assert (l_p - l_d).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("H", [16, 128])
+def test_a_row_of_one_key_returns_its_values(cuda, H):
+    """A prompt's first token attends to itself alone: P of the largest key is
+    exactly 1 and the sum too, so o is the key's value bit for bit, wherever
+    the key lies in its block; lse = max_logits up to a rounding of log2 units."""
+    T, K, s_kv = 64, 128, 200
+    q, kv, idx = _case(T, H, K, s_kv, seed=H)
+    first = idx[:, 0].clone()
+    idx[:] = -1
+    where = torch.arange(T, device=cuda) * 2 + 1
+    idx[torch.arange(T, device=cuda), where] = first
+    o, mx, lse = ops.sparse_mla_prefill(q, kv, idx, 192 ** -0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(o, kv[first.long(), None, :512].expand(T, H, 512))
+    assert torch.allclose(mx, lse, rtol=2.0 ** -22, atol=0)
+
+
+def test_keys_of_no_weight_add_nothing(cuda):
+    """A key far below the largest one has its true weight, not a floor: values
+    of 1e30 at weights below 2^-200 leave no trace, in the block of the largest
+    key, before it and after it."""
+    T, H, K, s_kv = 3, 64, 96, 96
+    q = torch.zeros(T, H, 576, dtype=torch.bfloat16, device=cuda)
+    q[..., 512] = 1
+    kv = torch.full((s_kv, 576), 1e30, dtype=torch.bfloat16, device=cuda)
+    kv[:, 512:] = 0
+    kv[:, 512] = -200.0
+    for t in range(T):
+        kv[32 * t + 5, :512] = t + 1.0
+        kv[32 * t + 5, 512] = 100.0 * t
+    idx = torch.arange(K, dtype=torch.int32, device=cuda)[None].repeat(T, 1)
+    idx[0, 37], idx[0, 69], idx[1, 69] = -1, -1, -1  # token t's largest key is in block t
+    o, _, _ = ops.sparse_mla_prefill(q, kv, idx, 1.0)
+    torch.cuda.synchronize()
+    expect = torch.arange(1, T + 1, device=cuda, dtype=torch.bfloat16)[:, None, None].expand(T, H, 512)
+    assert torch.equal(o, expect)
+
+
+def test_nan_scores_reach_the_output(cuda):
+    """A NaN in a head's query makes that head's output NaN, one in a key's rope
+    dims every head's of the tokens that select the key; nothing else changes."""
+    T, H, K, s_kv = 4, 128, 256, 600
+    q, kv, idx = _case(T, H, K, s_kv, seed=9)
+    idx[idx == 17] = 18
+    clean, _, _ = ops.sparse_mla_prefill(q, kv, idx, 192 ** -0.5)
+    q[2, 5, 100] = float("nan")
+    kv[17, 560] = float("nan")
+    idx[1, 3] = 17
+    o, _, _ = ops.sparse_mla_prefill(q, kv, idx, 192 ** -0.5)
+    torch.cuda.synchronize()
+    bad = torch.zeros(T, H, dtype=torch.bool, device=cuda)
+    bad[1] = True
+    bad[2, 5] = True
+    assert torch.isnan(o[bad]).all()
+    assert torch.equal(o[~bad], clean[~bad])

@@ -213,10 +213,14 @@ DSA_API int dsa_topk_to_physical(const int32_t* topk_indices, int64_t topk_strid
 /* Split count the sparse MLA decode uses for this shape (1 = no workspace):
  * of the (token, 64-head group) items, those that fill the CUs in whole rounds
  * run unsplit, and each of the rest splits its keys this many ways (at most 8,
- * at least four 64-key blocks each, block counts that differ by at most one). */
+ * at least four 64-key blocks each, block counts that differ by at most one;
+ * for a num_cus that is not this device's, an equal division of the blocks). */
 DSA_API int dsa_sparse_mla_num_splits(int num_tokens, int num_heads, int topk, int num_cus);
 
-/* Workspace bytes dsa_sparse_mla_decode needs for `num_splits`. */
+/* Workspace bytes dsa_sparse_mla_decode needs for `num_splits` on the current
+ * device: the partials of the items that are split. With more items than CUs,
+ * and parts that fit them, those are the items of the last, partial round, so
+ * that the size stays below num_cus * 64 * 513 * 4 bytes (33.6 MB). */
 DSA_API size_t dsa_sparse_mla_workspace_bytes(int num_tokens, int num_heads, int num_splits);
 
 /* Sparse MLA decode over the packed fp8 MLA cache.
@@ -238,9 +242,11 @@ DSA_API size_t dsa_sparse_mla_workspace_bytes(int num_tokens, int num_heads, int
  * no valid index yields o = 0 and lse = -inf.
  * num_heads % 16 == 0; topk % 64 == 0; num_splits in [1, topk/64] with
  * workspace >= dsa_sparse_mla_workspace_bytes(...) when num_splits > 1
- * (num_splits <= 0 picks dsa_sparse_mla_num_splits for this device). The
- * rule's own count splits as described there; any other must cut topk into
- * equal splits of whole 64-key blocks, and applies to every item.
+ * (num_splits <= 0 picks dsa_sparse_mla_num_splits for this device; without a
+ * workspace for it, more items than CUs, or an odd number of blocks, run
+ * unsplit). A count other than the rule's own must cut topk into equal splits of
+ * whole 64-key blocks. With more items than CUs, and where the parts of the last
+ * partial round fit the CUs, only that round's items are split, else every item.
  * Replaces flash_mla.flash_mla_with_kvcache(q, k_cache, None, None,
  * head_dim_v=512, sched_meta, None, softmax_scale, causal=False,
  * is_fp8_kvcache=True, indices=...) as called by FlashMlaAttention.forward

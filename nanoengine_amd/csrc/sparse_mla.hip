@@ -55,6 +55,7 @@
 // write normalised partial outputs and LSEs to a caller-provided workspace; a
 // combine kernel merges them with the LSE rule of merge_attention_states.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 
 #include "dsa_common.h"
@@ -149,8 +150,10 @@ struct MlaParams {
   float scale_log2;
   uint16_t* out;
   float* lse;
-  float* ws_o;    // [splits, T, H, 512] (splits > 1)
-  float* ws_lse;  // [splits, T, H]
+  // partials of the split items (splits > 1): (token, head) rows ws_row0 .. ws_row0 + ws_rows - 1
+  float* ws_o;    // [splits, ws_rows, 512]
+  float* ws_lse;  // [splits, ws_rows]
+  int64_t ws_row0, ws_rows;
   float* max_out; // [T, H] largest scaled score (natural units), or null (splits == 1 only)
   // chunked prefill (paged, splits == 1): token t attends over ceil(counts[2t] / 64)
   // blocks of cache slots from idx (valid slots first), then ceil(counts[2t+1] / 32)
@@ -1015,7 +1018,7 @@ __device__ __forceinline__ void pv_waves(const MlaParams& P, uint8_t* smem, cons
         if (P.max_out) P.max_out[(int64_t)c.t_tok * P.H + head] = any ? mm * kLn2 : -__builtin_inff();
       }
     } else {
-      const int64_t row0 = ((int64_t)split * P.T + c.t_tok) * P.H + h_half;
+      const int64_t row0 = split * P.ws_rows + (int64_t)c.t_tok * P.H + h_half - P.ws_row0;
       uint8_t* st = smem + dq * kStageOut;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -1119,18 +1122,19 @@ sparse_mla_kernel(const MlaParams P) {
 // (3.9 us for 4 tokens of 128 heads in 8 splits; one split after another, the
 // LSEs first: 5.5).
 __global__ void __launch_bounds__(64)
-sparse_mla_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_lse, int T, int H, int whole,
-                          int head_groups, int splits, uint16_t* __restrict__ out, float* __restrict__ lse_out) {
+sparse_mla_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_lse, int64_t ws_row0,
+                          int64_t ws_rows, int H, int whole, int head_groups, int splits, uint16_t* __restrict__ out,
+                          float* __restrict__ lse_out) {
   const int item = whole + (int)blockIdx.x / kMlaHeadsPerWG;
   const int head = item % head_groups * kMlaHeadsPerWG + (int)blockIdx.x % kMlaHeadsPerWG;
   if (head >= H) return;
   const int lane = threadIdx.x;
   const int64_t th = (int64_t)(item / head_groups) * H + head;
-  const int64_t stride = (int64_t)T * H;
+  const int64_t part = th - ws_row0, stride = ws_rows;
   constexpr int kGroup = 8;
-  const float* src = ws_o + th * kMlaDv + lane * 8;
+  const float* src = ws_o + part * kMlaDv + lane * 8;
   auto load_lse = [&](int s0) {  // split s0 + lane
-    return s0 + lane < splits ? ws_lse[(s0 + lane) * stride + th] : -__builtin_inff();
+    return s0 + lane < splits ? ws_lse[(s0 + lane) * stride + part] : -__builtin_inff();
   };
   v4f a[kGroup], b[kGroup];
   auto load_group = [&](int s0) {
@@ -1178,6 +1182,63 @@ sparse_mla_combine_kernel(const float* __restrict__ ws_o, const float* __restric
   if (lane == 0 && lse_out) lse_out[th] = wsum > 0.f ? m + logf(wsum) : -__builtin_inff();
 }
 
+static int64_t mla_items(int num_tokens, int num_heads) {
+  return (int64_t)num_tokens * ((num_heads + kMlaHeadsPerWG - 1) / kMlaHeadsPerWG);
+}
+
+// CUs of the current device (256 where there is none to ask), looked up once
+// per device.
+static int current_cus() {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> known[kMaxDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  if (dev >= 0 && dev < kMaxDevices)
+    if (const int n = known[dev].load(std::memory_order_relaxed)) return n;
+  const int n = dsa_num_cus(dev);
+  if (n > 0 && dev >= 0 && dev < kMaxDevices) known[dev].store(n, std::memory_order_relaxed);
+  return n > 0 ? n : 256;
+}
+
+// What a split count means for a batch on `cus` CUs. Past one round of items
+// the ones that fill the CUs in whole rounds stay unsplit, provided that the
+// parts of the others fit one round; then fewer than `cus` parts exist, however
+// many tokens there are, and the partials take at most cus x 64 rows (33.6 MB).
+// In every other case each item is split.
+struct MlaPartition {
+  int64_t whole;        // items [0, whole) are not split
+  int64_t row0, rows;   // (token, head) rows with partials
+};
+static MlaPartition mla_partition(int num_tokens, int num_heads, int splits, int cus) {
+  const int64_t items = mla_items(num_tokens, num_heads), rest = items % cus;
+  const int64_t all = (int64_t)num_tokens * num_heads;
+  if (items <= cus || rest == 0 || rest * splits > cus) return {0, 0, all};
+  const int groups = (num_heads + kMlaHeadsPerWG - 1) / kMlaHeadsPerWG;
+  const int64_t whole = items - rest;
+  const int64_t row0 = whole / groups * num_heads + whole % groups * kMlaHeadsPerWG;
+  return {whole, row0, all - row0};
+}
+
+static size_t mla_partial_bytes(const MlaPartition& p, int splits) {
+  return splits > 1 ? (size_t)splits * p.rows * (kMlaDv + 1) * sizeof(float) : 0;
+}
+
+// The split count chosen for `cus` CUs. A workgroup's time is a fixed start-up
+// (~8 us) plus a cost per 64-row block (2 to 2.6 us), and one workgroup runs per
+// CU at a time. The items that fill the CUs in whole rounds are not split; the
+// remaining ones (all of a small batch) split as far as they still fit the CUs
+// in one round, with at least 4 blocks per workgroup (below that the start-up
+// and the combine outweigh the shorter key list). Block counts may differ by one.
+static int mla_split_rule(int num_tokens, int num_heads, int topk, int cus) {
+  const int64_t rest = mla_items(num_tokens, num_heads) % cus;
+  if (rest == 0) return 1;
+  const int most = std::min(8, topk / (4 * kMlaKeys));
+  return std::max(1, (int)std::min<int64_t>(most, cus / rest));
+}
+
 }  // namespace dsa
 
 extern "C" {
@@ -1185,23 +1246,17 @@ extern "C" {
 int dsa_sparse_mla_num_splits(int num_tokens, int num_heads, int topk, int num_cus) {
   if (num_tokens <= 0 || num_heads <= 0 || topk <= 0) return 1;
   if (num_cus <= 0) num_cus = 256;
-  const int groups = (num_heads + dsa::kMlaHeadsPerWG - 1) / dsa::kMlaHeadsPerWG;
-  // A workgroup's time is a fixed start-up (~8 us) plus a cost per 64-row block
-  // (2 to 2.6 us), and one workgroup runs per CU at a time. The items that fill
-  // the CUs in whole rounds are not split; the remaining ones (all of a small
-  // batch) split as far as they still fit the CUs in one round, with at least 4
-  // blocks per workgroup (below that the start-up and the combine outweigh the
-  // shorter key list). Block counts may differ by one.
-  const int64_t rest = ((int64_t)num_tokens * groups) % num_cus;
-  if (rest == 0) return 1;
-  const int most = std::min(8, topk / (4 * dsa::kMlaKeys));
-  return std::max(1, (int)std::min<int64_t>(most, num_cus / rest));
+  int splits = dsa::mla_split_rule(num_tokens, num_heads, topk, num_cus);
+  // uneven parts are the launch's own choice on this device: a count for another
+  // number of CUs is one that any device takes
+  if (num_cus != dsa::current_cus())
+    while (splits > 1 && topk % (splits * dsa::kMlaKeys) != 0) --splits;
+  return splits;
 }
 
 size_t dsa_sparse_mla_workspace_bytes(int num_tokens, int num_heads, int num_splits) {
   if (num_splits <= 1 || num_tokens <= 0 || num_heads <= 0) return 0;
-  const size_t rows = (size_t)num_splits * num_tokens * num_heads;
-  return rows * dsa::kMlaDv * sizeof(float) + rows * sizeof(float);
+  return dsa::mla_partial_bytes(dsa::mla_partition(num_tokens, num_heads, num_splits, dsa::current_cus()), num_splits);
 }
 
 int dsa_sparse_mla_decode(const void* q, int64_t q_token_stride, int64_t q_head_stride,
@@ -1289,23 +1344,29 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
     return set_error(kInvalidArgument, "sparse_mla: q, kv_cache and out must be 16-byte aligned");
   if ((q_token_stride % 8) || (q_head_stride % 8))
     return set_error(kInvalidArgument, "sparse_mla: q strides must be multiples of 8 elements");
-  // the rule's split count leaves whole rounds of items unsplit; any other one
-  // splits every item into equal parts
-  const int64_t items = (int64_t)num_tokens * ((num_heads + kMlaHeadsPerWG - 1) / kMlaHeadsPerWG);
-  int64_t whole = 0;
+  int cus = 256;
   if (num_splits != 1) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    const int cus = std::max(1, dsa_num_cus(dev));
-    const int rule = dsa_sparse_mla_num_splits(num_tokens, num_heads, topk, cus);
-    if (num_splits <= 0) num_splits = rule;
-    if (num_splits == rule)
-      whole = items - items % cus;
-    else if (num_splits > topk / kMlaKeys || (topk / num_splits) % kMlaKeys != 0 || topk % num_splits != 0)
+    cus = current_cus();
+    const int rule = mla_split_rule(num_tokens, num_heads, topk, cus);
+    // Without room for the partials the library's own choice is not to split
+    // where a caller may not expect partials: more items than CUs, or a number
+    // of blocks that two parts would not share evenly.
+    if (num_splits <= 0) {
+      num_splits = rule;
+      const size_t bytes = mla_partial_bytes(mla_partition(num_tokens, num_heads, rule, cus), rule);
+      if (bytes > 0 && (!workspace || workspace_bytes < bytes) &&
+          (mla_items(num_tokens, num_heads) > cus || topk / kMlaKeys % 2 != 0))
+        num_splits = 1;
+    } else if (num_splits != rule &&
+               (num_splits > topk / kMlaKeys || (topk / num_splits) % kMlaKeys != 0 || topk % num_splits != 0)) {
       return set_error(kInvalidArgument, "sparse_mla: num_splits=%d does not split topk=%d into 64-row blocks",
                        num_splits, topk);
+    }
   }
-  const size_t need = dsa_sparse_mla_workspace_bytes(num_tokens, num_heads, num_splits);
+  const MlaPartition part = mla_partition(num_tokens, num_heads, num_splits, cus);
+  const int64_t items = mla_items(num_tokens, num_heads);
+  const int64_t whole = num_splits > 1 ? part.whole : 0;
+  const size_t need = mla_partial_bytes(part, num_splits);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(kWorkspaceTooSmall, "sparse_mla: workspace %zu B < %zu B", workspace_bytes, need);
 
@@ -1352,18 +1413,19 @@ int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head
     P.fresh_idx = fresh->idx;
     P.fresh_idx_stride = fresh->idx_stride;
   }
+  P.ws_row0 = part.row0;
+  P.ws_rows = part.rows;
   if (num_splits > 1) {
-    const size_t rows = (size_t)num_splits * num_tokens * num_heads;
     P.ws_o = static_cast<float*>(workspace);
-    P.ws_lse = P.ws_o + rows * kMlaDv;
+    P.ws_lse = P.ws_o + (size_t)num_splits * part.rows * kMlaDv;
   }
   const int64_t nwg = whole + (items - whole) * num_splits;
   if (int rc = launch_mla(P, fresh ? kSlotsThenRows : kSlots, nwg, (hipStream_t)stream, "dsa_sparse_mla_decode"))
     return rc;
   if (num_splits > 1) {
     hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)((items - whole) * kMlaHeadsPerWG)), dim3(64), 0,
-                       (hipStream_t)stream, P.ws_o, P.ws_lse, num_tokens, num_heads, P.whole, P.head_groups,
-                       num_splits, P.out, lse);
+                       (hipStream_t)stream, P.ws_o, P.ws_lse, P.ws_row0, P.ws_rows, num_heads, P.whole,
+                       P.head_groups, num_splits, P.out, lse);
     return check_launch("dsa_sparse_mla_decode(combine)");
   }
   return kOk;

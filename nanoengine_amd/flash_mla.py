@@ -15,11 +15,15 @@ from . import ops
 
 
 class SparseMlaSchedule:
-    """Opaque schedule: the split count and a workspace per shape. Every
-    shape's workspace is kept for the schedule's lifetime, because a HIP graph
-    captured at one shape holds that workspace's address: freeing it when the
-    shape changes would let later replays write their split partials over
-    whatever the allocator put there next."""
+    """Opaque schedule: the split count and a workspace per shape. A shape's
+    workspace is kept for the schedule's lifetime, because a HIP graph captured
+    at one shape holds that workspace's address: freeing it when the shape
+    changes would let later replays write their split partials over whatever the
+    allocator put there next. Batches of more (token, 64-head group) items than
+    CUs, of which only the last round is split, keep none (``workspace`` is
+    None): each call takes its own from torch's allocator, so that a schedule
+    does not hold up to 33.6 MB for every batch size it meets, and such calls
+    may run on several streams."""
 
     def __init__(self) -> None:
         self.num_splits: int | None = None
@@ -33,8 +37,11 @@ class SparseMlaSchedule:
             return
         if key not in self._by_key:
             splits = ops.sparse_mla_num_splits(num_tokens, num_heads, topk, device)
-            need = ops.sparse_mla_workspace_bytes(num_tokens, num_heads, splits)
-            self._by_key[key] = (splits, torch.empty(max(need, 1), dtype=torch.uint8, device=device))
+            ws = None
+            if not ops.sparse_mla_past_one_round(num_tokens, num_heads, device):
+                need = ops.sparse_mla_workspace_bytes(num_tokens, num_heads, splits)
+                ws = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
+            self._by_key[key] = (splits, ws)
         self.num_splits, self.workspace = self._by_key[key]
         self.key = key
 

@@ -372,6 +372,11 @@ def sparse_mla_num_splits(num_tokens: int, num_heads: int, topk: int, device=Non
     return int(_lib.load().dsa_sparse_mla_num_splits(num_tokens, num_heads, topk, num_cus(device)))
 
 
+def sparse_mla_past_one_round(num_tokens: int, num_heads: int, device=None) -> bool:
+    """More (token, 64-head group) items than CUs: only the last round of them is split."""
+    return num_tokens * -(-num_heads // 64) > num_cus(device)
+
+
 def sparse_mla_decode(q: torch.Tensor, k_cache: torch.Tensor, indices: torch.Tensor, sm_scale: float,
                       out: torch.Tensor | None = None, lse: torch.Tensor | None = None,
                       num_splits: int | None = None,

@@ -52,7 +52,19 @@ class DsaDecodeStep:
         self.num_splits = ops.sparse_mla_num_splits(rows, num_heads, index_topk, dev)
         need = ops.sparse_mla_workspace_bytes(rows, num_heads, self.num_splits)
         self.workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+        # past one round of CUs the object's own buffer serves the stream it was made on only
+        self._ws_stream = (ops._stream(self.workspace.device)
+                           if self.num_splits > 1 and ops.sparse_mla_past_one_round(rows, num_heads, dev) else None)
         self.topk_workspace = torch.empty(max(ops.topk_workspace_bytes(rows), 16), dtype=torch.uint8, device=dev)
+
+    def _split_workspace(self) -> torch.Tensor | None:
+        """The buffer for split partials; None (the call takes its own from
+        torch's allocator) on another stream than the constructor's for batches
+        past one round of CUs, whose attention calls with an ``out`` and ``lse`` of
+        their own may overlap."""
+        if self._ws_stream is not None and self._ws_stream != ops._stream(self.workspace.device):
+            return None
+        return self.workspace
 
     def expand_lens(self, context_lens: torch.Tensor) -> torch.Tensor:
         """Per-query causal lengths, flattened [batch*next_n] int32."""
@@ -88,7 +100,7 @@ class DsaDecodeStep:
             logical, physical = indexer_state.require(layer_idx, self.batch * self.next_n, self.topk,
                                                       require_physical=True)
             ops.sparse_mla_decode(q_mla, kv_cache, physical, sm_scale, out=o_buf, lse=lse_buf,
-                                  num_splits=self.num_splits, workspace=self.workspace)
+                                  num_splits=self.num_splits, workspace=self._split_workspace())
             return o_buf, lse_buf, logical, physical
         B, n = self.batch, self.next_n
         q4 = q_idx_fp8.view(B, n, *q_idx_fp8.shape[1:])
@@ -103,5 +115,5 @@ class DsaDecodeStep:
         if indexer_state is not None:
             indexer_state.publish(layer_idx, self.logical, self.physical)
         ops.sparse_mla_decode(q_mla, kv_cache, self.physical, sm_scale, out=o_buf, lse=lse_buf,
-                              num_splits=self.num_splits, workspace=self.workspace)
+                              num_splits=self.num_splits, workspace=self._split_workspace())
         return o_buf, lse_buf, self.logical, self.physical

@@ -163,3 +163,48 @@ def test_microbenchmark_library_exports_its_probes():
     for name in ["dsa_mb_page_read", "dsa_mb_page_read_layout", "dsa_mb_row_gather", "dsa_mb_lds_read", "dsa_mb_valu_issue",
                  "dsa_mb_mfma_rate", "dsa_mb_mix", "dsa_mb_fp8_mfma_sum"]:
         assert hasattr(mb, name), name
+
+
+def test_split_partials_are_bounded_past_one_round_of_cus(lib):
+    """Only the items of the last, partial round of CUs are split, so that the
+    partials take at most one round's rows (256 CUs x 64 heads) at any batch;
+    within one round every item's rows are there."""
+    row = (512 + 1) * 4
+    for heads in (16, 64, 80, 128, 192):
+        groups = -(-heads // 64)
+        for tokens in [*range(1, 700), 1025, 2049, 4097, 8193]:
+            splits = lib.dsa_sparse_mla_num_splits(tokens, heads, 2048, 256)
+            need = lib.dsa_sparse_mla_workspace_bytes(tokens, heads, splits)
+            assert need <= 256 * 64 * row, (tokens, heads, splits, need)
+            if splits > 1:
+                rest = tokens * groups % 256
+                assert need <= splits * rest * 64 * row
+                if tokens * groups <= 256:
+                    assert need == splits * tokens * heads * row
+    assert lib.dsa_sparse_mla_workspace_bytes(129, 128, 8) == 8 * 128 * row
+    assert lib.dsa_sparse_mla_workspace_bytes(2049, 128, 8) == 8 * 128 * row
+    # a count whose parts do not fit one round splits every item
+    assert lib.dsa_sparse_mla_workspace_bytes(200, 128, 2) == 2 * 200 * 128 * row
+
+
+def test_split_counts_for_other_devices_divide_the_blocks(lib):
+    """A count asked for another number of CUs is one every device's decode takes."""
+    for cus in (64, 128, 304):
+        for tokens in range(1, 200):
+            for topk in (512, 576, 2048):
+                splits = lib.dsa_sparse_mla_num_splits(tokens, 128, topk, cus)
+                assert topk % (64 * splits) == 0, (tokens, topk, cus, splits)
+
+
+def test_a_schedule_keeps_workspaces_of_one_round_only(monkeypatch):
+    import torch
+    from nanoengine_amd import flash_mla, ops
+    monkeypatch.setattr(ops, "num_cus", lambda device=None: 256)
+    sched, _ = flash_mla.get_mla_metadata()
+    for tokens in range(1, 1000):
+        sched.prepare(tokens, 128, 2048, torch.device("meta"))
+        assert (sched.workspace is None) == (tokens > 128)
+    kept = sum(ws.numel() for _, ws in sched._by_key.values() if ws is not None)
+    # the largest of every batch size up to one round
+    splits = {t: min(8, 256 // (2 * t)) for t in range(1, 129)}
+    assert kept <= sum(s * t * 128 * 513 * 4 for t, s in splits.items() if s > 1) + 128 < 1.75e9

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle as O
-from nanoengine_amd import flash_mla, ops, synth
+from nanoengine_amd import _lib, flash_mla, ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -335,3 +335,80 @@ def test_combine_takes_any_number_of_splits(cuda, splits, K):
     assert torch.all((a - b).abs() <= 2.0 ** -8 * (torch.maximum(a.abs(), b.abs()) + 1.0))
     assert torch.all((lse[0] - lse1[0]).abs() <= 1e-5)
     assert (o[1] == 0).all() and torch.equal(lse[1], lse1[1])
+
+
+@pytest.mark.parametrize("T,H", [(129, 128), (300, 80), (90, 192), (515, 16)])
+def test_partials_past_one_round_stay_in_their_workspace(cuda, T, H):
+    """More items than CUs: the partials of the last round's items only, in a
+    workspace of the size asked for and not a byte past it; o and lse are those
+    of the unsplit kernel within the bounds above."""
+    K = 2048
+    q, kv, idx = _case(T, H, K, num_blocks=80, seed=T + H)
+    splits = ops.sparse_mla_num_splits(T, H, K, cuda)
+    need = ops.sparse_mla_workspace_bytes(T, H, splits)
+    assert splits > 1 and 0 < need <= 256 * 64 * 513 * 4
+    ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=cuda)
+    o, lse = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5, num_splits=splits, workspace=ws[:need])
+    o1, lse1 = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5, num_splits=1)
+    torch.cuda.synchronize()
+    assert (ws[need:] == 0x5A).all()
+    a, b = o.float(), o1.float()
+    assert torch.all((a - b).abs() <= 2.0 ** -8 * (torch.maximum(a.abs(), b.abs()) + 1.0))
+    assert torch.all((lse - lse1).abs() <= 1e-5)
+
+
+@pytest.mark.parametrize("T,K,runs", [(129, 2048, True), (5, 576, True), (20, 2048, False)])
+def test_the_library_choice_without_a_workspace(cuda, T, K, runs):
+    """num_splits <= 0 without a workspace: batches past one round of CUs and odd
+    numbers of blocks run unsplit, other small batches are refused."""
+    H = 128
+    q, kv, idx = _case(T, H, K, num_blocks=80, seed=T)
+    o, lse = torch.empty(T, H, 512, dtype=torch.bfloat16, device=cuda), torch.empty(T, H, device=cuda)
+    stride, rows = ops.mla_kv_geometry(kv)
+    status = _lib.load().dsa_sparse_mla_decode(
+        q.data_ptr(), q.stride(0), q.stride(1), kv.data_ptr(), stride, rows, kv.shape[0], idx.data_ptr(),
+        idx.stride(0), T, H, K, 192 ** -0.5, o.data_ptr(), lse.data_ptr(), 0, None, 0,
+        torch.cuda.current_stream().cuda_stream)
+    assert (status == 0) == runs
+    if runs:
+        o1, lse1 = ops.sparse_mla_decode(q, kv, idx, 192 ** -0.5, num_splits=1)
+        assert torch.equal(o, o1) and torch.equal(lse, lse1)
+
+
+def test_one_schedule_past_one_round_on_two_streams(cuda):
+    """Batches past one round of CUs share nothing between calls of one schedule:
+    two streams and a captured graph give the results of ordered calls."""
+    T, H, K, scale = 140, 128, 512, 192 ** -0.5
+    sched, _ = flash_mla.get_mla_metadata()
+    sets = []
+    for seed in (1, 2):
+        q, kv, idx = _case(T, H, K, num_blocks=80, seed=seed)
+        sets.append((q.view(T, 1, H, 576), kv, idx.view(T, 1, K)))
+
+    def call(i):
+        q, kv, idx = sets[i]
+        return flash_mla.flash_mla_with_kvcache(q, kv, None, None, 512, sched, None, scale, is_fp8_kvcache=True,
+                                                indices=idx)
+
+    expect = [[t.clone() for t in call(i)] for i in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(10):
+        got = []
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got.append(call(i))
+        torch.cuda.synchronize()
+        for i in range(2):
+            assert all(torch.equal(a, b) for a, b in zip(got[i], expect[i]))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        outs = call(0)
+    for _ in range(3):
+        for t in outs:
+            t.zero_()
+        call(1)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, expect[0]))

@@ -76,7 +76,8 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_floa
 // samples: f sampled scores are expected in the top-k, the threshold is the
 // sample's rank f + 4 sqrt(f) + 8. Of a 128K decode row f = 16: 6144 entries
 // overflowed once in 10 rows, 16384 hold 7.8 standard deviations. Of a 128K
-// prefill row f = 32: 3 rows in 10000 overflowed 6144, 8192 hold 5.8.
+// prefill row f = 32: 3 rows in 10000 overflowed 6144, 8192 hold 5.8. The list
+// select takes every list that holds between top_k and CAP entries.
 template <int CAP>
 struct RowListT {
   static constexpr int kCap = CAP;
@@ -87,7 +88,7 @@ struct RowListT {
   uint32_t key[CAP];
   uint32_t pos[CAP];
 };
-constexpr int kListCap = 6144;  // also the entries a select keeps in LDS
+constexpr int kListCap = 6144;  // also the entries the finish kernel keeps in LDS
 using RowWs = RowListT<kListCap>;
 using DecodeList = RowListT<16384>;
 using PrefillList = RowListT<8192>;

@@ -55,7 +55,7 @@ struct ScoreBins {
   __device__ __forceinline__ ScoreBins(float lowest, float highest) {
     lo = lowest;
     const float range = highest - lowest;
-    scale = range > 0.f && range < 3.0e38f ? (float)(kHistBins - 1) / range : 0.f;
+    scale = range > 0.f && range < __builtin_inff() ? (float)(kHistBins - 1) / range : 0.f;
   }
   __device__ __forceinline__ ScoreBins(uint32_t kmin, uint32_t kmax)
       : ScoreBins(key_to_float(kmin), key_to_float(kmax)) {}
@@ -81,6 +81,40 @@ struct BitBins {
   }
   __device__ __forceinline__ uint32_t bin(float score) const {
     return score < lo ? 0u : min((__float_as_uint(score) - base) >> shift, (uint32_t)(kHistBins - 1));
+  }
+};
+
+// The same on order keys: 4096 bins linear in the key from kmin to kmax; lower
+// keys share bin 0, higher ones the last.
+struct KeyBins {
+  uint32_t base;
+  int shift;
+  __device__ __forceinline__ KeyBins(uint32_t kmin, uint32_t kmax)
+      : base(kmin), shift(max(0, 32 - (int)__clz((int)(max(kmin, kmax) - kmin)) - 12)) {}
+  __device__ __forceinline__ uint32_t of(uint32_t key) const {
+    return key < base ? 0u : min((key - base) >> shift, (uint32_t)(kHistBins - 1));
+  }
+};
+
+// 4096 bins for the scores of keys kmin to kmax: positive ones linear in the
+// key; ones that cross zero linear in the score, unless the largest is far above
+// the lowest's magnitude (an outlier, a long tail), where the 40 octaves below
+// it take the bins. One type, chosen at run time: an instantiation of the list
+// select for each would run its code cold.
+struct ListBins {
+  ScoreBins scores;
+  KeyBins keys;
+  bool linear;
+  __device__ __forceinline__ ListBins(uint32_t kmin, uint32_t kmax)
+      : scores(kmin, kmax), keys(kmin, kmax), linear(false) {
+    if (kmin > order_key(0.f)) return;
+    const float lo = key_to_float(kmin), hi = key_to_float(kmax);
+    if (hi > -16.f * lo) keys = KeyBins(order_key(hi * 0x1p-40f), kmax);
+    else linear = true;
+  }
+  __device__ __forceinline__ uint32_t of(uint32_t key) const {
+    const uint32_t a = scores.of(key), b = keys.of(key);
+    return linear ? a : b;
   }
 };
 

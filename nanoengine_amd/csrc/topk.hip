@@ -61,19 +61,15 @@ struct TopkSmem {
 };
 constexpr size_t kTopkSmemBytes = sizeof(TopkSmem);
 
-// LDS of the list select: the candidates of a level's threshold bin are kept
-// as 16-bit indices into the row's list (values re-read from global), so two
-// workgroups fit on a CU. A row the kernel repairs itself uses TopkSmem.
+// LDS of the list select (two workgroups fit on a CU). A row the kernel repairs
+// itself uses TopkSmem.
 struct ListSmem {
   uint32_t hist[kHistBins];
   uint32_t bitmap[kBitmapWords];
-  uint16_t list[2][kListCap];
   uint64_t rank[kRankCap];
   uint32_t wave_sum[16];
-  uint32_t list_count[2];
-  uint32_t tb, above, eq;
+  uint32_t count, tb, above, eq;
 };
-static_assert(DecodeList::kCap <= 65536 && PrefillList::kCap <= 65536, "list indices are 16-bit");
 static_assert(sizeof(ListSmem) <= sizeof(TopkSmem), "a repairing launch covers the list layout");
 
 __device__ __forceinline__ uint32_t radix_digit(int level, uint32_t key, uint32_t pos) {
@@ -483,15 +479,7 @@ topk_finish_kernel(const RowIn in, RowWs* __restrict__ ws, const int32_t* __rest
              out_page, out_raw, top_k, blockIdx.x);
 }
 
-// ---------------------------------------------------------------- list select
-// Exact top-k of a row's candidate list (fused indexer path), ranked by
-// (score, lower position). The first digit is the score's linear bin; the
-// threshold bin then holds a few candidates, whose rank each of them counts
-// directly. (Radix digits of the key's bits, all levels, took 17.0 us for four
-// rows of 4K tokens, whose scores cross zero: sign and exponent bits put most
-// candidates into a few bins, where the LDS atomics serialise.) A row whose list is unusable (fewer than k entries, more than the
-// list capacity, or more than kListCap of them sharing the first digit's
-// threshold bin, as when most of its scores tie) is redone or deferred.
+// ---------------------------------------------------------------- row repair
 // Full indexer logits of one row by the calling workgroup (kTopkThreads
 // threads): wave w computes pages w, w + 8, ... of the row through three
 // rotating page buffers, logits[t] for t < len.
@@ -524,8 +512,20 @@ __device__ void repair_row_logits(const RowRepair& rp, const int32_t* __restrict
   }
 }
 
-// The list select of one row per workgroup. kRepair: a row whose list is
-// unusable is redone in the kernel from its full logits (rp.q set, the launch
+// ---------------------------------------------------------------- list select
+// Exact top-k of a row's candidate list (fused indexer path), ranked by
+// (score, lower position), one row per workgroup. The first digit is a bin of
+// the score (ListBins); the threshold bin's few candidates count those ahead of
+// them. A crowded bin is binned again over its own range, and ties take radix
+// levels, each a pass over the list: no usable list is redone from the logits,
+// however its scores lie. (Radix digits of the key's bits, all levels, took 17.0
+// us for four rows of 4K tokens, whose scores cross zero: sign and exponent bits
+// put most candidates into a few bins, where the LDS atomics serialise. Bins
+// linear in the score only: 128 rows of 64K, normal scores 14.0 us here and
+// there, one outlier in each 27.0 against 15.8; 16 rows of 128K with a long tail
+// 712 against 15.2, as a crowded bin of more than 6144 made the row be redone.)
+// kRepair: a row whose list is unusable (fewer than k entries, or more than its
+// capacity) is redone in the kernel from its full logits (rp.q set, the launch
 // reserves TopkSmem); otherwise it is appended to rp.defer_rows.
 template <bool kRepair, typename RowList>
 __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_lens, int64_t max_len,
@@ -554,7 +554,7 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
     return;
   }
   const uint32_t cand = __builtin_amdgcn_readfirstlane(w.count);
-  const auto select_list = [&]() -> bool {
+  const auto select_list = [&]() {
   // The first kReg * NT candidates into registers (element e = u * NT + tid),
   // all loads in flight at once; any beyond them (a misjudged threshold) are
   // read again by each pass. Slots past the list are skipped by uniform
@@ -571,11 +571,11 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
       cl[u] = w.pos[e];
     }
   }
-  auto each = [&](auto&& f) {  // f(element, key, position) over this thread's candidates
+  auto each = [&](auto&& f) {  // f(key, position) over this thread's candidates
 #pragma unroll
     for (int u = 0; u < kReg; ++u)
-      if ((uint32_t)(u * NT) < cand && (uint32_t)(u * NT + tid) < cand) f((uint32_t)(u * NT + tid), ch[u], cl[u]);
-    for (uint32_t e = kReg * NT + tid; e < cand; e += NT) f(e, w.key[e], w.pos[e]);
+      if ((uint32_t)(u * NT) < cand && (uint32_t)(u * NT + tid) < cand) f(ch[u], cl[u]);
+    for (uint32_t e = kReg * NT + tid; e < cand; e += NT) f(w.key[e], w.pos[e]);
   };
   // The selected positions are marked in LDS: a byte each where the row fits
   // (plain stores), else a bit each. In a short row most positions are
@@ -608,99 +608,142 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   }
   for (int i = tid; i < nwords; i += NT) s.bitmap[i] = 0u;
   for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
-  if (tid == 0) s.list_count[0] = 0u;
+  if (tid == 0) s.count = 0u;
+  auto block_range = [&](uint32_t& low, uint32_t& high) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      low = min(low, (uint32_t)__shfl_xor(low, off, 64));
+      high = max(high, (uint32_t)__shfl_xor(high, off, 64));
+    }
+    if (lane == 0) {
+      s.wave_sum[wave] = low;
+      s.wave_sum[NT / 64 + wave] = high;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) {
+      low = min(low, s.wave_sum[i]);
+      high = max(high, s.wave_sum[NT / 64 + i]);
+    }
+  };
+  // the range of the scores above -inf (which ranks below every bin's start)
+  const uint32_t ninf = order_key(-__builtin_inff()), fmax_key = order_key(3.4028235e38f);
   uint32_t kmin = 0xffffffffu, kmax = 0u;
-  each([&](uint32_t, uint32_t key, uint32_t) {
-    kmin = min(kmin, key);
+  each([&](uint32_t key, uint32_t) {
+    kmin = min(kmin, key > ninf ? key : 0xffffffffu);
     kmax = max(kmax, key);
   });
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
-    kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
-  }
-  if (lane == 0) {
-    s.wave_sum[wave] = kmin;
-    s.wave_sum[NT / 64 + wave] = kmax;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NT / 64; ++i) {
-    kmin = min(kmin, s.wave_sum[i]);
-    kmax = max(kmax, s.wave_sum[NT / 64 + i]);
-  }
+  block_range(kmin, kmax);
   uint8_t* const flags = reinterpret_cast<uint8_t*>(s.bitmap);
   auto mark = [&](uint32_t pos) {
     if (bytes) flags[pos] = 1;
     else atomicOr(&s.bitmap[pos >> 5], 1u << (pos & 31));
   };
 
-  // first digit, straight from the registers: 4096 bins linear in the score,
-  // so that the threshold bin holds a few candidates whatever the scores' range
-  const ScoreBins bins(kmin, kmax);
   uint32_t remain = (uint32_t)top_k;
-  each([&](uint32_t, uint32_t key, uint32_t) { atomicAdd(&s.hist[bins.of(key)], 1u); });
-  __syncthreads();
-  find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
-  const uint32_t tb = s.tb, above = s.above, eq = s.eq;
-  remain -= above;
-  bool last = eq == remain;  // the whole bin is selected
-  if (!last && eq > (uint32_t)kListCap) return false;  // more than LDS holds (find_threshold ended with a barrier)
-  each([&](uint32_t e, uint32_t key, uint32_t pos) {
-    const uint32_t d = bins.of(key);
-    if (d > tb || (last && d == tb)) {
-      mark(pos);
-    } else if (!last && d == tb) {
-      const uint32_t slot = atomicAdd(&s.list_count[0], 1u);
-      s.list[0][slot] = (uint16_t)e;
-      if (slot < (uint32_t)kRankCap) s.rank[slot] = rank_composite(key, pos);
-    }
-  });
-  __syncthreads();
-  if (!last && eq <= (uint32_t)kRankCap) {
-    // each of the threshold bin's candidates counts those ahead of it
-    if ((uint32_t)tid < eq) {
+  bool done = false;
+  // One digit over the candidates that `visit` passes on: those in a higher bin
+  // than the threshold's are selected, the ones in it ranked if they are few;
+  // otherwise [kmin, kmax] becomes their range (bins never decrease with the
+  // key, so that the range holds no others). Bin 0 is counted in registers: a
+  // crowd in it would serialise on one LDS word.
+  auto digit = [&](const ListBins bins, auto&& visit) {
+    uint32_t lowest = 0;
+    visit([&](uint32_t key, uint32_t) {
+      const uint32_t d = bins.of(key);
+      if (d) atomicAdd(&s.hist[d], 1u);
+      else ++lowest;
+    });
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) lowest += (uint32_t)__shfl_xor(lowest, off, 64);
+    if (lane == 0 && lowest) atomicAdd(&s.hist[0], lowest);
+    __syncthreads();
+    find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
+    const uint32_t tb = s.tb, eq = s.eq;
+    remain -= s.above;
+    const bool whole_bin = eq == remain, ranked = !whole_bin && eq <= (uint32_t)kRankCap;
+    uint32_t low = 0xffffffffu, high = 0u;
+    visit([&](uint32_t key, uint32_t pos) {
+      const uint32_t d = bins.of(key);
+      if (d > tb || (whole_bin && d == tb)) {
+        mark(pos);
+      } else if (d == tb) {
+        if (ranked) {
+          s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key, pos);
+        } else {
+          low = min(low, key);
+          high = max(high, key);
+        }
+      }
+    });
+    __syncthreads();
+    done = whole_bin || ranked;
+    if (ranked && (uint32_t)tid < eq) {
+      // each of the threshold bin's candidates counts those ahead of it
       const uint64_t mine = s.rank[tid];
       uint32_t ahead = 0;
       for (uint32_t j = 0; j < eq; ++j) ahead += s.rank[j] > mine ? 1u : 0u;
       if (ahead < remain) mark(kIdxMax - (uint32_t)(mine & kIdxMax));
     }
-    last = true;
-  }
+    if (!done) {
+      block_range(low, high);
+      kmin = low;
+      kmax = high;
+    }
+  };
+  digit(ListBins(kmin, min(kmax, fmax_key)), each);
 
-  // a crowded threshold bin (many equal or nearly equal scores): radix levels
-  // of 12 bits of [ key - kmin : nb ][ (2^18-1) - position : 18 ] over its list
-  const CompositeDigits digits(kmin, kmax);
-  int cur = 0;
-  for (int L = 0; L < digits.levels && !last; ++L) {
-    const uint32_t n = s.list_count[cur];
-    const int nbins = digits.bins(L);
-    const int nxt = cur ^ 1;
-    // list_count[cur] is read by every thread above; list_count[nxt] was last
-    // read a level ago
-    for (int i = tid; i < nbins; i += NT) s.hist[i] = 0u;
-    if (tid == 0) s.list_count[nxt] = 0u;
-    __syncthreads();
-    // the list's candidates, re-read from the row's list (L2)
-    auto cand_key = [&](uint32_t i) { return w.key[s.list[cur][i]]; };
-    auto cand_pos = [&](uint32_t i) { return w.pos[s.list[cur][i]]; };
-    for (uint32_t e = tid; e < n; e += NT) atomicAdd(&s.hist[digits.of(cand_key(e), cand_pos(e), L)], 1u);
-    __syncthreads();
-    find_threshold<NT>(s.hist, s.wave_sum, nbins, remain, &s.tb, &s.above, &s.eq);
-    const uint32_t tb = s.tb, above = s.above, eq = s.eq;
-    remain -= above;
-    last = (eq == remain) || L == digits.levels - 1;
-    for (uint32_t e = tid; e < n; e += NT) {
-      const uint32_t pos = cand_pos(e), d = digits.of(cand_key(e), pos, L);
-      if (d > tb || (last && d == tb)) {
-        mark(pos);
-      } else if (!last && d == tb) {
-        const uint32_t slot = atomicAdd(&s.list_count[nxt], 1u);
-        s.list[nxt][slot] = s.list[cur][e];
+  if (!done) {
+    // The crowded paths read the list again (from L2, four entries in flight), so
+    // that they cost the usual one no registers.
+    auto again = [&](auto&& f) {
+#pragma unroll 1
+      for (uint32_t e0 = tid; e0 < cand; e0 += 4 * NT) {
+        uint32_t key[4], pos[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t e = e0 + u * NT;
+          key[u] = e < cand ? w.key[e] : 0u;
+          pos[u] = e < cand ? w.pos[e] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (e0 + u * NT < cand && key[u] >= kmin && key[u] <= kmax) f(key[u], pos[u]);
+      }
+    };
+    for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
+    // -inf, alone below every other score, must not stretch the range
+    uint32_t low = 0xffffffffu, high = 0u;
+    again([&](uint32_t key, uint32_t) {
+      low = min(low, key > ninf ? key : 0xffffffffu);
+      high = max(high, key);
+    });
+    __syncthreads();  // every thread has read the bin's range
+    block_range(low, high);
+    digit(ListBins(low, min(high, fmax_key)), again);
+    if (!done) {
+      // ties: radix levels of 12 bits of [ key - kmin ][ (2^18-1) - position : 18 ]
+      const CompositeDigits digits(kmin, kmax);
+      uint64_t prefix = 0;  // the digits chosen so far
+      for (int L = 0; L < digits.levels && !done; ++L) {
+        __syncthreads();  // every thread has read the previous level's outcome
+        for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
+        __syncthreads();
+        again([&](uint32_t key, uint32_t pos) {
+          if (digits.above(key, pos, L) == prefix) atomicAdd(&s.hist[digits.of(key, pos, L)], 1u);
+        });
+        __syncthreads();
+        find_threshold<NT>(s.hist, s.wave_sum, digits.bins(L), remain, &s.tb, &s.above, &s.eq);
+        const uint32_t t = s.tb;
+        remain -= s.above;
+        done = s.eq == remain || L == digits.levels - 1;
+        again([&](uint32_t key, uint32_t pos) {
+          const uint32_t d = digits.of(key, pos, L);
+          if (digits.above(key, pos, L) == prefix && (d > t || (done && d == t))) mark(pos);
+        });
+        prefix = prefix * (uint32_t)digits.bins(L) + t;
       }
     }
-    __syncthreads();
-    cur = nxt;
   }
 
   // compaction in position order and output
@@ -719,13 +762,14 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   } else {
     for (int i = tid; i < top_k; i += NT) out.emit(i, i < (int)total ? (int32_t)sel[i] : -1);
   }
-  return true;
   };
-  if (cand >= (uint32_t)top_k && cand <= (uint32_t)RowList::kCap && select_list()) return;
+  if (cand >= (uint32_t)top_k && cand <= (uint32_t)RowList::kCap) {
+    select_list();
+    return;
+  }
 
   // A row whose list cannot give the exact top-k (the sample misjudged its
-  // threshold, or its scores tie) is redone here, from its full logits, or
-  // left to the caller.
+  // threshold) is redone here, from its full logits, or left to the caller.
   if (tid == 0) w.failed = 1u;
   if constexpr (kRepair) {
     repair_row_logits(rp, page_table + (int64_t)(b / pt_div) * pt_stride, b, len);

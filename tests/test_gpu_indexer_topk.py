@@ -208,3 +208,69 @@ def test_short_contexts_with_repeated_scores(cuda, length, pages, one_score, max
     g_phys, g_logi = _fused(inp, cl, max_ctx, 2048, 1)
     assert np.array_equal(g_logi, e_logi)
     assert np.array_equal(g_phys, e_phys)
+
+
+def _list_flags(workspace, rows):
+    """(candidates, redone) of each row's candidate list: 16-byte header, 16384 keys and positions."""
+    head = workspace.view(torch.int32)[: rows * (4 + 2 * 16384)].view(rows, -1)[:, :4].cpu()
+    return head[:, 1], head[:, 2]
+
+
+def _long_rows(rows, length, seed):
+    """Decode rows over one shared context: queries of their own, the same pages."""
+    one = synth.make_indexer_inputs([length], next_n=1, seed=seed, device="cuda")
+    many = synth.make_indexer_inputs([64] * rows, next_n=1, seed=seed + 1, device="cuda")
+    width = max(one.block_tables.shape[1], 2048)  # a context limit of 128K: lists, not whole rows
+    bt = torch.zeros(rows, width, dtype=torch.int32, device="cuda")
+    bt[:, : one.block_tables.shape[1]] = one.block_tables
+    one.q_fp8, one.weights, one.block_tables = many.q_fp8, many.weights, bt
+    cl = torch.full((rows, 1), length, dtype=torch.int32, device="cuda")
+    return one, cl, width * 64
+
+
+@pytest.mark.parametrize("kind", ["normal", "outlier", "inf", "tail", "near", "ties"])
+@pytest.mark.parametrize("length", [131072, 6000])
+def test_long_lists_of_crowded_scores_are_not_redone(cuda, kind, length):
+    """Lists past 6144 entries (hot keys that the sample does not see), positive
+    ones and ones that cross zero, whose scores carry an outlier, an infinity, a
+    long tail, or lie close together: selected exactly from the list, without
+    the one-workgroup redo from the row's logits."""
+    print(f"long lists {kind} {length}", flush=True)
+    rows = 8
+    inp, cl, max_ctx = _long_rows(rows, length, seed=5)
+    # the key scales: a hot key's scores grow, whatever their sign
+    pages = inp.block_tables[0, : -(-length // 64)].long()
+    raw = inp.cache[pages]
+    scale = raw[:, 64 * 128:].contiguous().view(torch.float32)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    step = max(1, -(-pages.numel() // 16))
+    unseen = (torch.arange(pages.numel(), device="cuda") % step != 0)[:, None]
+    if length > 100000:
+        scale = torch.where(unseen & (torch.rand(scale.shape, generator=g, device="cuda") < 0.06), scale * 16, scale)
+    if kind in ("outlier", "inf"):
+        scale[3, 7:40] *= 1e9 if kind == "outlier" else 1e36  # the product with some scores overflows
+    if kind == "tail":
+        scale = scale * torch.exp(4 * torch.randn(scale.shape, generator=g, device="cuda"))
+    if kind in ("near", "ties"):  # one key everywhere: scores 1e-6 apart, or the same
+        raw[:, : 64 * 128] = raw[0, :128].repeat(64)
+        spread = torch.rand(scale.shape, generator=g, device="cuda") if kind == "near" else torch.zeros_like(scale)
+        scale = scale[0, 0] * (1 + 1e-6 * spread)
+        # most keys score nothing, so that lists of 2048 to 16384 remain
+        scale = torch.where(torch.rand(scale.shape, generator=g, device="cuda") < min(1.0, 8000 / length), scale, 0.0)
+    raw[:, 64 * 128:] = scale.contiguous().view(torch.uint8)
+    inp.cache[pages] = raw
+    e_phys, e_logi = _unfused(inp, cl, max_ctx, 2048, 1)
+    ws = torch.zeros(ops.indexer_topk_workspace_bytes(rows, 1, max_ctx), dtype=torch.uint8, device=cuda)
+    phys = torch.full((rows, 2048), 7, dtype=torch.int32, device=cuda)
+    logi = torch.full_like(phys, 7)
+    ops.indexer_topk(inp.q_fp8.view(rows, 1, 64, 128), inp.cache, inp.weights, cl, inp.block_tables, max_ctx, 2048,
+                     phys, logi, workspace=ws)
+    torch.cuda.synchronize()
+    count, redone = _list_flags(ws, rows)
+    print(kind, length, count.tolist(), redone.tolist(), flush=True)
+    assert np.array_equal(logi.cpu().numpy(), e_logi)
+    assert np.array_equal(phys.cpu().numpy(), e_phys)
+    usable = (count >= 2048) & (count <= 16384)
+    assert torch.equal(redone != 0, ~usable)
+    if kind not in ("near", "ties"):
+        assert usable.all() and (length < 100000 or (count > 6144).any())

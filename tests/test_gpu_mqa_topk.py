@@ -188,3 +188,33 @@ def test_nan_and_overflowing_scores_match_two_step(cuda):
     got = _fused(q, kv, sc, w, ks, ke, n)
     torch.cuda.synchronize()
     assert torch.equal(got, exp)
+
+
+@pytest.mark.parametrize("kind", ["normal", "outlier", "tail"])
+def test_long_lists_of_crowded_scores_are_not_deferred(cuda, kind):
+    """Lists past 6144 entries (hot keys between the sampled ones) with an
+    outlier or a long tail: exact, and no row is left to the host-ordered fix-up."""
+    print(f"mqa_topk long lists {kind}", flush=True)
+    m, n = 40, 131072
+    q, kv, sc, w = _inputs(cuda, m, n, seed=31, weights=torch.linspace(0.1, 1, 40 * 64, device=cuda).view(40, 64) * 0.01)
+    g = torch.Generator(device=cuda).manual_seed(7)
+    sc = torch.full_like(sc, 2.0 ** -6)
+    if kind == "tail":
+        sc = sc * torch.exp(4 * torch.randn(n, generator=g, device=cuda))
+    unseen = torch.arange(n, device=cuda) % 64 != 0
+    hot = unseen & (torch.rand(n, generator=g, device=cuda) < (3200 if kind == "tail" else 2500) / n)  # the tail's sample sees fewer candidates
+    sc[hot] *= 64 if kind != "tail" else 1e6
+    if kind == "outlier":
+        sc[777] *= 1e12
+    sc = sc.contiguous()
+    ks = torch.zeros(m, dtype=torch.int32, device=cuda)
+    ke = torch.full((m,), n, dtype=torch.int32, device=cuda)
+    expect = _two_step(q, kv, sc, w, ks, ke, n)
+    ws = torch.zeros(ops.mqa_topk_workspace_bytes(m, n), dtype=torch.uint8, device=cuda)
+    out = torch.full((m, 2048), -7, dtype=torch.int32, device=cuda)
+    ops.mqa_topk(q, kv, sc, w, ks, ke, n, out, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(out, expect)
+    head = ws.view(torch.int32)[: m * (4 + 2 * 8192)].view(m, -1)[:, :4].cpu()
+    print(kind, head[:, 1].tolist(), head[:, 2].tolist(), flush=True)
+    assert (head[:, 2] == 0).all() and (head[:, 1] > 6144).any()

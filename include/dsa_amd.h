@@ -131,15 +131,17 @@ DSA_API size_t dsa_topk_workspace_bytes(int batch);
  *   out_page        [batch, top_k] int32, contiguous
  *   out_raw         [batch, top_k] int32 or NULL
  *   workspace       >= dsa_topk_workspace_bytes(batch) bytes, 16-byte aligned,
- *                   or NULL (then every row takes the slower multi-pass path;
- *                   the result is the same)
+ *                   or NULL (then rows longer than 64K, or not 16-byte
+ *                   aligned, take the slower multi-pass path; the result is the
+ *                   same)
  * Row b selects the top_k largest scores among positions [0, seq_lens[b])
  * (ties: lowest positions; NaN ranks as -inf), writes them in ascending
  * position order as raw positions and as slots
  * (page_table[p >> log2(page_size)] << log2(page_size)) | (p & (page_size-1)),
  * then pads with -1. seq_lens[b] <= top_k emits 0..seq_lens[b]-1.
  * top_k in {512, 2048}; page_size a power of two;
- * row length <= dsa_topk_max_len(); `max_len` bounds seq_lens (the score width).
+ * row length <= dsa_topk_max_len(); `max_len` is the score width: it bounds
+ * seq_lens, and every row's storage holds that many scores.
  * Calls that share a workspace must be ordered (same stream).
  * Replaces topk_transform(scores, seq_lens, page_tables, out_page_indices,
  * page_size, top_k, out_raw_indices)

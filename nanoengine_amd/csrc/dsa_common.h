@@ -135,10 +135,6 @@ int launch_mqa_logits(bool filter, const uint8_t* q, const uint8_t* kv, const fl
                       int64_t weights_stride, const int32_t* ks, const int32_t* ke, int num_rows, int64_t num_keys,
                       float* logits, int64_t logits_stride, PrefillList* ws, hipStream_t st);
 
-// Sparse MLA decode over physical slots of the paged fp8 cache (the body of
-// dsa_sparse_mla_decode). max_out (splits == 1 only) receives each head's
-// largest scaled score in natural units; with compact set, each row's valid
-// indices must come first and a workgroup stops at its first block with none.
 // A chunked prefill's keys for the sparse MLA decode kernel: token t attends
 // over the first counts[2t] entries of its cache-slot list (valid slots first)
 // and over counts[2t+1] fresh bf16 rows rows[idx[t][i]] (row stride in
@@ -152,6 +148,10 @@ struct MlaFresh {
   const int32_t* idx;
   int64_t idx_stride;
 };
+// Sparse MLA decode over physical slots of the paged fp8 cache (the body of
+// dsa_sparse_mla_decode), with the fresh rows of a chunked prefill where `fresh`
+// is given. max_out (splits == 1 only) receives each head's largest scaled score
+// in natural units.
 int sparse_mla_decode_impl(const void* q, int64_t q_token_stride, int64_t q_head_stride, const uint8_t* kv_cache,
                            int64_t kv_block_stride_bytes, int kv_block_size, int64_t kv_num_blocks,
                            const int32_t* indices, int64_t idx_stride, int num_tokens, int num_heads, int topk,

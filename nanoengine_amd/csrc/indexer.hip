@@ -592,8 +592,9 @@ indexer_filter_kernel(const uint8_t* __restrict__ q, const uint8_t* __restrict__
   for (int j = 0; j < NQ; ++j) flush(j);
 }
 
-// The most tokens (rows times the longest context) scored by the persistent
-// kernel and kept; the callers give the measurements.
+// The most tokens scored by the persistent kernel and kept: batch entries times
+// the longest context for the logits operator, rows (batch entries times next_n)
+// times it for whole-row selects; the callers give the measurements.
 constexpr int64_t kScoreTokens = 3 << 20;
 
 static int filter_grid() {
@@ -673,7 +674,9 @@ extern "C" int dsa_indexer_logits(const uint8_t* q_fp8, const uint8_t* kv_cache,
   // rows of 3K to 40K tokens: 23.7 us against 28.0 of one workgroup per 24
   // pages; 64 rows of 16K 28.4 / 31.8, 32 of 64K 52 / 55). Past kScoreTokens
   // there are workgroups enough and it loses by a little: 256 x 16K 106 / 106,
-  // 128 x 64K 220 / 205.
+  // 128 x 64K 220 / 205. Batch entries count, not rows: a page is read once for
+  // both query tokens (next_n = 2, 180 x 16K: 101 / 103, ragged 63 / 72; 47 x 64K
+  // 103 / 104, ragged 61 / 69).
   if (batch * max_context_len <= kScoreTokens &&
       launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch, next_n,
                                max_context_len, 0, nullptr, logits, logits_stride, (hipStream_t)stream))
@@ -753,11 +756,11 @@ extern "C" int dsa_indexer_topk(const uint8_t* q_fp8, const uint8_t* kv_cache, c
   // Short contexts and few long ones: every score (in the logits buffer), then
   // a select over whole rows. The sample pass and the list pay for themselves
   // where the scores' own bytes and the row select's rounds of the CUs do not.
-  // Indexer us, lists against whole rows: 4 x 4K 24.5 / 15.3, 64 x 16K 49.7 /
-  // 39.4, 1024 x 8K 284 / 256, 200 x 16K 77 / 67 but 250 x 16K 116 / 120;
-  // 8 x 32K 32.9 / 24.3, 64 x 32K 71.2 / 67.6 but 128 x 32K 116 / 122; 1 x 64K
-  // 36.1 / 28.7, 8 x 64K 39.8 / 40.0, 32 x 64K 71 / 76. (The row select has
-  // since become 1 to 2 us slower, for scores that crowd linear bins.)
+  // Indexer us from a graph, lists against whole rows: 4 x 4K 28.6 / 20.2,
+  // 64 x 16K 55.0 / 46.9, 1024 x 8K 298 / 270, 200 x 16K 107 / 104 and 250 x 16K
+  // 129 / 128; 8 x 32K 37.1 / 31.4, 64 x 32K 77.7 / 76.4 but 96 x 32K 101 / 104
+  // and 128 x 32K 124 / 131; 1 x 64K 39.7 / 36.1, 2 x 64K 43.3 / 37.9 but
+  // 8 x 64K 44.3 / 48.2 and 32 x 64K 77 / 85.
   if (max_context_len <= 8192 || (max_context_len <= 32768 && rows * max_context_len <= kScoreTokens) ||
       (max_context_len <= kRowSelectLen && rows <= 2)) {
     if (launch_filter_persistent(q_fp8, kv_cache, weights, context_lens, block_tables, block_table_stride, batch,

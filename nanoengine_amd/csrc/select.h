@@ -140,4 +140,137 @@ struct CompositeDigits {
   }
 };
 
+// Adds one to hist[d] for every calling lane; where half of a wave shares the
+// first lane's bin (ties), one atomic for those: on one LDS word they would go
+// one after another.
+__device__ __forceinline__ void crowd_add(uint32_t* hist, uint32_t d) {
+  const uint32_t first = __builtin_amdgcn_readfirstlane(d);  // of the lanes here
+  const uint64_t same = __ballot(d == first);
+  const uint32_t n = (uint32_t)__popcll(same);
+  const bool share = n >= 32 && d == first;
+  if (!share || (int)(threadIdx.x & 63) == __builtin_ctzll(same)) atomicAdd(&hist[d], share ? n : 1u);
+}
+
+// The smallest and largest of the block's values (NT threads), to all of them.
+template <int NT>
+__device__ __forceinline__ void block_range(uint32_t* wave_sum, uint32_t& low, uint32_t& high) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    low = min(low, (uint32_t)__shfl_xor(low, off, 64));
+    high = max(high, (uint32_t)__shfl_xor(high, off, 64));
+  }
+  if (lane == 0) {
+    wave_sum[wave] = low;
+    wave_sum[NT / 64 + wave] = high;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) {
+    low = min(low, wave_sum[i]);
+    high = max(high, wave_sum[NT / 64 + i]);
+  }
+}
+
+// Of the elements with keys in [kmin, kmax], too many to rank by counting, the
+// `remain` first ones (fewer than there are) are marked: the range is binned
+// again (outliers and long tails leave most scores in one bin), the threshold
+// bin ranked if that leaves it few elements, and otherwise (ties) radix levels
+// follow over what it spans. pass(f) calls f(key, position) for every element of
+// the row, in or out of the range; mark(position) selects one; ties(key, n) may
+// mark the n lowest positions of one key by itself (true), else the levels do.
+// Bins: the second binning (two kinds of bins at run time cost rows of 8K with an
+// outlier 1 us).
+// s holds the block's hist, wave_sum, rank, tb, above, eq and a count that is 0
+// on entry. All threads call it, with the same arguments.
+template <int NT, typename Bins, typename Smem, typename Pass, typename Mark, typename Ties>
+__device__ __forceinline__ void select_crowd(Smem& s, uint32_t kmin, uint32_t kmax, uint32_t remain, Pass&& pass,
+                                             Mark&& mark, Ties&& ties) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  auto each = [&](auto&& f) {
+    pass([&](uint32_t key, uint32_t pos) {
+      if (key >= kmin && key <= kmax) f(key, pos);
+    });
+  };
+  if (kmin != kmax) {
+    for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
+    // -inf, alone below every other score, must not stretch the range
+    const uint32_t ninf = order_key(-__builtin_inff());
+    uint32_t low = kmin, high = kmax;
+    if (kmin <= ninf) {
+      low = 0xffffffffu;
+      each([&](uint32_t key, uint32_t) { low = min(low, key > ninf ? key : 0xffffffffu); });
+      __syncthreads();  // every thread has read the range
+      block_range<NT>(s.wave_sum, low, high);
+    }
+    __syncthreads();
+    const Bins bins(low, min(high, order_key(3.4028235e38f)));
+    uint32_t lowest = 0;
+    each([&](uint32_t key, uint32_t) {
+      const uint32_t d = bins.of(key);
+      if (d) crowd_add(s.hist, d);
+      else ++lowest;
+    });
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) lowest += (uint32_t)__shfl_xor(lowest, off, 64);
+    if (lane == 0 && lowest) atomicAdd(&s.hist[0], lowest);
+    __syncthreads();
+    find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
+    const uint32_t tb = s.tb, eq = s.eq;
+    remain -= s.above;
+    const bool whole_bin = eq == remain, ranked = !whole_bin && eq <= (uint32_t)kRankCap;
+    low = 0xffffffffu;
+    high = 0u;
+    each([&](uint32_t key, uint32_t pos) {
+      const uint32_t d = bins.of(key);
+      if (d > tb || (whole_bin && d == tb)) {
+        mark(pos);
+      } else if (d == tb) {
+        if (ranked) {
+          s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key, pos);
+        } else {
+          low = min(low, key);
+          high = max(high, key);
+        }
+      }
+    });
+    __syncthreads();
+    if (whole_bin) return;
+    if (ranked) {
+      if ((uint32_t)tid < eq) {
+        const uint64_t mine = s.rank[tid];
+        uint32_t ahead = 0;
+        for (uint32_t j = 0; j < eq; ++j) ahead += s.rank[j] > mine ? 1u : 0u;
+        if (ahead < remain) mark(kIdxMax - (uint32_t)(mine & kIdxMax));
+      }
+      return;
+    }
+    block_range<NT>(s.wave_sum, low, high);
+    kmin = low;
+    kmax = high;
+  }
+  if (kmin == kmax && ties(kmin, remain)) return;
+  const CompositeDigits digits(kmin, kmax);
+  uint64_t prefix = 0;  // the digits chosen so far
+  for (int L = 0; L < digits.levels; ++L) {
+    __syncthreads();  // every thread has read the previous level's outcome
+    for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
+    __syncthreads();
+    each([&](uint32_t key, uint32_t pos) {
+      if (digits.above(key, pos, L) == prefix) crowd_add(s.hist, digits.of(key, pos, L));
+    });
+    __syncthreads();
+    find_threshold<NT>(s.hist, s.wave_sum, digits.bins(L), remain, &s.tb, &s.above, &s.eq);
+    const uint32_t t = s.tb;
+    remain -= s.above;
+    const bool done = s.eq == remain || L == digits.levels - 1;
+    each([&](uint32_t key, uint32_t pos) {
+      const uint32_t d = digits.of(key, pos, L);
+      if (digits.above(key, pos, L) == prefix && (d > t || (done && d == t))) mark(pos);
+    });
+    if (done) return;
+    prefix = prefix * (uint32_t)digits.bins(L) + t;
+  }
+}
+
 }  // namespace dsa

@@ -536,7 +536,7 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   extern __shared__ __align__(16) uint8_t smem_raw[];
   ListSmem& s = *reinterpret_cast<ListSmem*>(smem_raw);
   constexpr int NT = kTopkThreads;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int b = blockIdx.x;
   const int64_t l = seq_lens[b];
   const int len = (int)(l < 0 ? 0 : (l > max_len ? max_len : l));
@@ -571,11 +571,18 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
       cl[u] = w.pos[e];
     }
   }
-  auto each = [&](auto&& f) {  // f(key, position) over this thread's candidates
+  uint32_t cd[kReg];  // their bins
+  // f(key, position, bin) over this thread's candidates; the bin is kept where it
+  // is in registers, and otherwise made again by bin_of(key)
+  auto each = [&](auto&& bin_of, auto&& f) {
 #pragma unroll
     for (int u = 0; u < kReg; ++u)
-      if ((uint32_t)(u * NT) < cand && (uint32_t)(u * NT + tid) < cand) f(ch[u], cl[u]);
-    for (uint32_t e = kReg * NT + tid; e < cand; e += NT) f(w.key[e], w.pos[e]);
+      if ((uint32_t)(u * NT) < cand && (uint32_t)(u * NT + tid) < cand) f(ch[u], cl[u], cd[u]);
+    for (uint32_t e = kReg * NT + tid; e < cand; e += NT) {
+      const uint32_t key = w.key[e];
+      uint32_t d = bin_of(key);
+      f(key, w.pos[e], d);
+    }
   };
   // The selected positions are marked in LDS: a byte each where the row fits
   // (plain stores), else a bit each. In a short row most positions are
@@ -609,93 +616,67 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   for (int i = tid; i < nwords; i += NT) s.bitmap[i] = 0u;
   for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
   if (tid == 0) s.count = 0u;
-  auto block_range = [&](uint32_t& low, uint32_t& high) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      low = min(low, (uint32_t)__shfl_xor(low, off, 64));
-      high = max(high, (uint32_t)__shfl_xor(high, off, 64));
-    }
-    if (lane == 0) {
-      s.wave_sum[wave] = low;
-      s.wave_sum[NT / 64 + wave] = high;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) {
-      low = min(low, s.wave_sum[i]);
-      high = max(high, s.wave_sum[NT / 64 + i]);
-    }
-  };
   // the range of the scores above -inf (which ranks below every bin's start)
   const uint32_t ninf = order_key(-__builtin_inff()), fmax_key = order_key(3.4028235e38f);
   uint32_t kmin = 0xffffffffu, kmax = 0u;
-  each([&](uint32_t key, uint32_t) {
+  each([](uint32_t) { return 0u; }, [&](uint32_t key, uint32_t, uint32_t&) {
     kmin = min(kmin, key > ninf ? key : 0xffffffffu);
     kmax = max(kmax, key);
   });
-  block_range(kmin, kmax);
+  block_range<NT>(s.wave_sum, kmin, kmax);
   uint8_t* const flags = reinterpret_cast<uint8_t*>(s.bitmap);
   auto mark = [&](uint32_t pos) {
     if (bytes) flags[pos] = 1;
     else atomicOr(&s.bitmap[pos >> 5], 1u << (pos & 31));
   };
 
-  uint32_t remain = (uint32_t)top_k;
-  bool done = false;
-  // One digit over the candidates that `visit` passes on: those in a higher bin
-  // than the threshold's are selected, the ones in it ranked if they are few;
-  // otherwise [kmin, kmax] becomes their range (bins never decrease with the
-  // key, so that the range holds no others). Bin 0 is counted in registers: a
+  // First digit, straight from the registers. Bin 0 is counted in registers: a
   // crowd in it would serialise on one LDS word.
-  auto digit = [&](const ListBins bins, auto&& visit) {
-    uint32_t lowest = 0;
-    visit([&](uint32_t key, uint32_t) {
-      const uint32_t d = bins.of(key);
-      if (d) atomicAdd(&s.hist[d], 1u);
-      else ++lowest;
-    });
+  const ListBins bins(kmin, min(kmax, fmax_key));
+  uint32_t remain = (uint32_t)top_k;
+  uint32_t lowest = 0;
+  each([](uint32_t) { return 0u; }, [&](uint32_t key, uint32_t, uint32_t& d) {
+    d = bins.of(key);
+    if (d) atomicAdd(&s.hist[d], 1u);
+    else ++lowest;
+  });
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) lowest += (uint32_t)__shfl_xor(lowest, off, 64);
-    if (lane == 0 && lowest) atomicAdd(&s.hist[0], lowest);
-    __syncthreads();
-    find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
-    const uint32_t tb = s.tb, eq = s.eq;
-    remain -= s.above;
-    const bool whole_bin = eq == remain, ranked = !whole_bin && eq <= (uint32_t)kRankCap;
-    uint32_t low = 0xffffffffu, high = 0u;
-    visit([&](uint32_t key, uint32_t pos) {
-      const uint32_t d = bins.of(key);
-      if (d > tb || (whole_bin && d == tb)) {
-        mark(pos);
-      } else if (d == tb) {
-        if (ranked) {
-          s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key, pos);
-        } else {
-          low = min(low, key);
-          high = max(high, key);
-        }
+  for (int off = 32; off >= 1; off >>= 1) lowest += (uint32_t)__shfl_xor(lowest, off, 64);
+  if (lane == 0 && lowest) atomicAdd(&s.hist[0], lowest);
+  __syncthreads();
+  find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
+  const uint32_t tb = s.tb, eq = s.eq;
+  remain -= s.above;
+  const bool whole_bin = eq == remain, ranked = !whole_bin && eq <= (uint32_t)kRankCap;
+  // Candidates in a higher bin are selected; the threshold bin's are ranked if
+  // they are few, or their range is taken (bins never decrease with the key, so
+  // that it holds no others).
+  uint32_t low = 0xffffffffu, high = 0u;
+  each([&](uint32_t key) { return bins.of(key); }, [&](uint32_t key, uint32_t pos, uint32_t d) {
+    if (d > tb || (whole_bin && d == tb)) {
+      mark(pos);
+    } else if (d == tb) {
+      if (ranked) {
+        s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key, pos);
+      } else {
+        low = min(low, key);
+        high = max(high, key);
       }
-    });
-    __syncthreads();
-    done = whole_bin || ranked;
-    if (ranked && (uint32_t)tid < eq) {
-      // each of the threshold bin's candidates counts those ahead of it
+    }
+  });
+  __syncthreads();
+  if (ranked) {
+    // each of the threshold bin's candidates counts those ahead of it
+    if ((uint32_t)tid < eq) {
       const uint64_t mine = s.rank[tid];
       uint32_t ahead = 0;
       for (uint32_t j = 0; j < eq; ++j) ahead += s.rank[j] > mine ? 1u : 0u;
       if (ahead < remain) mark(kIdxMax - (uint32_t)(mine & kIdxMax));
     }
-    if (!done) {
-      block_range(low, high);
-      kmin = low;
-      kmax = high;
-    }
-  };
-  digit(ListBins(kmin, min(kmax, fmax_key)), each);
-
-  if (!done) {
-    // The crowded paths read the list again (from L2, four entries in flight), so
-    // that they cost the usual one no registers.
+  } else if (!whole_bin) {
+    // A crowded bin reads the list again (from L2, four entries in flight), so
+    // that it costs the usual case no registers.
+    block_range<NT>(s.wave_sum, low, high);
     auto again = [&](auto&& f) {
 #pragma unroll 1
       for (uint32_t e0 = tid; e0 < cand; e0 += 4 * NT) {
@@ -708,42 +689,10 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-          if (e0 + u * NT < cand && key[u] >= kmin && key[u] <= kmax) f(key[u], pos[u]);
+          if (e0 + u * NT < cand) f(key[u], pos[u]);
       }
     };
-    for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
-    // -inf, alone below every other score, must not stretch the range
-    uint32_t low = 0xffffffffu, high = 0u;
-    again([&](uint32_t key, uint32_t) {
-      low = min(low, key > ninf ? key : 0xffffffffu);
-      high = max(high, key);
-    });
-    __syncthreads();  // every thread has read the bin's range
-    block_range(low, high);
-    digit(ListBins(low, min(high, fmax_key)), again);
-    if (!done) {
-      // ties: radix levels of 12 bits of [ key - kmin ][ (2^18-1) - position : 18 ]
-      const CompositeDigits digits(kmin, kmax);
-      uint64_t prefix = 0;  // the digits chosen so far
-      for (int L = 0; L < digits.levels && !done; ++L) {
-        __syncthreads();  // every thread has read the previous level's outcome
-        for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
-        __syncthreads();
-        again([&](uint32_t key, uint32_t pos) {
-          if (digits.above(key, pos, L) == prefix) atomicAdd(&s.hist[digits.of(key, pos, L)], 1u);
-        });
-        __syncthreads();
-        find_threshold<NT>(s.hist, s.wave_sum, digits.bins(L), remain, &s.tb, &s.above, &s.eq);
-        const uint32_t t = s.tb;
-        remain -= s.above;
-        done = s.eq == remain || L == digits.levels - 1;
-        again([&](uint32_t key, uint32_t pos) {
-          const uint32_t d = digits.of(key, pos, L);
-          if (digits.above(key, pos, L) == prefix && (d > t || (done && d == t))) mark(pos);
-        });
-        prefix = prefix * (uint32_t)digits.bins(L) + t;
-      }
-    }
+    select_crowd<NT, ListBins>(s, low, high, remain, again, mark, [](uint32_t, uint32_t) { return false; });
   }
 
   // compaction in position order and output
@@ -804,15 +753,17 @@ topk_list_defer_kernel(const int32_t* __restrict__ seq_lens, int64_t max_len, Pr
 // row once: thread t holds positions [4t, 4t + 4) of every chunk of 4096 in
 // registers. First digit: the score's bin (linear in its bits or in the score),
 // counted over the whole row; the threshold bin's few elements count those ahead
-// of them, a crowded bin is binned again, and ties take radix levels. The selected positions are a bitmap in LDS,
-// compacted in position order by one block scan.
+// of them, a crowded bin is binned again, and ties are numbered by position. The
+// selected positions are a bitmap in LDS, compacted in position order by one
+// block scan.
 //
 // What bounds it: a chain of short phases in one CU (loads, extremes, LDS
 // histogram, threshold, ranks, compaction). A 1/8 sample's threshold, the
 // candidates above it listed and three radix levels over the list took
-// 30 us a call for 33 rows of 40000 scores where this takes 19.7, for normal
-// scores as for ones with an outlier or a long tail. (Bins linear in the score
-// alone: 17.4 for normal scores, but 91 with one outlier of 1e9.)
+// 31 us a call for 33 rows of 40000 scores where this takes 20.3, for normal
+// scores as for ones with an outlier or a long tail, and 153 for four distinct
+// scores where this takes 61. (Bins linear in the score alone: 17.4 for normal
+// scores, but 91 with one outlier of 1e9.)
 // Instantiated per power of two of the row's chunks: a kernel for longer rows
 // spends its registers and tests on chunks that a short one does not have.
 constexpr int kRowThreads = 1024;
@@ -918,6 +869,7 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
 #pragma unroll
   for (int i = 0; i < NW; ++i) second = fminf(second, s.floors[i]);
   uint32_t remain = (uint32_t)top_k;
+  uint32_t crowd_low = 0u, crowd_high = 0u;  // the keys of a threshold bin too crowded to rank
   auto decide = [&](const auto bins) {
 
   // ---- first digit. Scores with a long tail (or many at the lowest value)
@@ -946,6 +898,7 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
   const bool whole_bin = eq == remain;
   const uint32_t sure = whole_bin ? tb : tb + 1;  // bins selected whole
   const bool ranked = !whole_bin && eq <= (uint32_t)kRankCap;
+  uint32_t low = 0xffffffffu, high = 0u;  // the keys of a crowded threshold bin
 #pragma unroll
   for (int c = 0; c < kChunks; ++c)
     if (c < nch) {
@@ -955,9 +908,17 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint32_t d = bins.bin(x[4 * c + e]);
-          if (d >= sure) quad |= 1u << e;
-          else if (ranked && d == tb)
-            s.rank[atomicAdd(&s.count, 1u)] = rank_composite(order_key(x[4 * c + e]), (uint32_t)(p + e));
+          if (d >= sure) {
+            quad |= 1u << e;
+          } else if (d == tb) {
+            const uint32_t key = order_key(x[4 * c + e]);
+            if (ranked) {
+              s.rank[atomicAdd(&s.count, 1u)] = rank_composite(key, (uint32_t)(p + e));
+            } else {
+              low = min(low, key);
+              high = max(high, key);
+            }
+          }
         }
       }
       // eight lanes' quads are a word of the bitmap
@@ -965,24 +926,33 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
       if ((lane & 7) == 0) s.bits[p >> 5] = word;
     }
   __syncthreads();
-  // the threshold bin's n listed elements: those with fewer than `room` ahead of them
-  auto rank_listed = [&](uint32_t n, uint32_t room) {
-    if ((uint32_t)tid < n) {
+  if (ranked) {
+    // the threshold bin's elements: those with fewer than `remain` ahead of them
+    if ((uint32_t)tid < eq) {
       const uint64_t mine = s.rank[tid];
       uint32_t ahead = 0;
-      for (uint32_t e = 0; e < n; ++e) ahead += s.rank[e] > mine ? 1u : 0u;
+      for (uint32_t e = 0; e < eq; ++e) ahead += s.rank[e] > mine ? 1u : 0u;
       const uint32_t pos = kIdxMax - (uint32_t)(mine & kIdxMax);
-      if (ahead < room) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
+      if (ahead < remain) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
     }
-  };
-  if (ranked) {
-    rank_listed(eq, remain);
   } else if (!whole_bin) {
-    // Too many elements for that: the bin's own range in 4096 bins again
-    // (outliers and long tails leave most scores in one bin), and, where they
-    // tie, radix levels. The row is read again (from L2, four chunks in flight),
-    // so that these paths cost the usual one no registers.
-    auto each = [&](auto&& visit) {
+    // Too many elements for that. The row is read again (from L2, four chunks in
+    // flight), so that this costs the usual case no registers.
+    block_range<NT>(s.wave_sum, low, high);
+    crowd_low = low;
+    crowd_high = high;
+  }
+  return ranked || whole_bin;
+  };
+  // The 2 x 1024 scores that are some thread's highest two are at least `second`,
+  // so that the top-k (at most 2048) is: above it the bins are linear in the
+  // float's bits (outliers and long tails then cost a few octaves of bins, not
+  // the range), unless it is negative (rows of a few scores per thread), where
+  // that would spend the bins around zero. Infinities fall into the end bins.
+  const float top = fminf(hi, 3.4028235e38f);
+  const bool decided = second > 0.f ? decide(BitBins(second, top)) : decide(ScoreBins(lo, top));
+  if (!decided) {
+    auto quads = [&](auto&& visit) {  // visit(chunk, position, the quad's keys)
 #pragma unroll 1
       for (int c0 = 0; c0 < nch; c0 += 4) {
         v4f v[4];
@@ -993,97 +963,66 @@ topk_row_kernel(const RowIn in, const int32_t* __restrict__ offsets, const int32
         for (int u = 0; u < 4; ++u) {
           const int p = kRowChunk * (c0 + u) + 4 * tid;
           if (p >= len) continue;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float y = score(p, e, v[u][e]);
-            if (bins.bin(y) == tb) visit(y, (uint32_t)(p + e));
-          }
+          uint4 key;
+          key.x = order_key(score(p, 0, v[u][0]));
+          key.y = order_key(score(p, 1, v[u][1]));
+          key.z = order_key(score(p, 2, v[u][2]));
+          key.w = order_key(score(p, 3, v[u][3]));
+          visit(c0 + u, p, key);
         }
       }
     };
-    float zlo = inf, zhi = -inf;
-    each([&](float y, uint32_t) {
-      zlo = fminf(zlo, y > -inf ? y : inf);
-      zhi = fmaxf(zhi, y);
-    });
-    block_extremes(zlo, zhi);
-    const ScoreBins zoom(zlo, fminf(zhi, 3.4028235e38f));
-    for (int i = tid; i < kHistBins; i += NT) s.hist[i] = 0u;
-    __syncthreads();
-    lowest = 0;
-    each([&](float y, uint32_t) {
-      const uint32_t d = zoom.bin(y);
-      if (d) atomicAdd(&s.hist[d], 1u);
-      else ++lowest;
-    });
-    add_lowest(lowest);
-    __syncthreads();
-    find_threshold<NT>(s.hist, s.wave_sum, kHistBins, remain, &s.tb, &s.above, &s.eq);
-    const uint32_t tb2 = s.tb, eq2 = s.eq, room = remain - s.above;
-    const bool whole2 = eq2 == room;
-    if (whole2 || eq2 <= (uint32_t)kRankCap) {
-      each([&](float y, uint32_t pos) {
-        const uint32_t d = zoom.bin(y);
-        if (d > tb2 || (whole2 && d == tb2)) atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
-        else if (d == tb2) s.rank[atomicAdd(&s.count, 1u)] = rank_composite(order_key(y), pos);
+    auto again = [&](auto&& visit) {
+      quads([&](int, int p, const uint4& key) {
+        visit(key.x, (uint32_t)p);
+        visit(key.y, (uint32_t)(p + 1));
+        visit(key.z, (uint32_t)(p + 2));
+        visit(key.w, (uint32_t)(p + 3));
       });
-      __syncthreads();
-      if (!whole2) rank_listed(eq2, room);
-    } else {
-    uint32_t kmin = 0xffffffffu, kmax = 0u;
-    each([&](float y, uint32_t) {
-      kmin = min(kmin, order_key(y));
-      kmax = max(kmax, order_key(y));
-    });
+    };
+    auto mark = [&](uint32_t pos) { atomicOr(&s.bits[pos >> 5], 1u << (pos & 31)); };
+    // One key's n lowest positions: positions rise with chunk, wave, lane and
+    // quad element, so that counts per (chunk, wave) and one scan number them all
+    // (33 rows of 40000 scores of ten values 37 us, all equal 33; by radix levels
+    // from the first bin's range on, 85 and 74).
+    auto ties = [&](uint32_t tie, uint32_t n) {
+      uint64_t found = 0;  // four bits per chunk
+      quads([&](int c, int p, const uint4& key) {
+        const uint32_t m = (key.x == tie ? 1u : 0u) | (key.y == tie && p + 1 < len ? 2u : 0u) |
+                           (key.z == tie && p + 2 < len ? 4u : 0u) | (key.w == tie && p + 3 < len ? 8u : 0u);
+        found |= (uint64_t)m << (4 * c);
+      });
+      for (int c = 0; c < nch; ++c) {
+        uint32_t in_wave = 0;
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      kmin = min(kmin, (uint32_t)__shfl_xor(kmin, off, 64));
-      kmax = max(kmax, (uint32_t)__shfl_xor(kmax, off, 64));
-    }
-    if (lane == 0) {
-      s.wave_sum[wave] = kmin;
-      s.wave_sum[NW + wave] = kmax;
-    }
-    __syncthreads();
+        for (int e = 0; e < 4; ++e) in_wave += (uint32_t)__popcll(__ballot((found >> (4 * c + e)) & 1ull));
+        if (lane == 0) s.hist[c * NW + wave] = in_wave;
+      }
+      __syncthreads();
+      uint32_t total = 0;
+      const uint32_t before = block_exclusive_scan<NT>(s.wave_sum, tid < nch * NW ? s.hist[tid] : 0u, &total);
+      if (tid < nch * NW) s.hist[tid] = before;
+      __syncthreads();
+      for (int c = 0; c < nch; ++c) {
+        uint32_t at = s.hist[c * NW + wave];
+        if (at >= n) break;
+        const uint32_t mine = (uint32_t)(found >> (4 * c)) & 15u;
 #pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      kmin = min(kmin, s.wave_sum[i]);
-      kmax = max(kmax, s.wave_sum[NW + i]);
-    }
-    const CompositeDigits digits(kmin, kmax);
-    uint64_t prefix = 0;  // the digits chosen so far
-    for (int L = 0; L < digits.levels; ++L) {
-      __syncthreads();  // every thread has read the previous level's outcome
-      for (int i = tid; i < digits.bins(L); i += NT) s.hist[i] = 0u;
-      __syncthreads();
-      each([&](float y, uint32_t pos) {
-        const uint32_t key = order_key(y);
-        if (digits.above(key, pos, L) == prefix) atomicAdd(&s.hist[digits.of(key, pos, L)], 1u);
-      });
-      __syncthreads();
-      find_threshold<NT>(s.hist, s.wave_sum, digits.bins(L), remain, &s.tb, &s.above, &s.eq);
-      const uint32_t t = s.tb;
-      remain -= s.above;
-      const bool done = s.eq == remain || L == digits.levels - 1;
-      each([&](float y, uint32_t pos) {
-        const uint32_t key = order_key(y), d = digits.of(key, pos, L);
-        if (digits.above(key, pos, L) == prefix && (d > t || (done && d == t)))
-          atomicOr(&s.bits[pos >> 5], 1u << (pos & 31));
-      });
-      if (done) break;
-      prefix = prefix * (uint32_t)digits.bins(L) + t;
-    }
-    }
+        for (int e = 0; e < 4; ++e) at += (uint32_t)__popcll(__ballot((mine >> e) & 1u) & ((1ull << lane) - 1ull));
+        uint32_t quad = 0u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((mine >> e) & 1u) {
+            if (at < n) quad |= 1u << e;
+            ++at;
+          }
+        const uint32_t word = or_8_lanes(quad << (4 * (lane & 7)));
+        if ((lane & 7) == 0) s.bits[(kRowChunk * c + 4 * tid) >> 5] |= word;
+      }
+      return true;
+    };
+    select_crowd<NT, ScoreBins>(s, crowd_low, crowd_high, remain, again, mark, ties);
   }
-  };
-  // The 2 x 1024 scores that are some thread's highest two are at least `second`,
-  // so that the top-k (at most 2048) is: above it the bins are linear in the
-  // float's bits (outliers and long tails then cost a few octaves of bins, not
-  // the range), unless it is negative (rows of a few scores per thread), where
-  // that would spend the bins around zero. Infinities fall into the end bins.
-  const float top = fminf(hi, 3.4028235e38f);
-  if (second > 0.f) decide(BitBins(second, top));
-  else decide(ScoreBins(lo, top));
   __syncthreads();
 
   // ---- positions in ascending order (thread t: `per` of them, a power of two,

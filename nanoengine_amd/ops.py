@@ -224,8 +224,9 @@ def topk_workspace(batch: int, device: torch.device) -> torch.Tensor:
 
 
 def _ws_args(ws):
-    """(pointer, bytes) for a workspace tensor; False selects the path that
-    needs no workspace (the full multi-pass exact select)."""
+    """(pointer, bytes) for a workspace tensor; False for none. Aligned rows of up
+    to 64K scores need none; longer or unaligned rows without one take the full
+    multi-pass exact select."""
     return (None, 0) if ws is None or ws is False else (ws.data_ptr(), ws.numel())
 
 

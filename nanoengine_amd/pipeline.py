@@ -6,9 +6,12 @@ decode (dlengine/runtime/models/deepseek_v2/deepseek_v2.py:1860-2018 calling
 ``Indexer.forward`` lightning.py:1357-1466 with ``translate_topk=True`` and then
 ``FlashMlaAttention.forward`` flash_mla.py:76-99). Every buffer is allocated
 once in the constructor, so a step allocates nothing (capturable in a HIP
-graph). By default the indexer and the top-k run fused (``ops.indexer_topk``:
-the logits are never written to memory); ``fused=False`` runs them as the two
-separate reference operators over a logits buffer.
+graph; batches past one round of CUs on a stream other than the constructor's
+take their split partials' buffer from torch's allocator). By default the
+indexer and the top-k run fused (``ops.indexer_topk``: the logits of long
+contexts are never written to memory, those of short ones and small batches go
+to the workspace); ``fused=False`` runs them as the two separate reference
+operators over a logits buffer.
 
 Buffer ownership: a call returns views of the object's own buffers (o, lse,
 logical, physical), and the next call on the same object overwrites them. A

@@ -187,8 +187,8 @@ def ops_logits(cuda, q4, cache, w, lens, bt):
 
 @pytest.mark.parametrize("next_n", [1, 2])
 def test_both_logits_kernels_agree(cuda, next_n):
-    """The logits kernel is chosen by the batch's size (rows times the longest
-    context): the persistent one's scores, and the -inf to the end of each
+    """The logits kernel is chosen by the batch's size (batch entries times the
+    longest context): the persistent one's scores, and the -inf to the end of each
     row's last page, are bit for bit those of the per-workgroup one; neither
     writes past that page."""
     lens = [1, 64, 65, 1000, 1537, 4095, 4096, 2500] * 8

@@ -16,8 +16,9 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(scores, lens, page_tables, page_size, top_k):
-    """Both selection routes (sampled candidate list, and the full multi-pass
-    select used without a workspace) must give the same exact answer."""
+    """With a workspace and without one the answer is the same and exact. Aligned
+    rows of up to 64K positions take the row select either way; longer or
+    unaligned ones the sampled candidate list, or the full multi-pass select."""
     B = scores.shape[0]
     res = []
     for ws in (None, False):
@@ -174,10 +175,9 @@ def test_rejects_bad_arguments(cuda):
 
 
 def test_sample_blind_spots_fall_back_exactly(cuda):
-    """Rows of up to 64K positions take the one-launch path, whose threshold comes
-    from a 1/8 sample of the row. Scores that put the whole top-k where the sample
-    does not look (positions 1 mod 4), or that make every position a candidate
-    (a constant row), must still give the exact answer through the fallback."""
+    """Rows of up to 64K positions that defeated a sampled threshold (16384 large
+    scores at the positions 1 mod 4, a constant row, a ramp): exact by the row
+    select, which samples nothing."""
     L = 65536
     rng = np.random.default_rng(7)
     base = rng.standard_normal(L).astype(np.float32)
@@ -262,3 +262,71 @@ def test_whole_row_select_at_chunk_edges(cuda, width, top_k):
     e_page, e_raw = O.topk_transform(scores, lens, pt, 64, top_k)
     assert np.array_equal(raw.cpu().numpy(), e_raw)
     assert np.array_equal(out.cpu().numpy(), e_page)
+
+
+@pytest.mark.parametrize("length", [2051, 4100, 9001, 40000, 65533])
+@pytest.mark.parametrize("top_k", [512, 2048])
+def test_whole_row_ties_take_the_lowest_positions(cuda, length, top_k):
+    """Rows of few distinct scores: the lowest positions of the value on the
+    border, whether its elements fill a whole bin of the first digit, come out
+    of the second one, lie at -inf beside the row's padding, or are spread so
+    thin that the last ones lie in the row's last quad."""
+    rng = np.random.default_rng(length * top_k)
+    rows = [rng.integers(0, 10, length).astype(np.float32) - 20,           # ten negative values
+            rng.integers(0, 4, length).astype(np.float32),
+            np.maximum(rng.standard_normal(length) - 2.2, 0),              # few positive, the rest zero
+            np.ones(length), np.full(length, -np.inf), np.full(length, np.nan),
+            np.where(np.arange(length) < top_k - 3, 1.0, -np.inf),         # the border among the -inf ones
+            np.where(np.arange(length) % 2 == 0, -0.0, 0.0),               # -0 ranks below +0
+            np.where(np.arange(length) >= length - top_k - 1, 2.0, 1.0),   # all of the border at the end
+            rng.integers(0, 3, length) * 1e30 - 1e30]
+    scores = np.stack([np.asarray(r, np.float32) for r in rows])
+    scores[0, 5] = 1e9                                                     # an outlier over them
+    B = len(rows)
+    stride = (length + 3) & ~3
+    padded = torch.full((B, stride), 7.0, device=cuda)[:, :length]
+    padded.copy_(torch.from_numpy(scores))
+    lens = np.full(B, length, np.int32)
+    pt = np.tile(np.arange((length + 63) // 64, dtype=np.int32), (B, 1))
+    out = torch.empty(B, top_k, dtype=torch.int32, device=cuda)
+    raw = torch.empty_like(out)
+    ops.topk_transform(padded, torch.from_numpy(lens).to(cuda), torch.from_numpy(pt).to(cuda), out, 64, top_k, raw)
+    torch.cuda.synchronize()
+    _, e_raw = O.topk_transform(scores, lens, pt, 64, top_k)
+    assert np.array_equal(raw.cpu().numpy(), e_raw)
+    assert np.array_equal(out.cpu().numpy(), e_raw)
+
+
+@pytest.mark.parametrize("length,stride", [(131072, 131072), (50001, 50001)])
+def test_three_launch_sample_blind_spots_fall_back_exactly(cuda, length, stride):
+    """Rows longer than 64K, or of an unaligned stride, take their threshold from
+    one 1024-score chunk in eight. Large scores in the chunks between: few (the
+    list holds them), more than a gather workgroup stages, more than the list
+    holds (both fall back to the full select); a row that ties throughout."""
+    rng = np.random.default_rng(length)
+    B = 5
+    scores = rng.standard_normal((B, length)).astype(np.float32)
+    pos = np.arange(length)
+    unseen = (pos // 1024) % 8 != 0
+    scores[0][unseen & (pos % 47 == 5)] += 100.0       # about one or 2.4 thousand
+    scores[1][(pos // 1024) % 8 == 3] += 100.0         # 1024 to a gather span, 8 or 16 thousand in all
+    scores[2][unseen & (pos < 16384)] += 100.0         # more than one workgroup stages
+    scores[3] = 0.5
+    scores[4][unseen] += 100.0
+    lens = np.full(B, length, np.int32)
+    pt = np.stack([rng.permutation((length + 63) // 64) for _ in range(B)]).astype(np.int32)
+    flat = torch.zeros((B - 1) * stride + length, device=cuda)
+    padded = flat.as_strided((B, length), (stride, 1))
+    padded.copy_(torch.from_numpy(scores))
+    out, raw = _run(padded, torch.from_numpy(lens).to(cuda), torch.from_numpy(pt).to(cuda), 64, 2048)
+    e_page, e_raw = O.topk_transform(scores, lens, pt, 64, 2048)
+    assert np.array_equal(raw, e_raw)
+    assert np.array_equal(out, e_page)
+    # the fall-backs really happened: a list's count past its 6144 entries
+    ws = torch.zeros(ops.topk_workspace_bytes(B), dtype=torch.uint8, device=cuda)
+    o = torch.empty(B, 2048, dtype=torch.int32, device=cuda)
+    ops.topk_transform(padded, torch.from_numpy(lens).to(cuda), torch.from_numpy(pt).to(cuda), o, 64, 2048,
+                       workspace=ws)
+    count = ws.view(torch.int32).view(B, -1)[:, 1].cpu()
+    print(count.tolist(), flush=True)
+    assert 2048 <= int(count[0]) <= 6144 and (count[1:] > 6144).all()

@@ -623,7 +623,7 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
     kmin = min(kmin, key > ninf ? key : 0xffffffffu);
     kmax = max(kmax, key);
   });
-  block_range<NT>(s.wave_sum, kmin, kmax);
+  const uint32_t wave_top = block_range<NT>(s.wave_sum, kmin, kmax);
   uint8_t* const flags = reinterpret_cast<uint8_t*>(s.bitmap);
   auto mark = [&](uint32_t pos) {
     if (bytes) flags[pos] = 1;
@@ -631,8 +631,10 @@ __device__ __forceinline__ void list_select_row(const int32_t* __restrict__ seq_
   };
 
   // First digit, straight from the registers. Bin 0 is counted in registers: a
-  // crowd in it would serialise on one LDS word.
-  const ListBins bins(kmin, min(kmax, fmax_key));
+  // crowd in it would serialise on one LDS word. Bins linear in the score end at
+  // the lowest of the waves' largest scores: a few outliers share the last bin
+  // with the few scores above that, far from the border.
+  const ListBins bins(kmin, min(kmax, fmax_key), min(wave_top, fmax_key));
   uint32_t remain = (uint32_t)top_k;
   uint32_t lowest = 0;
   each([](uint32_t) { return 0u; }, [&](uint32_t key, uint32_t, uint32_t& d) {

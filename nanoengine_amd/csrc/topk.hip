@@ -26,8 +26,8 @@
 //      bitmap, compacted with one block prefix scan (ascending order, so the
 //      output is deterministic) and written with the page translation.
 // No global sort, no bounded candidate buffer on the exact path. The row
-// select and the fused indexer's list select (topk_list_kernel) take the
-// score's linear bin as their first digit.
+// select and the fused indexer's list select (topk_list_kernel) take a bin of
+// the score as their first digit.
 #include <mutex>
 
 #include "dsa_common.h"
@@ -521,9 +521,10 @@ __device__ void repair_row_logits(const RowRepair& rp, const int32_t* __restrict
 // however its scores lie. (Radix digits of the key's bits, all levels, took 17.0
 // us for four rows of 4K tokens, whose scores cross zero: sign and exponent bits
 // put most candidates into a few bins, where the LDS atomics serialise. Bins
-// linear in the score only: 128 rows of 64K, normal scores 14.0 us here and
-// there, one outlier in each 27.0 against 15.8; 16 rows of 128K with a long tail
-// 712 against 15.2, as a crowded bin of more than 6144 made the row be redone.)
+// linear in the score between the list's extremes: 128 rows of 64K, normal
+// scores 14.0 us here and there, one outlier in each 26.8 against 15.3; 16 rows
+// of 128K with a long tail 716 against 15.0, as a crowded bin of more than 6144
+// made the row be redone.)
 // kRepair: a row whose list is unusable (fewer than k entries, or more than its
 // capacity) is redone in the kernel from its full logits (rp.q set, the launch
 // reserves TopkSmem); otherwise it is appended to rp.defer_rows.

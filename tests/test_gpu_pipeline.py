@@ -150,3 +150,40 @@ def test_full_shared_full_layers_keep_each_output(cuda):
         eo, el = ops.sparse_mla_decode(layers[i][0], layers[i][1], sel, 192 ** -0.5)
         torch.cuda.synchronize()
         assert torch.equal(outs[i][0], eo) and torch.equal(outs[i][1], el), f"layer {i}"
+
+
+def test_shared_layers_past_one_round_on_two_streams(cuda):
+    """Shared layers of one object, each with its own out and lse, on two streams:
+    past one round of CUs, where part of the batch is split, the second stream's
+    calls take a buffer of their own."""
+    from nanoengine_amd.state import IndexerTopKState
+    B, H, K, scale = 140, 128, 512, 192 ** -0.5
+    step = DsaDecodeStep(B, 1, 4096, num_heads=H, index_topk=K, device=cuda)
+    assert step.num_splits > 1 and step.workspace.numel() <= 256 * 64 * 513 * 4
+    g = torch.Generator(device=cuda).manual_seed(6)
+    kv = synth.make_mla_cache(80, seed=6, device="cuda")
+    picks = torch.randint(0, 80 * 64, (B, K), generator=g, device=cuda, dtype=torch.int32)
+    state = IndexerTopKState()
+    state.publish(2, picks.clone(), picks)
+    sets = [(synth.make_mla_query(B, H, seed=60 + i, device="cuda"),
+             torch.empty(B, H, 512, dtype=torch.bfloat16, device=cuda), torch.empty(B, H, device=cuda))
+            for i in range(2)]
+
+    def call(i):
+        q, o, lse = sets[i]
+        step(None, None, None, None, None, None, q, kv, scale, layer_idx=3, indexer_state=state, shared=True, out=o,
+             lse=lse)
+
+    expect = []
+    for i in range(2):
+        call(i)
+        expect.append((sets[i][1].clone(), sets[i][2].clone()))
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(10):
+        call(0)
+        with torch.cuda.stream(other):
+            call(1)
+        torch.cuda.synchronize()
+        for i in range(2):
+            assert torch.equal(sets[i][1], expect[i][0]) and torch.equal(sets[i][2], expect[i][1])
